@@ -5,141 +5,460 @@
 //
 // Layouts: activations [E][C][nxe] float (node index = lidx), weights [Cout][Cin][27] with
 // offset k = (dz+1)*9 + (dy+1)*3 + (dx+1).
+#include <atomic>
+
 #include "cnn_kernels.hpp"
 #include "common.hpp"
 
 namespace sfem_amd {
 
-__device__ __forceinline__ int nbr(int L, int x, int y, int z, int k) {
-    const int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-    const int xx = x + dx, yy = y + dy, zz = z + dz;
-    if (xx < 0 || xx > L || yy < 0 || yy > L || zz < 0 || zz > L) return -1;
-    return lidx(L, xx, yy, zz);
+// ------------------------------------------------------------------ FP32 convolutions
+// The element's channels sit in LDS with a zero halo that lines and planes share: line stride
+// L + 2 (the cell after a line's last node is both its x = L + 1 and the next line's x = -1),
+// plane stride (L + 2)^2 likewise, so all 27 neighbours of a node are plain reads at constant
+// offsets from one address, without tests.  At L = 8 a channel takes 1,111 words against 1,331
+// for a halo of its own per line, which lets two blocks with 16 channels share a CU.
+//
+// A block works on NB consecutive nodes of one element and stages the planes that those and their
+// neighbours lie in: all of them (NB >= the element's nodes) when the batch fills the GPU with a block
+// per element, the few around 64 nodes when it does not (a training batch of 32 elements is 64 of
+// the odd network): more and smaller blocks, several to a CU, so that one block's loads overlap
+// another's products.
+template <int L, int NB>
+struct ConvShape {
+    static constexpr int N1 = L + 1, NXE = N1 * N1 * N1, PLANE = N1 * N1;
+    static constexpr bool FULL = NB >= NXE;
+    static constexpr int LS = L + 2, PS = LS * LS, OFF = PS + LS + 1;
+    // planes the block's nodes can touch, and the most nodes staged (a plane more on each side)
+    static constexpr int PL = FULL || (NB - 1) / PLANE + 2 > N1 ? N1 : (NB - 1) / PLANE + 2;
+    static constexpr int STAGED = (PL + 2 < N1 ? PL + 2 : N1) * PLANE;
+    static constexpr int NPAD = PL * PS + (L + 1) * LS + L + 1 + OFF + 1;
+    // channel strides (words) by the access of the matrix operand: 16 (mod 32) where a half-wave
+    // reads 16 consecutive nodes of two channels, 2 (mod 32) where it reads two nodes of 16 channels:
+    // either way its 32 words lie in different banks
+    static constexpr int CSN = NPAD + ((16 - NPAD % 32) + 32) % 32;
+    static constexpr int CSC = NPAD + ((2 - NPAD % 32) + 32) % 32;
+    static constexpr int ROWS = FULL ? NXE : NB;  // nodes of the unpadded rows, read as CSC
+    static constexpr int RSC = ROWS + ((2 - ROWS % 32) + 32) % 32;
+};
+// LDS cell of node v when the staged planes start at zlo - 1
+template <int L>
+__device__ __forceinline__ int conv_pad(int v, int zlo) {
+    using S = ConvShape<L, 1 << 20>;
+    const int x = v % S::N1, y = (v / S::N1) % S::N1, z = v / (S::N1 * S::N1);
+    return (z - zlo) * S::PS + y * S::LS + x + S::OFF;
+}
+template <int L>
+__host__ __device__ constexpr int conv_shift(int k) {
+    using S = ConvShape<L, 1 << 20>;
+    return (k / 9 - 1) * S::PS + ((k / 3) % 3 - 1) * S::LS + (k % 3 - 1);
 }
 
-// out[e][co][v] = sum_ci sum_k W[co][ci][k] act(in[e][ci][v + off_k]);  act = relu if relu_in
-__global__ void __launch_bounds__(256) conv_fwd_kernel(const int L, const ptrdiff_t E, const int Cin, const int Cout,
-                                                       const float *__restrict__ in, const float *__restrict__ W,
-                                                       const int relu_in, float *__restrict__ out) {
-    extern __shared__ float smem[];
-    const int nxe = nxe_of(L);
-    float *sin = smem;  // [Cin][nxe]; the weights (<= 28 KB) are read through the caches
-    const float *sw = W;
-    const ptrdiff_t e = blockIdx.x;
-    if (e >= E) return;  // uniform per block
-    for (int i = threadIdx.x; i < Cin * nxe; i += blockDim.x) {
-        float v = in[(size_t)e * Cin * nxe + i];
-        sin[i] = relu_in ? fmaxf(v, 0.f) : v;
-    }
-    __syncthreads();
-    const int N1 = L + 1;
-    // blockIdx.y splits the element's outputs over gridDim.y blocks (each stages the whole input)
-    for (int t = blockIdx.y * blockDim.x + threadIdx.x; t < Cout * nxe; t += blockDim.x * gridDim.y) {
-        const int co = t / nxe, v = t - co * nxe;
-        const int x = v % N1, y = (v / N1) % N1, z = v / (N1 * N1);
-        int nb[27];
+// The planes around nodes [n0, n1) of C channels of one element: load() issues every load of a thread
+// (CH >= C channels of its nodes, absent channels re-reading channel 0), store() puts them into the
+// halo layout, after relu if asked, times sg; the halo and the absent channels are zero.
+template <int L, int NB, int CS, int CH, int BLOCK>
+struct ConvStage {
+    using S = ConvShape<L, NB>;
+    static constexpr int NV = (S::STAGED + BLOCK - 1) / BLOCK;
+    float r[CH][NV];
+    int v0, v1, zlo;
+    __device__ __forceinline__ void load(const float *__restrict__ in, int C, int n0, int n1) {
+        zlo = n0 / S::PLANE;
+        const int zhi = (n1 - 1) / S::PLANE;
+        v0 = (zlo > 0 ? zlo - 1 : 0) * S::PLANE;
+        v1 = (zhi < L ? zhi + 2 : L + 1) * S::PLANE;
 #pragma unroll
-        for (int k = 0; k < 27; k++) nb[k] = nbr(L, x, y, z, k);
-        float acc = 0.f;
-        for (int ci = 0; ci < Cin; ci++) {
-            const float *w = sw + ((size_t)co * Cin + ci) * 27;
-            const float *a = sin + (size_t)ci * nxe;
+        for (int c = 0; c < CH; c++)
+#pragma unroll
+            for (int b = 0; b < NV; b++) {
+                const int v = v0 + threadIdx.x + b * BLOCK;
+                r[c][b] = in[(size_t)(c < C ? c : 0) * S::NXE + (v < v1 ? v : v0)];
+            }
+    }
+    static __device__ __forceinline__ void clear(float *__restrict__ lds) {
+        for (int i = threadIdx.x; i < CH * CS / 2; i += BLOCK) ((float2 *)lds)[i] = float2{0.f, 0.f};
+    }
+    // after clear() and a barrier
+    __device__ __forceinline__ void store(float *__restrict__ lds, int C, bool relu, float sg) const {
+#pragma unroll
+        for (int b = 0; b < NV; b++) {
+            const int v = v0 + threadIdx.x + b * BLOCK;
+            if (v >= v1) continue;
+            float *q = lds + conv_pad<L>(v, zlo);
+#pragma unroll
+            for (int c = 0; c < CH; c++)
+                if (c < C) q[c * CS] = sg * (relu ? fmaxf(r[c][b], 0.f) : r[c][b]);
+        }
+    }
+};
+// element e of a batch whose second half is the negated first one (half > 0), see conv_mfma_kernel
+__device__ __forceinline__ const float *conv_source(const float *in, ptrdiff_t e, ptrdiff_t half, size_t per, float &sg) {
+    const bool neg = half > 0 && e >= half;
+    sg = neg ? -1.f : 1.f;
+    return in + (size_t)(neg ? e - half : e) * per;
+}
+
+typedef float cv_f4 __attribute__((ext_vector_type(4)));
+
+// out[e][m][v] = sum_c sum_k w(m, c, k) act(in[e][c][v + off_k]), M output and C input channels (<= 16):
+//   forward: w = W[m][c][k], act = relu if relu_in;
+//   backward (bwd): w = W[c][m][26 - k], the gradient w.r.t. a layer's input from the gradient of its
+//   output, zero where mask[e][m][v] <= 0 (the layer's input before its relu; null: no mask).
+// half > 0: elements half .. 2 half - 1 of the input are the first half negated (the odd network's
+// second evaluation), read from there.
+//
+// On the matrix cores in FP32 (16x16x4: M = output channels, N = 16 consecutive nodes, K = four input
+// channels at one offset; one input channel (Q == 0): K = four offsets).  What bounds it: 108
+// products of 32 cycles per tile at 16 -> 16 channels; the operand reads (one LDS word per lane and
+// product, at constant offsets) take a quarter of that.  The weights stay in registers (27 Q per lane).
+// A block is four waves; with NB = 64 each has one tile.  64 elements, L = 8, 16 -> 16:
+// 15 us, where a node per thread with scalar products over LDS took 100 us (4 us of products at 154
+// TFLOP/s; the rest is launch, load latency and staging).
+template <int L, int Q, int NB>
+__global__ void __launch_bounds__(256, 2)
+    conv_mfma_kernel(const ptrdiff_t half, const int C, const int M, const float *__restrict__ in,
+                     const float *__restrict__ W, const int relu_in, const int bwd, const float *__restrict__ mask,
+                     float *__restrict__ out) {
+    using S = ConvShape<L, NB>;
+    constexpr int CS = S::CSN, QC = Q ? Q : 1;
+    extern __shared__ __align__(16) float conv_lds[];
+    const ptrdiff_t e = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int n0 = S::FULL ? 0 : (int)blockIdx.y * NB;
+    const int n1 = S::FULL || n0 + NB > S::NXE ? S::NXE : n0 + NB;
+    float sg;
+    const float *src = conv_source(in, e, half, (size_t)C * S::NXE, sg);
+    ConvStage<L, NB, CS, Q ? 4 * Q : 1, 256> st;
+    st.load(src, C, n0, n1);
+    float a[QC * 27];
+    if constexpr (Q > 0) {
+        // the weights through LDS (one coalesced read per block), rows two words apart mod 32 so that
+        // the 16 rows a half-wave reads lie in different banks
+        constexpr int NW = (16 * 4 * Q * 27 + 255) / 256;
+        const int rows = bwd ? C : M, len = (bwd ? M : C) * 27, rs = len + 2, nw = rows * len;
+        const unsigned inv = 0xffffffffu / (unsigned)len + 1;  // i / len = umulhi(i, inv) for i < 2^16
+        float wr[NW];
+#pragma unroll
+        for (int j = 0; j < NW; j++) {
+            const int i = threadIdx.x + j * 256;
+            wr[j] = W[i < nw ? i : 0];
+        }
+#pragma unroll
+        for (int j = 0; j < NW; j++) {
+            const int i = threadIdx.x + j * 256;
+            if (i < nw) conv_lds[i + 2 * (int)__umulhi((unsigned)i, inv)] = wr[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int ch = 4 * q + g;
+            const bool ok = c < M && ch < C;
+            const float *w = conv_lds + (ok ? (bwd ? ch * rs + c * 27 + 26 : c * rs + ch * 27) : 26);
+#pragma unroll
+            for (int k = 0; k < 27; k++) {
+                const float v = w[bwd ? -k : k];
+                a[q * 27 + k] = ok ? v : 0.f;
+            }
+        }
+        __syncthreads();
+    } else {
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            const int k = 4 * j + g;
+            const bool ok = c < M && k < 27;
+            const float v = W[ok ? c * 27 + (bwd ? 26 - k : k) : 0];
+            a[j] = ok ? v : 0.f;
+        }
+    }
+    st.clear(conv_lds);
+    __syncthreads();
+    st.store(conv_lds, C, relu_in != 0, sg);
+    __syncthreads();
+    int sh[7];
+    if constexpr (Q == 0) {
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            const int k = 4 * j + g < 27 ? 4 * j + g : 13;
+            sh[j] = (k / 9 - 1) * S::PS + ((k / 3) % 3 - 1) * S::LS + (k % 3 - 1);
+        }
+    }
+    for (int t0 = n0 + 16 * wave; t0 < n1; t0 += 64) {
+        const int n = t0 + c;
+        const bool real = n < n1;
+        const int base = conv_pad<L>(real ? n : n0, st.zlo);
+        cv_f4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two chains of products
+        if constexpr (Q > 0) {
+            const float *b = conv_lds + g * CS + base;
 #pragma unroll
             for (int k = 0; k < 27; k++)
-                if (nb[k] >= 0) acc += w[k] * a[nb[k]];
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    acc[(k * Q + q) & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        a[q * 27 + k], b[4 * q * CS + conv_shift<L>(k)], acc[(k * Q + q) & 1], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 7; j++)
+                acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], conv_lds[base + sh[j]], acc[j & 1], 0, 0, 0);
         }
-        out[((size_t)e * Cout + co) * nxe + v] = acc;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = 4 * g + r;
+            if (!real || m >= M) continue;
+            const size_t o = ((size_t)e * M + m) * S::NXE + n;
+            float v = acc[0][r] + acc[1][r];
+            if (mask && mask[o] <= 0.f) v = 0.f;
+            out[o] = v;
+        }
     }
 }
 
-// din[e][ci][v] = relu'(pre) * sum_co sum_k W[co][ci][k] dout[e][co][v - off_k]
-// (act_in holds the layer input before the activation when relu_in, for the mask)
-__global__ void __launch_bounds__(256) conv_bwd_data_kernel(const int L, const ptrdiff_t E, const int Cin,
-                                                            const int Cout, const float *__restrict__ dout,
-                                                            const float *__restrict__ W,
-                                                            const float *__restrict__ act_in, const int relu_in,
-                                                            float *__restrict__ din) {
-    extern __shared__ float smem[];
-    const int nxe = nxe_of(L);
-    float *sd = smem;  // [Cout][nxe]
-    const float *sw = W;
+// The same convolution for at most three output channels (the network's last layer), where 13 to 15 of
+// the matrix tile's 16 rows would be padding: 64 nodes at a time, each of the four waves taking every
+// fourth input channel (weights uniform: scalar loads), summed over the waves in LDS in wave order.
+// Bound by the LDS reads (27 C words per node).
+template <int L, int M, int NB>
+__global__ void __launch_bounds__(256)
+    conv_narrow_kernel(const ptrdiff_t half, const int C, const float *__restrict__ in, const float *__restrict__ W,
+                       const int relu_in, const int bwd, const float *__restrict__ mask, float *__restrict__ out) {
+    using S = ConvShape<L, NB>;
+    constexpr int CS = S::CSN;
+    extern __shared__ __align__(16) float conv_lds[];
+    __shared__ float red[4][M][64];
     const ptrdiff_t e = blockIdx.x;
-    if (e >= E) return;
-    for (int i = threadIdx.x; i < Cout * nxe; i += blockDim.x) sd[i] = dout[(size_t)e * Cout * nxe + i];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = S::FULL ? 0 : (int)blockIdx.y * NB;
+    const int n1 = S::FULL || n0 + NB > S::NXE ? S::NXE : n0 + NB;
+    float sg;
+    const float *src = conv_source(in, e, half, (size_t)C * S::NXE, sg);
+    ConvStage<L, NB, CS, 16, 256> st;
+    st.load(src, C, n0, n1);
+    st.clear(conv_lds);
     __syncthreads();
-    const int N1 = L + 1;
-    for (int t = blockIdx.y * blockDim.x + threadIdx.x; t < Cin * nxe; t += blockDim.x * gridDim.y) {
-        const int ci = t / nxe, v = t - ci * nxe;
-        const int x = v % N1, y = (v / N1) % N1, z = v / (N1 * N1);
-        float acc = 0.f;
-        // out[m] += W[k] in[m + off_k]  =>  din[v] += W[k] dout[v - off_k]
+    st.store(conv_lds, C, relu_in != 0, sg);
+    __syncthreads();
+    for (int t0 = n0; t0 < n1; t0 += 64) {
+        const int v = t0 + lane;
+        const float *b = conv_lds + conv_pad<L>(v < n1 ? v : n0, st.zlo);
+        float acc[M];
 #pragma unroll
-        for (int k = 0; k < 27; k++) {
-            const int m = nbr(L, x, y, z, 26 - k);  // v - off_k
-            if (m < 0) continue;
-            for (int co = 0; co < Cout; co++) acc += sw[((size_t)co * Cin + ci) * 27 + k] * sd[(size_t)co * nxe + m];
+        for (int m = 0; m < M; m++) acc[m] = 0.f;
+        for (int ch = wave; ch < C; ch += 4) {
+#pragma unroll
+            for (int k = 0; k < 27; k++) {
+                const float x = b[ch * CS + conv_shift<L>(k)];
+#pragma unroll
+                for (int m = 0; m < M; m++) acc[m] += W[bwd ? (ch * M + m) * 27 + 26 - k : (m * C + ch) * 27 + k] * x;
+            }
         }
-        if (relu_in && act_in[((size_t)e * Cin + ci) * nxe + v] <= 0.f) acc = 0.f;
-        din[((size_t)e * Cin + ci) * nxe + v] = acc;
+#pragma unroll
+        for (int m = 0; m < M; m++) red[wave][m][lane] = acc[m];
+        __syncthreads();
+        for (int m = wave; m < M; m += 4)
+            if (v < n1) {
+                const size_t o = ((size_t)e * M + m) * S::NXE + v;
+                const float s = (red[0][m][lane] + red[1][m][lane]) + (red[2][m][lane] + red[3][m][lane]);
+                out[o] = mask && mask[o] <= 0.f ? 0.f : s;
+            }
+        __syncthreads();
     }
 }
 
-// partial[b][co][ci][k] = sum over the block's elements and nodes of dout[co][v] act(in[ci][v+off_k]);
-// blockIdx.y selects a chunk of kCoChunk output channels (LDS: Cin + kCoChunk channels).
-constexpr int kCoChunk = 4;
-__global__ void __launch_bounds__(256) conv_bwd_weight_kernel(const int L, const ptrdiff_t E, const int Cin,
-                                                              const int Cout, const float *__restrict__ dout,
-                                                              const float *__restrict__ in, const int relu_in,
-                                                              float *__restrict__ partial) {
-    extern __shared__ float smem[];
-    const int nxe = nxe_of(L);
-    const int co0 = blockIdx.y * kCoChunk;
-    const int nco = min(kCoChunk, Cout - co0);
-    float *sin = smem;                     // [Cin][nxe]
-    float *sd = smem + (size_t)Cin * nxe;   // [nco][nxe]
-    const int nw_chunk = nco * Cin * 27;     // <= 4 * 16 * 27 = 1728 -> <= 7 per thread
-    float acc[8];
+// Weight gradients, partial[block][co][ci][k] = sum over the block's elements and nodes of
+// dout[co][v] act(in[ci][v + off_k]), on the matrix cores in FP32 with K = four nodes.
+//
+// Wide layers (more than three channels on both sides): M = co, N = ci, one 16x16 accumulator per
+// offset; the eight waves of a block take seven offsets and every second step of four nodes each, and
+// the two halves are added in LDS.  What bounds it: 27 products per four nodes (32 cycles each), the LDS
+// reads take a third of that; the next step's operands are read before the current products.
+// blockIdx.y takes a quarter of an element's nodes when the batch holds few elements (NB).  64
+// elements, L = 8, 16 -> 16: 19 us, where one weight per thread with a scalar loop over the nodes took
+// 143 us.
+// C channels of nodes [n0, n1) as unpadded rows of stride RS (channels C .. 15 zero)
+template <int NXE, int RS, int BLOCK>
+__device__ __forceinline__ void conv_stage_rows(float *__restrict__ lds, const float *__restrict__ src, int C,
+                                                bool relu, int n0, int n1) {
+    for (int v = n0 + threadIdx.x; v < n1; v += BLOCK) {
+        float r[16];
 #pragma unroll
-    for (int i = 0; i < 8; i++) acc[i] = 0.f;
+        for (int c = 0; c < 16; c++) r[c] = src[(size_t)(c < C ? c : 0) * NXE + v];
+#pragma unroll
+        for (int c = 0; c < 16; c++) lds[c * RS + v - n0] = c < C ? (relu ? fmaxf(r[c], 0.f) : r[c]) : 0.f;
+    }
+}
+template <int L, int NB>
+__global__ void __launch_bounds__(512)
+    conv_weight_kernel(const ptrdiff_t E, const int Cin, const int Cout, const float *__restrict__ dout,
+                       const float *__restrict__ in, const int relu_in, const ptrdiff_t stride,
+                       float *__restrict__ partial) {
+    using S = ConvShape<L, NB>;
+    constexpr int KW = 7;
+    extern __shared__ __align__(16) float conv_lds[];
+    float *sin = conv_lds, *sd = conv_lds + 16 * S::CSC;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int kw = wave & 3, par = wave >> 2;
+    const int n0 = S::FULL ? 0 : (int)blockIdx.y * NB;
+    const int n1 = S::FULL || n0 + NB > S::NXE ? S::NXE : n0 + NB;
+    int sh[KW];
+    cv_f4 acc[KW];
+#pragma unroll
+    for (int j = 0; j < KW; j++) {
+        const int k = kw * KW + j < 27 ? kw * KW + j : 13;
+        sh[j] = c * S::CSC + (k / 9 - 1) * S::PS + ((k / 3) % 3 - 1) * S::LS + (k % 3 - 1);
+        acc[j] = cv_f4{0.f, 0.f, 0.f, 0.f};
+    }
     for (ptrdiff_t e = blockIdx.x; e < E; e += gridDim.x) {
         __syncthreads();
-        for (int i = threadIdx.x; i < Cin * nxe; i += blockDim.x) {
-            const float v = in[(size_t)e * Cin * nxe + i];
-            sin[i] = relu_in ? fmaxf(v, 0.f) : v;
-        }
-        for (int i = threadIdx.x; i < nco * nxe; i += blockDim.x)
-            sd[i] = dout[((size_t)e * Cout + co0) * nxe + i];
+        ConvStage<L, NB, S::CSC, 16, 512> st;
+        st.load(in + (size_t)e * Cin * S::NXE, Cin, n0, n1);
+        st.clear(sin);
+        conv_stage_rows<S::NXE, S::RSC, 512>(sd, dout + (size_t)e * Cout * S::NXE, Cout, false, n0, n1);
         __syncthreads();
-        for (int j = 0; j < 8; j++) {
-            const int t = threadIdx.x + j * blockDim.x;
-            if (t >= nw_chunk) break;
-            const int col = t / (Cin * 27), r = t - col * Cin * 27, ci = r / 27, k = r - ci * 27;
-            const int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-            const float *d = sd + (size_t)col * nxe;
-            const float *a = sin + (size_t)ci * nxe;
-            float s = 0.f;
-            for (int z = (dz < 0 ? 1 : 0); z <= L - (dz > 0 ? 1 : 0); z++)
-                for (int y = (dy < 0 ? 1 : 0); y <= L - (dy > 0 ? 1 : 0); y++)
-                    for (int x = (dx < 0 ? 1 : 0); x <= L - (dx > 0 ? 1 : 0); x++)
-                        s += d[lidx(L, x, y, z)] * a[lidx(L, x + dx, y + dy, z + dz)];
-            acc[j] += s;
+        st.store(sin, Cin, relu_in != 0, 1.f);
+        __syncthreads();
+        float a, b[KW];
+        auto operands = [&](int v0) {
+            const int v = v0 + g;
+            const bool ok = v < n1;
+            const float x = sd[c * S::RSC + (ok ? v - n0 : 0)];
+            a = ok ? x : 0.f;
+            const float *q = sin + conv_pad<L>(ok ? v : n0, st.zlo);
+#pragma unroll
+            for (int j = 0; j < KW; j++) b[j] = q[sh[j]];
+        };
+        operands(n0 + 4 * par);
+        for (int v0 = n0 + 4 * par; v0 < n1; v0 += 8) {
+            const float ac = a;
+            float bc[KW];
+#pragma unroll
+            for (int j = 0; j < KW; j++) bc[j] = b[j];
+            operands(v0 + 8);  // past the end: a = 0 and node n0's values, not used
+#pragma unroll
+            for (int j = 0; j < KW; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ac, bc[j], acc[j], 0, 0, 0);
         }
     }
-    const int nw = Cout * Cin * 27;
-    for (int j = 0; j < 8; j++) {
-        const int t = threadIdx.x + j * blockDim.x;
-        if (t >= nw_chunk) break;
-        partial[(size_t)blockIdx.x * nw + (size_t)co0 * Cin * 27 + t] = acc[j];
+    // the second half's accumulators through LDS (28 KB: the staging space is at least as large)
+    __syncthreads();
+    cv_f4 *red = (cv_f4 *)conv_lds;
+    if (par)
+#pragma unroll
+        for (int j = 0; j < KW; j++) red[(kw * KW + j) * 64 + lane] = acc[j];
+    __syncthreads();
+    cv_f4 other[KW];
+    if (!par)
+#pragma unroll
+        for (int j = 0; j < KW; j++) other[j] = red[(kw * KW + j) * 64 + lane];
+    __syncthreads();
+    // into [co][ci][k] order in LDS, so that the partial is written in whole lines
+    if (!par)
+#pragma unroll
+        for (int j = 0; j < KW; j++) {
+            const int k = kw * KW + j;
+            if (k >= 27 || c >= Cin) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (4 * g + r < Cout) conv_lds[((4 * g + r) * Cin + c) * 27 + k] = acc[j][r] + other[j][r];
+        }
+    __syncthreads();
+    float *p = partial + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * stride;
+    for (int i = threadIdx.x; i < Cout * Cin * 27; i += 512) p[i] = conv_lds[i];
+}
+
+// Narrow layers (at most three channels on one side, C there, R rows on the other): M = the rows, N =
+// the 27 C (channel, offset) pairs in tiles of 16 columns, each lane with its column's address:
+//   rows = dout, columns = act(in) at v + off_k   (cols_are_dout 0: the first layer)
+//   rows = act(in), columns = dout at v - off_k   (cols_are_dout 1: the last layer)
+// half: as in conv_mfma_kernel, for the first layer's input.
+template <int L, int C, int NB>
+__global__ void __launch_bounds__(256, 2)
+    conv_weight_narrow_kernel(const ptrdiff_t E, const ptrdiff_t half, const int R, const int cols_are_dout,
+                              const float *__restrict__ rows, const float *__restrict__ cols, const int relu_in,
+                              const ptrdiff_t stride, float *__restrict__ partial) {
+    using S = ConvShape<L, NB>;
+    constexpr int NT = (27 * C + 15) / 16;
+    extern __shared__ __align__(16) float conv_lds[];
+    float *sc = conv_lds, *sr = conv_lds + C * S::CSN;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int n0 = S::FULL ? 0 : (int)blockIdx.y * NB;
+    const int n1 = S::FULL || n0 + NB > S::NXE ? S::NXE : n0 + NB;
+    int col[NT];
+    cv_f4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int j = 16 * t + c, ch = j < 27 * C ? j / 27 : 0, k = j < 27 * C ? j % 27 : 13;
+        const int sft = (k / 9 - 1) * S::PS + ((k / 3) % 3 - 1) * S::LS + (k % 3 - 1);
+        col[t] = ch * S::CSN + (cols_are_dout ? -sft : sft);
+        acc[t] = cv_f4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (ptrdiff_t e = blockIdx.x; e < E; e += gridDim.x) {
+        __syncthreads();
+        float sg;
+        const float *src = conv_source(cols, e, half, (size_t)C * S::NXE, sg);
+        ConvStage<L, NB, S::CSN, C, 256> st;
+        st.load(src, C, n0, n1);
+        st.clear(sc);
+        conv_stage_rows<S::NXE, S::RSC, 256>(sr, rows + (size_t)e * R * S::NXE, R, cols_are_dout && relu_in, n0, n1);
+        __syncthreads();
+        st.store(sc, C, !cols_are_dout && relu_in, sg);
+        __syncthreads();
+        // the waves take every fourth step of four nodes; summed over the waves below
+        for (int v0 = n0 + 4 * wave; v0 < n1; v0 += 16) {
+            const int v = v0 + g;
+            const bool ok = v < n1;
+            const float x = sr[c * S::RSC + (ok ? v : n0) - n0];
+            const float a = ok ? x : 0.f;
+            const float *b = sc + conv_pad<L>(ok ? v : n0, st.zlo);
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[col[t]], acc[t], 0, 0, 0);
+        }
+    }
+    // the four waves' accumulators, added in wave order (their LDS lies in the staging space)
+    __syncthreads();
+    cv_f4 *red = (cv_f4 *)conv_lds;
+#pragma unroll
+    for (int t = 0; t < NT; t++) red[(wave * NT + t) * 64 + lane] = acc[t];
+    __syncthreads();
+    float *p = partial + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * stride;
+    for (int t = wave; t < NT; t += 4) {
+        cv_f4 s = red[t * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 4; w++) s += red[(w * NT + t) * 64 + lane];
+        const int j = 16 * t + c;
+        if (j >= 27 * C) continue;
+        const int ch = j / 27, k = j % 27;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = 4 * g + r;
+            if (m < R) p[(cols_are_dout ? ch * R + m : m * C + ch) * 27 + k] = s[r];
+        }
     }
 }
 
-__global__ void sum_partials_f32_kernel(const int nb, const int nw, const float *__restrict__ partial,
-                                        const float scale, float *__restrict__ out) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nw) return;
-    float s = 0.f;
-    for (int b = 0; b < nb; b++) s += partial[(size_t)b * nw + t];
-    out[t] += scale * s;
+// grad[t] = sum over the nb partials, 16 threads per weight (each every 16th partial), in a fixed order;
+// nothing is written unless the target's norm (loss[1]) is positive.  The last block also copies the
+// loss sums, and each block its gradients, into pinned host memory (host: 2 doubles, then the
+// gradients as floats when with_grad).
+__global__ void __launch_bounds__(1024)
+    sum_weight_partials_kernel(const int nb, const int nw, const float *__restrict__ partial,
+                               const double *__restrict__ loss, float *__restrict__ grad, double *__restrict__ host,
+                               const int with_grad) {
+    __shared__ float s[16][65];
+    const int o = threadIdx.x & 63, j = threadIdx.x >> 6, t = blockIdx.x * 64 + o;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x < 2) host[threadIdx.x] = loss[threadIdx.x];
+    if (!(loss[1] > 0)) return;  // uniform
+    float v = 0.f;
+    if (t < nw) {
+#pragma unroll 8
+        for (int b = j; b < nb; b += 16) v += partial[(size_t)b * nw + t];
+    }
+    s[j][o] = v;
+    __syncthreads();
+    if (j == 0 && t < nw) {
+#pragma unroll
+        for (int i = 1; i < 16; i++) v += s[i][o];
+        grad[t] = v;
+        if (with_grad) ((float *)(host + 2))[t] = v;
+    }
 }
 
 // out = a - b (the odd symmetrisation g(z) - g(-z))
@@ -149,23 +468,20 @@ __global__ void sub_halves_kernel(const ptrdiff_t n, const float *__restrict__ a
         out[i] = a[i] - b[i];
 }
 
-// x2 = [x; -x]
-__global__ void make_pm_kernel(const ptrdiff_t n, const float *__restrict__ x, float *__restrict__ x2) {
-    for (ptrdiff_t i = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (ptrdiff_t)gridDim.x * blockDim.x) {
-        x2[i] = x[i];
-        x2[n + i] = -x[i];
-    }
-}
-
-// squared-error partials: part[b] = (sum (o - t)^2, sum t^2) over a fixed grid
-__global__ void __launch_bounds__(256) sq_err_partial_kernel(const ptrdiff_t n, const float *__restrict__ o,
-                                                             const float *__restrict__ t, double *__restrict__ part) {
+// o = a - b (the odd symmetrisation) against the target: part[b] = (sum (o - t)^2, sum t^2) over a
+// fixed grid, o kept as the difference d = o - t
+constexpr int kErrBlocks = 256;
+__global__ void __launch_bounds__(256) sq_err_partial_kernel(const ptrdiff_t n, const float *__restrict__ ga,
+                                                             const float *__restrict__ gb, const float *__restrict__ t,
+                                                             float *__restrict__ diff, double *__restrict__ part) {
     __shared__ double s1[256], s2[256];
     double a = 0, b = 0;
     for (ptrdiff_t i = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (ptrdiff_t)gridDim.x * blockDim.x) {
-        const double d = (double)o[i] - (double)t[i];
+        const float o = ga[i] - gb[i], ti = t[i];
+        const double d = (double)o - (double)ti;
+        diff[i] = o - ti;
         a += d * d;
-        b += (double)t[i] * (double)t[i];
+        b += (double)ti * (double)ti;
     }
     s1[threadIdx.x] = a;
     s2[threadIdx.x] = b;
@@ -183,15 +499,34 @@ __global__ void __launch_bounds__(256) sq_err_partial_kernel(const ptrdiff_t n, 
     }
 }
 
-// dpm = [2 (o - t) / norm; -2 (o - t) / norm]
-__global__ void dloss_kernel(const ptrdiff_t n, const float *__restrict__ o, const float *__restrict__ t,
-                             const float inv_norm, float *__restrict__ dpm) {
+// The sums of the partials (every block sums all of them in the same order: no host round trip between
+// the loss and the backward pass), then dpm = [2 d / norm; -2 d / norm]; block 0 keeps the sums.
+__global__ void __launch_bounds__(256) dloss_kernel(const ptrdiff_t n, const float *__restrict__ diff,
+                                                    const double *__restrict__ part, double *__restrict__ loss,
+                                                    float *__restrict__ dpm) {
+    __shared__ double s1[kErrBlocks], s2[kErrBlocks];
+    s1[threadIdx.x] = part[2 * threadIdx.x];
+    s2[threadIdx.x] = part[2 * threadIdx.x + 1];
+    __syncthreads();
+    for (int st = kErrBlocks / 2; st > 0; st >>= 1) {
+        if (threadIdx.x < st) {
+            s1[threadIdx.x] += s1[threadIdx.x + st];
+            s2[threadIdx.x] += s2[threadIdx.x + st];
+        }
+        __syncthreads();
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        loss[0] = s1[0];
+        loss[1] = s2[0];
+    }
+    const float inv_norm = (float)(1.0 / s2[0]);
     for (ptrdiff_t i = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (ptrdiff_t)gridDim.x * blockDim.x) {
-        const float d = 2.f * (o[i] - t[i]) * inv_norm;
+        const float d = 2.f * diff[i] * inv_norm;
         dpm[i] = d;
         dpm[n + i] = -d;
     }
 }
+static_assert(kErrBlocks == 256, "dloss_kernel loads one partial per thread");
 
 __global__ void adam_kernel(const int n, const float *__restrict__ g, float *__restrict__ w, float *__restrict__ m,
                             float *__restrict__ v, const float lr, const float b1, const float b2, const float eps,
@@ -235,51 +570,179 @@ __global__ void scatter_elements_kernel(const ptrdiff_t E, const int nxe, const 
 }
 
 // ------------------------------------------------------------------ launchers
-static size_t smem_fwd(int L, int Cin, int /*Cout*/) { return sizeof(float) * ((size_t)Cin * nxe_of(L)); }
-
-// blocks per element for n outputs of 256-thread blocks (training batches hold few elements)
-static unsigned conv_split(int n) {
-    const int b = (n + 255) / 256;
-    return (unsigned)(b < 1 ? 1 : (b > 16 ? 16 : b));
+// Dynamic LDS above the default 64 KB needs the function attribute, once per function and device.
+template <auto Fn>
+static int raise_lds_limit(size_t bytes) {
+    static std::atomic<uint64_t> done{0};
+    if (bytes <= 64 * 1024) return SFEM_SUCCESS;
+    int dev = 0;
+    SFEM_AMD_HIP_CHECK(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_acquire) & bit) return SFEM_SUCCESS;
+    SFEM_AMD_HIP_CHECK(
+        hipFuncSetAttribute((const void *)Fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    done.fetch_or(bit, std::memory_order_acq_rel);
+    return SFEM_SUCCESS;
 }
 
-int cnn_conv_forward(int L, ptrdiff_t E, int Cin, int Cout, const float *in, const float *W, int relu_in, float *out,
-                     hipStream_t s) {
-    if (E == 0) return SFEM_SUCCESS;
-    conv_fwd_kernel<<<dim3((unsigned)E, conv_split(Cout * nxe_of(L))), 256, smem_fwd(L, Cin, Cout), s>>>(
-        L, E, Cin, Cout, in, W, relu_in, out);
+// Blocks on whole elements once the batch alone fills the GPU (two blocks on each of 256 CUs); below,
+// blocks on 64 nodes (convolutions) or a quarter of the nodes (weight gradients) of an element.
+constexpr ptrdiff_t kConvFull = 512;
+constexpr int kWhole = 1 << 20;
+// whole steps of four nodes where that leaves the last of four blocks some
+constexpr int conv_quarter(int nxe) { return 3 * ((nxe + 15) / 16 * 4) < nxe ? (nxe + 15) / 16 * 4 : (nxe + 3) / 4; }
+template <int L>
+constexpr int kQuarter = conv_quarter(nxe_of(L));
+static_assert(3 * kQuarter<1> < nxe_of(1) && 4 * kQuarter<1> >= nxe_of(1) && 4 * kQuarter<8> >= nxe_of(8));
+
+template <int L, int Q, int NB>
+static int launch_conv_mfma(ptrdiff_t E, ptrdiff_t half, int C, int M, const float *in, const float *W, int relu_in,
+                            int bwd, const float *mask, float *out, hipStream_t s) {
+    using S = ConvShape<L, NB>;
+    const size_t act = sizeof(float) * (size_t)(Q ? 4 * Q : 1) * S::CSN;
+    const size_t w = Q ? sizeof(float) * (size_t)(bwd ? C : M) * ((bwd ? M : C) * 27 + 2) : 0;
+    const size_t lds = act > w ? act : w;
+    if (raise_lds_limit<conv_mfma_kernel<L, Q, NB>>(lds)) return SFEM_FAILURE;
+    const dim3 grid((unsigned)E, S::FULL ? 1 : (S::NXE + NB - 1) / NB);
+    conv_mfma_kernel<L, Q, NB><<<grid, 256, lds, s>>>(half, C, M, in, W, relu_in, bwd, mask, out);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
+}
+template <int L, int M, int NB>
+static int launch_conv_narrow(ptrdiff_t E, ptrdiff_t half, int C, const float *in, const float *W, int relu_in, int bwd,
+                              const float *mask, float *out, hipStream_t s) {
+    using S = ConvShape<L, NB>;
+    const size_t lds = sizeof(float) * (size_t)16 * S::CSN;
+    if (raise_lds_limit<conv_narrow_kernel<L, M, NB>>(lds)) return SFEM_FAILURE;
+    const dim3 grid((unsigned)E, S::FULL ? 1 : (S::NXE + NB - 1) / NB);
+    conv_narrow_kernel<L, M, NB><<<grid, 256, lds, s>>>(half, C, in, W, relu_in, bwd, mask, out);
+    SFEM_AMD_HIP_CHECK(hipGetLastError());
+    return SFEM_SUCCESS;
+}
+template <int L, int NB>
+static int launch_conv(ptrdiff_t E, ptrdiff_t half, int C, int M, const float *in, const float *W, int relu_in, int bwd,
+                       const float *mask, float *out, hipStream_t s) {
+    // one input channel: the matrix kernel's K runs over the offsets, whatever M; else at most three
+    // output channels run without the matrix cores (conv_narrow_kernel)
+    if (C > 1 && M == 1) return launch_conv_narrow<L, 1, NB>(E, half, C, in, W, relu_in, bwd, mask, out, s);
+    if (C > 1 && M == 2) return launch_conv_narrow<L, 2, NB>(E, half, C, in, W, relu_in, bwd, mask, out, s);
+    if (C > 1 && M == 3) return launch_conv_narrow<L, 3, NB>(E, half, C, in, W, relu_in, bwd, mask, out, s);
+    switch (C == 1 ? 0 : (C + 3) / 4) {
+        case 0: return launch_conv_mfma<L, 0, NB>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 1: return launch_conv_mfma<L, 1, NB>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 2: return launch_conv_mfma<L, 2, NB>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 3: return launch_conv_mfma<L, 3, NB>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 4: return launch_conv_mfma<L, 4, NB>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+    }
+    set_last_error("cnn: at most 16 channels");
+    return SFEM_FAILURE;
+}
+template <int L>
+static int launch_conv_any(ptrdiff_t E, ptrdiff_t half, int C, int M, const float *in, const float *W, int relu_in,
+                           int bwd, const float *mask, float *out, hipStream_t s) {
+    if constexpr (nxe_of(L) > 64)
+        if (E < kConvFull) return launch_conv<L, 64>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+    return launch_conv<L, kWhole>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+}
+static int conv(int L, ptrdiff_t E, ptrdiff_t half, int C, int M, const float *in, const float *W, int relu_in, int bwd,
+                const float *mask, float *out, hipStream_t s) {
+    if (E == 0) return SFEM_SUCCESS;
+    if (M > 16) {
+        set_last_error("cnn: at most 16 channels");
+        return SFEM_FAILURE;
+    }
+    switch (L) {
+        case 1: return launch_conv_any<1>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 2: return launch_conv_any<2>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 3: return launch_conv_any<3>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 4: return launch_conv_any<4>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 5: return launch_conv_any<5>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 6: return launch_conv_any<6>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 7: return launch_conv_any<7>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+        case 8: return launch_conv_any<8>(E, half, C, M, in, W, relu_in, bwd, mask, out, s);
+    }
+    set_last_error("cnn: level must be 1..8");
+    return SFEM_FAILURE;
+}
+
+int cnn_conv_forward(int L, ptrdiff_t E, ptrdiff_t half, int Cin, int Cout, const float *in, const float *W, int relu_in,
+                     float *out, hipStream_t s) {
+    return conv(L, E, half, Cin, Cout, in, W, relu_in, 0, nullptr, out, s);
 }
 
 int cnn_conv_backward_data(int L, ptrdiff_t E, int Cin, int Cout, const float *dout, const float *W, const float *act_in,
                            int relu_in, float *din, hipStream_t s) {
-    if (E == 0) return SFEM_SUCCESS;
-    const size_t smem = sizeof(float) * ((size_t)Cout * nxe_of(L));
-    conv_bwd_data_kernel<<<dim3((unsigned)E, conv_split(Cin * nxe_of(L))), 256, smem, s>>>(L, E, Cin, Cout, dout, W,
-                                                                                         act_in, relu_in, din);
+    return conv(L, E, 0, Cout, Cin, dout, W, 0, 1, relu_in ? act_in : nullptr, din, s);
+}
+
+// the weight-gradient kernels' grid: blocks on elements times blocks per element
+static dim3 weight_grid(ptrdiff_t E) {
+    return E < kConvFull / 4 ? dim3((unsigned)E, 4) : dim3((unsigned)(E < kConvFull ? E : kConvFull), 1);
+}
+int cnn_weight_partials(ptrdiff_t E) {
+    const dim3 g = weight_grid(E);
+    return (int)(g.x * g.y);
+}
+template <int L, int C, int NB>
+static int launch_weight_narrow(ptrdiff_t E, ptrdiff_t half, int R, int cols_are_dout, const float *rows,
+                                const float *cols, int relu_in, ptrdiff_t stride, float *partial, hipStream_t s) {
+    using S = ConvShape<L, NB>;
+    const size_t stage = sizeof(float) * ((size_t)C * S::CSN + 16 * (size_t)S::RSC);
+    const size_t red = 16 * (size_t)64 * 4 * ((27 * C + 15) / 16);
+    const size_t lds = stage > red ? stage : red;
+    if (raise_lds_limit<conv_weight_narrow_kernel<L, C, NB>>(lds)) return SFEM_FAILURE;
+    conv_weight_narrow_kernel<L, C, NB>
+        <<<weight_grid(E), 256, lds, s>>>(E, half, R, cols_are_dout, rows, cols, relu_in, stride, partial);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }
-
-int cnn_conv_backward_weights(int L, ptrdiff_t E, int Cin, int Cout, const float *dout, const float *in, int relu_in,
-                              float *partial, int nblocks, float *dW, hipStream_t s) {
-    const int nw = Cout * Cin * 27;
-    if (kCoChunk * Cin * 27 > 8 * 256) {
-        set_last_error("cnn: layer too wide for the weight-gradient kernel");
+template <int L, int NB>
+static int launch_weight(ptrdiff_t E, ptrdiff_t half, int Cin, int Cout, const float *dout, const float *in, int relu_in,
+                         ptrdiff_t stride, float *partial, hipStream_t s) {
+    using S = ConvShape<L, NB>;
+    if (Cin == 1) return launch_weight_narrow<L, 1, NB>(E, half, Cout, 0, dout, in, relu_in, stride, partial, s);
+    if (Cin == 2) return launch_weight_narrow<L, 2, NB>(E, half, Cout, 0, dout, in, relu_in, stride, partial, s);
+    if (Cin == 3) return launch_weight_narrow<L, 3, NB>(E, half, Cout, 0, dout, in, relu_in, stride, partial, s);
+    if (Cout == 1) return launch_weight_narrow<L, 1, NB>(E, 0, Cin, 1, in, dout, relu_in, stride, partial, s);
+    if (Cout == 2) return launch_weight_narrow<L, 2, NB>(E, 0, Cin, 1, in, dout, relu_in, stride, partial, s);
+    if (Cout == 3) return launch_weight_narrow<L, 3, NB>(E, 0, Cin, 1, in, dout, relu_in, stride, partial, s);
+    const size_t stage = sizeof(float) * 16 * (size_t)(S::CSC + S::RSC), red = 16 * (size_t)64 * 28;
+    const size_t lds = stage > red ? stage : red;
+    if (raise_lds_limit<conv_weight_kernel<L, NB>>(lds)) return SFEM_FAILURE;
+    conv_weight_kernel<L, NB><<<weight_grid(E), 512, lds, s>>>(E, Cin, Cout, dout, in, relu_in, stride, partial);
+    SFEM_AMD_HIP_CHECK(hipGetLastError());
+    return SFEM_SUCCESS;
+}
+template <int L>
+static int launch_weight_any(ptrdiff_t E, ptrdiff_t half, int Cin, int Cout, const float *dout, const float *in,
+                             int relu_in, ptrdiff_t stride, float *partial, hipStream_t s) {
+    if (weight_grid(E).y > 1)
+        return launch_weight<L, kQuarter<L>>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+    return launch_weight<L, kWhole>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+}
+int cnn_conv_backward_weights(int L, ptrdiff_t E, ptrdiff_t half, int Cin, int Cout, const float *dout, const float *in,
+                              int relu_in, ptrdiff_t stride, float *partial, hipStream_t s) {
+    if (E == 0) return SFEM_SUCCESS;
+    if (Cin > 16 || Cout > 16) {
+        set_last_error("cnn: at most 16 channels");
         return SFEM_FAILURE;
     }
-    if (E == 0) return SFEM_SUCCESS;
-    const size_t smem = sizeof(float) * ((size_t)(Cin + kCoChunk) * nxe_of(L));
-    dim3 grid(nblocks, (Cout + kCoChunk - 1) / kCoChunk);
-    conv_bwd_weight_kernel<<<grid, 256, smem, s>>>(L, E, Cin, Cout, dout, in, relu_in, partial);
-    sum_partials_f32_kernel<<<(nw + 255) / 256, 256, 0, s>>>(nblocks, nw, partial, 1.f, dW);
-    SFEM_AMD_HIP_CHECK(hipGetLastError());
-    return SFEM_SUCCESS;
+    switch (L) {
+        case 1: return launch_weight_any<1>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 2: return launch_weight_any<2>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 3: return launch_weight_any<3>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 4: return launch_weight_any<4>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 5: return launch_weight_any<5>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 6: return launch_weight_any<6>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 7: return launch_weight_any<7>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+        case 8: return launch_weight_any<8>(E, half, Cin, Cout, dout, in, relu_in, stride, partial, s);
+    }
+    set_last_error("cnn: level must be 1..8");
+    return SFEM_FAILURE;
 }
-
-int cnn_make_pm(ptrdiff_t n, const float *x, float *x2, hipStream_t s) {
-    make_pm_kernel<<<grid_for(n), kBlock, 0, s>>>(n, x, x2);
+int cnn_sum_weight_partials(int nb, int nw, const float *partial, const double *loss, float *grad, double *host,
+                            int with_grad, hipStream_t s) {
+    sum_weight_partials_kernel<<<(nw + 63) / 64, 1024, 0, s>>>(nb, nw, partial, loss, grad, host, with_grad);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }
@@ -290,26 +753,11 @@ int cnn_sub_halves(ptrdiff_t n, const float *a, const float *b, float *out, hipS
     return SFEM_SUCCESS;
 }
 
-int cnn_sq_err(ptrdiff_t n, const float *o, const float *t, double *ws, double *err_host, double *norm_host,
-               hipStream_t s) {
-    const int nb = 256;
-    sq_err_partial_kernel<<<nb, 256, 0, s>>>(n, o, t, ws);
+int cnn_loss_and_gradient(ptrdiff_t n, const float *ga, const float *gb, const float *t, float *diff, double *part,
+                          double *loss, float *dpm, hipStream_t s) {
+    sq_err_partial_kernel<<<kErrBlocks, 256, 0, s>>>(n, ga, gb, t, diff, part);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
-    double h[2 * 256];
-    SFEM_AMD_HIP_CHECK(hipMemcpyAsync(h, ws, sizeof(h), hipMemcpyDeviceToHost, s));
-    SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
-    double a = 0, b = 0;
-    for (int i = 0; i < nb; i++) {
-        a += h[2 * i];
-        b += h[2 * i + 1];
-    }
-    *err_host = a;
-    *norm_host = b;
-    return SFEM_SUCCESS;
-}
-
-int cnn_dloss(ptrdiff_t n, const float *o, const float *t, float inv_norm, float *dpm, hipStream_t s) {
-    dloss_kernel<<<grid_for(n), kBlock, 0, s>>>(n, o, t, inv_norm, dpm);
+    dloss_kernel<<<grid_for(n), kBlock, 0, s>>>(n, diff, part, loss, dpm);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }

@@ -20,12 +20,14 @@ struct sfem_amd_cnn {
     bool w16_valid{false};
     int step{0};
     // workspaces (grown on demand)
-    DevArray<float> x2, dpm, out2, part;
+    DevArray<float> dpm, diff, part;
     std::vector<DevArray<float> *> acts;  // pre-activations of each layer output, [2E][C][nxe]
     DevArray<float> dA, dB;
-    DevArray<double> ws;
+    DevArray<double> ws;          // 512 loss partials, then the two loss sums
+    double *host{nullptr};        // pinned: the loss sums, then nparams gradients
     ~sfem_amd_cnn() {
         for (auto *a : acts) delete a;
+        if (host) (void)hipHostFree(host);
     }
 };
 
@@ -44,14 +46,15 @@ int check_level(int L) {
     return SFEM_SUCCESS;
 }
 
-// FP32 forward of g on the batch x2 ([2E][io][nxe]); keeps every layer's output in acts.
-int forward_g(sfem_amd_cnn *c, int L, ptrdiff_t E2, hipStream_t s) {
+// FP32 forward of g on z and -z (E elements each); keeps every layer's output ([2E][C][nxe]) in acts.
+int forward_g(sfem_amd_cnn *c, int L, ptrdiff_t E, const float *z, hipStream_t s) {
     const size_t nxe = nxe_of(L);
-    const float *in = c->x2.p;
+    const float *in = z;
     for (int l = 0; l < c->layers; l++) {
         const int ci = c->chans[l], co = c->chans[l + 1];
-        if (ensure(*c->acts[l], (size_t)E2 * co * nxe)) return SFEM_FAILURE;
-        if (cnn_conv_forward(L, E2, ci, co, in, c->W.p + c->offset[l], l > 0, c->acts[l]->p, s)) return SFEM_FAILURE;
+        if (ensure(*c->acts[l], 2 * (size_t)E * co * nxe)) return SFEM_FAILURE;
+        if (cnn_conv_forward(L, 2 * E, l ? 0 : E, ci, co, in, c->W.p + c->offset[l], l > 0, c->acts[l]->p, s))
+            return SFEM_FAILURE;
         in = c->acts[l]->p;
     }
     return SFEM_SUCCESS;
@@ -59,9 +62,7 @@ int forward_g(sfem_amd_cnn *c, int L, ptrdiff_t E2, hipStream_t s) {
 
 int forward_f(sfem_amd_cnn *c, int L, ptrdiff_t E, const float *z, float *out, hipStream_t s) {
     const size_t n = (size_t)E * c->io * nxe_of(L);
-    if (ensure(c->x2, 2 * n)) return SFEM_FAILURE;
-    if (cnn_make_pm((ptrdiff_t)n, z, c->x2.p, s)) return SFEM_FAILURE;
-    if (forward_g(c, L, 2 * E, s)) return SFEM_FAILURE;
+    if (forward_g(c, L, E, z, s)) return SFEM_FAILURE;
     const float *g = c->acts[c->layers - 1]->p;
     return cnn_sub_halves((ptrdiff_t)n, g, g + n, out, s);
 }
@@ -132,7 +133,8 @@ int sfem_amd_cnn_create_channels(int channels, int hidden, int layers, const flo
     SFEM_AMD_HIP_CHECK(hipMemset(c->m.p, 0, sizeof(float) * off));
     SFEM_AMD_HIP_CHECK(hipMemset(c->v.p, 0, sizeof(float) * off));
     for (int l = 0; l < layers; l++) c->acts.push_back(new DevArray<float>());
-    if (c->ws.alloc(512)) return SFEM_FAILURE;
+    if (c->ws.alloc(514)) return SFEM_FAILURE;
+    SFEM_AMD_HIP_CHECK(hipHostMalloc((void **)&c->host, 2 * sizeof(double) + sizeof(float) * off));
     *out = c.release();
     return SFEM_SUCCESS;
 }
@@ -185,35 +187,38 @@ int sfem_amd_cnn_loss_grad(sfem_amd_cnn *c, int L, ptrdiff_t E, const float *z, 
     if (check_level(L)) return SFEM_FAILURE;
     hipStream_t s = as_stream(stream);
     const size_t nxe = nxe_of(L), n = (size_t)E * c->io * nxe;
-    if (ensure(c->out2, n) || ensure(c->dpm, 2 * n)) return SFEM_FAILURE;
-    if (forward_f(c, L, E, z, c->out2.p, s)) return SFEM_FAILURE;
-    double err = 0, norm = 0;
-    if (cnn_sq_err((ptrdiff_t)n, c->out2.p, target, c->ws.p, &err, &norm, s)) return SFEM_FAILURE;
-    SFEM_AMD_REQUIRE(norm > 0, "cnn_loss_grad: zero target");
-    *loss = err / norm;
-    if (cnn_dloss((ptrdiff_t)n, c->out2.p, target, (float)(1.0 / norm), c->dpm.p, s)) return SFEM_FAILURE;
-    SFEM_AMD_HIP_CHECK(hipMemsetAsync(c->grad.p, 0, sizeof(float) * c->nparams, s));
-    const ptrdiff_t E2 = 2 * E;
-    const int nblocks = (int)std::min<ptrdiff_t>(E2, 512);
-    if (ensure(c->part, (size_t)nblocks * 27 * 16 * 16)) return SFEM_FAILURE;
+    const int nblocks = cnn_weight_partials(2 * E);
+    if (ensure(c->diff, n) || ensure(c->dpm, 2 * n) || ensure(c->part, (size_t)nblocks * c->nparams))
+        return SFEM_FAILURE;
+    if (forward_g(c, L, E, z, s)) return SFEM_FAILURE;
+    // the loss stays on the device until the end: the whole step is queued without a host round trip
+    const float *g = c->acts[c->layers - 1]->p;
+    double *sums = c->ws.p + 512;
+    if (cnn_loss_and_gradient((ptrdiff_t)n, g, g + n, target, c->diff.p, c->ws.p, sums, c->dpm.p, s))
+        return SFEM_FAILURE;
     const float *d = c->dpm.p;
     for (int l = c->layers - 1; l >= 0; l--) {
         const int ci = c->chans[l], co = c->chans[l + 1];
-        const float *in = l == 0 ? c->x2.p : c->acts[l - 1]->p;
-        if (cnn_conv_backward_weights(L, E2, ci, co, d, in, l > 0, c->part.p, nblocks, c->grad.p + c->offset[l], s))
+        const float *in = l == 0 ? z : c->acts[l - 1]->p;
+        if (cnn_conv_backward_weights(L, 2 * E, l ? 0 : E, ci, co, d, in, l > 0, (ptrdiff_t)c->nparams,
+                                      c->part.p + c->offset[l], s))
             return SFEM_FAILURE;
         if (l > 0) {
             DevArray<float> &dn = (l % 2) ? c->dA : c->dB;
-            if (ensure(dn, (size_t)E2 * ci * nxe)) return SFEM_FAILURE;
-            if (cnn_conv_backward_data(L, E2, ci, co, d, c->W.p + c->offset[l], c->acts[l - 1]->p, 1, dn.p, s))
+            if (ensure(dn, 2 * (size_t)E * ci * nxe)) return SFEM_FAILURE;
+            if (cnn_conv_backward_data(L, 2 * E, ci, co, d, c->W.p + c->offset[l], c->acts[l - 1]->p, 1, dn.p, s))
                 return SFEM_FAILURE;
             d = dn.p;
         }
     }
-    if (grad_host) {
-        SFEM_AMD_HIP_CHECK(hipMemcpyAsync(grad_host, c->grad.p, sizeof(float) * c->nparams, hipMemcpyDeviceToHost, s));
-        SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
-    }
+    // (no gradient is written for a target without a positive norm)
+    if (cnn_sum_weight_partials(nblocks, (int)c->nparams, c->part.p, sums, c->grad.p, c->host, grad_host ? 1 : 0, s))
+        return SFEM_FAILURE;
+    SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
+    const double err = c->host[0], norm = c->host[1];
+    SFEM_AMD_REQUIRE(norm > 0, "cnn_loss_grad: zero target");
+    *loss = err / norm;
+    if (grad_host) std::copy((const float *)(c->host + 2), (const float *)(c->host + 2) + c->nparams, grad_host);
     return SFEM_SUCCESS;
 }
 

@@ -65,6 +65,63 @@ def test_cnn_loss_and_gradient_match_oracle():
         assert err < 1e-4
 
 
+@pytest.mark.parametrize("L,E,hidden,layers,channels", [
+    (1, 1, 16, 4, 1),    # the smallest element: fewer nodes than a tile, one element split over blocks
+    (8, 2, 16, 4, 1),    # the largest: the last tile holds 9 of 16 nodes
+    (7, 3, 16, 4, 3),    # 512 nodes, no padding node; three input and output channels
+    (3, 5, 5, 3, 3),     # channel counts that fill neither a tile's rows nor a group of four
+    (4, 3, 2, 3, 1),     # narrow layers in the middle
+    (5, 2, 9, 2, 3),     # no hidden-to-hidden layer
+    (6, 1, 13, 5, 3),
+    (2, 300, 16, 4, 1),  # more elements than blocks: one block per element, several elements each
+])
+def test_cnn_fp32_convolutions_match_oracle(L, E, hidden, layers, channels):
+    """Forward, loss and weight gradients of the FP32 path over the shapes its kernels branch on.  Sums
+    of at most 27 * 16 float products per layer: forward 432 * 2^-24 < 3e-5 at worst and ~1e-6
+    with random signs; the gradients sum over up to 2 * 300 * 27 nodes besides."""
+    n = (L + 1) ** 3
+    Ws = [w.astype(np.float32).astype(np.float64) for w in LS.init_weights(hidden, layers, 21, channels=channels)]
+    flat = np.concatenate([w.ravel() for w in Ws]).astype(np.float32)
+    rng = np.random.default_rng(22)
+    shape = (E, n) if channels == 1 else (E, channels, n)
+    z = rng.normal(size=shape).astype(np.float32)
+    t = rng.normal(size=shape).astype(np.float32)
+    cnn = S.CNN(hidden, layers, flat, channels=channels)
+    ref, _ = LS.forward(z.astype(np.float64), Ws, L)
+    out = S.DeviceArray(z.size, np.float32)
+    cnn.forward(L, dev(z), out, mode=0)
+    assert rel(out.numpy().reshape(shape), ref) < 1e-5
+    loss_ref, grads_ref = LS.loss_and_grads(z.astype(np.float64), t.astype(np.float64), Ws, L)
+    loss, g = cnn.loss_grad(L, dev(z), dev(t))
+    assert abs(loss - loss_ref) / loss_ref < 1e-5
+    off = 0
+    for i, gr in enumerate(grads_ref):
+        gi = g[off:off + gr.size].reshape(gr.shape)
+        off += gr.size
+        assert rel(gi, gr) < 1e-4, i
+    # the same batch again: the same words (fixed summation orders)
+    loss2, g2 = cnn.loss_grad(L, dev(z), dev(t))
+    assert loss2 == loss and np.array_equal(g, g2)
+
+
+def test_cnn_zero_target_is_refused_and_keeps_the_gradient():
+    """A target of norm zero is an error, and an Adam step after it still uses the last gradient."""
+    L, E = 2, 2
+    n = (L + 1) ** 3
+    Ws, flat = oracle_weights(3)
+    z = np.random.default_rng(4).normal(size=(E, n)).astype(np.float32)
+    steps = []
+    for bad in (False, True):
+        cnn = S.CNN(16, 4, flat)
+        cnn.loss_grad(L, dev(z), dev(z))
+        if bad:
+            with pytest.raises(S.SfemError, match="zero target"):
+                cnn.loss_grad(L, dev(z), dev(np.zeros_like(z)))
+        cnn.adam_step(1e-3)
+        steps.append(cnn.get_weights())
+    assert np.array_equal(steps[0], steps[1])
+
+
 @pytest.mark.parametrize("L", [1, 2, 3, 4, 5, 6, 7, 8])
 def test_cnn_mfma_inference_matches_fp32(L):
     n = (L + 1) ** 3
