@@ -62,9 +62,10 @@ const char *sfem_amd_last_error(void);
  * arithmetic) or in element form (the shared 24x24 micro-element matrix, on the matrix cores for even
  * levels); 0 picks the stencil form for FP64 operators at levels >= 10, 1 forces the element form,
  * 2 the stencil form (levels 2-6, 8, 10, 12, 16).  Both give the reference's operator; the
- * summation order differs.  "hex8_patches" (default 1): hex8 elasticity applies on meshes of at least
- * 2^15 elements run on element patches (512 elements grown over shared nodes, accumulated in LDS,
- * patch-boundary nodes summed in a fixed order); 0 runs one element per lane with atomics.
+ * summation order differs.  "hex8_patches" (default 1): tet4 and hex8 applies on meshes of at least
+ * 2^15 elements run on element patches (512 or 2,048 elements grown over shared nodes, accumulated in
+ * LDS, patch-boundary nodes summed in a fixed order; the partition is made by a mesh's first apply, on
+ * the host); 0 runs one element per lane with atomics.
  * "mixed_cg" (default 1): flexible CGs created afterwards around a bridged FP32 preconditioner keep
  * z in FP32 (see sfem_amd_cg_create; the same iterates); 0 runs them through the bridge's casts. */
 int sfem_amd_set_option(const char *name, int value);

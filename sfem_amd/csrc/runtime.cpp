@@ -186,148 +186,25 @@ const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t 
     return slot.get();
 }
 
-// Element patches of a tet4/hex8 mesh: breadth-first growth over shared nodes, at most kP elements
-// each, the next seed taken from the unassigned neighbours of the previous patch (lowest id first),
-// else the lowest unassigned element.  On a structured box of hexahedra the patches come out as
-// compact blocks (about 1.56 patch nodes per element at 512 elements, against 1.42 for a perfect
-// 8^3 cube and 8 for no sharing).
-static_assert(ElementPatches::kP == kPatchElements, "patch size of the host partition and the kernels");
-const ElementPatches *mesh_patches(const sfem_amd_mesh *m) {
-    if (m->patches) return m->patches.get();
-    if (m->type == SFEM_AMD_SSHEX8 || m->E <= 0 || m->nv <= 0) return nullptr;
-    constexpr int P = ElementPatches::kP;
-    const int nv = m->nv;
-    const ptrdiff_t E = m->E, N = m->nnodes;
-    if ((double)E * nv >= 2147483647.0 || N >= 2147483647) {
-        set_last_error("element patches: mesh exceeds int32 indexing");
-        return nullptr;
-    }
-    std::vector<int32_t> el((size_t)E * nv);  // SoA [nv][E]
-    if (hipMemcpy(el.data(), m->idx.p, sizeof(int32_t) * el.size(), hipMemcpyDeviceToHost) != hipSuccess) {
-        set_last_error("element patches: connectivity download failed");
-        return nullptr;
-    }
-    // node -> elements
-    std::vector<int32_t> n2e_off((size_t)N + 1, 0);
-    for (const int32_t g : el) n2e_off[(size_t)g + 1]++;
-    for (ptrdiff_t g = 0; g < N; g++) n2e_off[g + 1] += n2e_off[g];
-    std::vector<int32_t> n2e((size_t)E * nv), fill(n2e_off.begin(), n2e_off.end() - 1);
-    for (int v = 0; v < nv; v++)
-        for (ptrdiff_t e = 0; e < E; e++) n2e[fill[el[(size_t)v * E + e]]++] = (int32_t)e;
-    // grow the patches
-    std::vector<int32_t> patch_of((size_t)E, -1), order, pstart, queue, hint;
-    order.reserve(E);
-    ptrdiff_t seed = 0;
-    for (;;) {
-        int32_t s0 = -1;
-        while (!hint.empty()) {
-            const int32_t c = hint.back();
-            hint.pop_back();
-            if (patch_of[c] < 0) {
-                s0 = c;
-                break;
-            }
-        }
-        if (s0 < 0) {
-            while (seed < E && patch_of[seed] >= 0) seed++;
-            if (seed >= E) break;
-            s0 = (int32_t)seed;
-        }
-        const int32_t pid = (int32_t)pstart.size();
-        pstart.push_back((int32_t)order.size());
-        queue.assign(1, s0);
-        patch_of[s0] = pid;
-        for (size_t head = 0; head < queue.size(); head++) {
-            const int32_t e = queue[head];
-            for (int v = 0; v < nv && queue.size() < (size_t)P; v++) {
-                const int32_t g = el[(size_t)v * E + e];
-                for (int32_t k = n2e_off[g]; k < n2e_off[g + 1] && queue.size() < (size_t)P; k++) {
-                    const int32_t f = n2e[k];
-                    if (patch_of[f] < 0) {
-                        patch_of[f] = pid;
-                        queue.push_back(f);
-                    }
-                }
-            }
-        }
-        order.insert(order.end(), queue.begin(), queue.end());
-        // unassigned neighbours of this patch, lowest id popped first
-        hint.clear();
-        for (const int32_t e : queue)
-            for (int v = 0; v < nv; v++) {
-                const int32_t g = el[(size_t)v * E + e];
-                for (int32_t k = n2e_off[g]; k < n2e_off[g + 1]; k++)
-                    if (patch_of[n2e[k]] < 0) hint.push_back(n2e[k]);
-            }
-        std::sort(hint.begin(), hint.end(), std::greater<int32_t>());
-        hint.erase(std::unique(hint.begin(), hint.end()), hint.end());
-    }
-    const ptrdiff_t np = (ptrdiff_t)pstart.size();
-    pstart.push_back((int32_t)E);
-    // local numbering, patch node lists and which nodes other patches share
-    std::vector<int32_t> count((size_t)np), perm((size_t)np * P, -1), node_off(1, 0), nodes;
-    std::vector<uint16_t> lconn((size_t)np * nv * P, 0);
-    std::vector<int32_t> local((size_t)N, -1), inside((size_t)N, 0);
-    std::vector<uint8_t> shared_flag;
-    int maxloc = 0;
-    for (ptrdiff_t p = 0; p < np; p++) {
-        const int32_t b = pstart[p], cnt = pstart[p + 1] - b;
-        count[p] = cnt;
-        const size_t first = nodes.size();
-        for (int32_t t = 0; t < cnt; t++) {
-            const int32_t e = order[(size_t)b + t];
-            perm[(size_t)p * P + t] = e;
-            for (int v = 0; v < nv; v++) {
-                const int32_t g = el[(size_t)v * E + e];
-                if (local[g] < 0) {
-                    local[g] = (int32_t)(nodes.size() - first);
-                    nodes.push_back(g);
-                }
-                inside[g]++;
-                lconn[((size_t)p * nv + v) * P + t] = (uint16_t)local[g];
-            }
-        }
-        const int nloc = (int)(nodes.size() - first);
-        if (nloc > 65535) {
-            set_last_error("element patches: more than 65535 nodes in a patch");
-            return nullptr;
-        }
-        maxloc = std::max(maxloc, nloc);
-        for (size_t i = first; i < nodes.size(); i++) {
-            const int32_t g = nodes[i];
-            shared_flag.push_back(inside[g] < n2e_off[g + 1] - n2e_off[g] ? 1 : 0);
-            local[g] = -1;
-            inside[g] = 0;
-        }
-        node_off.push_back((int32_t)nodes.size());
-    }
-    // node-sorted partial positions of the shared entries (patch order within a node)
-    std::vector<int32_t> pcount((size_t)N + 1, 0);
-    for (size_t i = 0; i < nodes.size(); i++)
-        if (shared_flag[i]) pcount[(size_t)nodes[i] + 1]++;
-    std::vector<int32_t> bnode, boff(1, 0), start((size_t)N, -1);
-    for (ptrdiff_t g = 0; g < N; g++)
-        if (pcount[g + 1]) {
-            start[g] = boff.back();
-            bnode.push_back((int32_t)g);
-            boff.push_back(boff.back() + pcount[g + 1]);
-        }
-    std::vector<int32_t> bslot(nodes.size(), -1);
-    for (size_t i = 0; i < nodes.size(); i++)
-        if (shared_flag[i]) bslot[i] = start[nodes[i]]++;
-    auto pt = std::make_unique<ElementPatches>();
-    pt->npatch = np;
-    pt->maxloc = maxloc;
-    pt->nodes_per_element = (double)nodes.size() / (double)E;
-    pt->nparts = boff.back();
-    pt->boundary.n = (ptrdiff_t)bnode.size();
-    if (pt->count.upload(count.data(), count.size()) || pt->perm.upload(perm.data(), perm.size()) ||
-        pt->lconn.upload(lconn.data(), lconn.size()) || pt->node_off.upload(node_off.data(), node_off.size()) ||
-        pt->nodes.upload(nodes.data(), nodes.size()) || pt->bslot.upload(bslot.data(), bslot.size()) ||
-        pt->boundary.node.upload(bnode.data(), bnode.size()) || pt->boundary.off.upload(boff.data(), boff.size()))
-        return nullptr;
-    m->patches = std::move(pt);
-    return m->patches.get();
+// ----------------------------------------------------------------- element patches
+static PatchView patch_view(const ElementPatches &pt, ptrdiff_t E) {
+    PatchView pv;
+    pv.npatch = pt.npatch;
+    pv.E = E;
+    pv.maxloc = pt.maxloc;
+    pv.start = pt.start.p;
+    pv.node_off = pt.node_off.p;
+    pv.nodes = pt.nodes.p;
+    pv.bslot = pt.bslot.p;
+    pv.lconn = pt.lconn.p;
+    return pv;
+}
+static SkeletonMap patch_boundary(const ElementPatches &pt) {
+    SkeletonMap sk{};
+    sk.node = pt.boundary.node.p;
+    sk.off = pt.boundary.off.p;
+    sk.n = pt.boundary.n;
+    return sk;
 }
 
 // ----------------------------------------------------------------- Laplacian
@@ -339,6 +216,10 @@ struct LaplacianOp final : OpBase {
     DevArray<float> coeff;
     DevArray<T> part;  // sshex8: skeleton contributions [E][sk_count(L)]
     DevArray<double> Kem;  // sshex8 stored sub-element matrices [E][64] (instead of the FFF)
+    // tet4/hex8 on element patches: the words in patch-slot order, shared-node partials
+    DevArray<float> fffp, coeffp;
+    DevArray<double> ppart;
+    int patch_state{0};  // 0 not yet tried, 1 ready, -1 not applicable
     int real_type() const override { return std::is_same<T, double>::value ? SFEM_AMD_FLOAT64 : SFEM_AMD_FLOAT32; }
     ptrdiff_t rows() const override { return m->nnodes; }
 
@@ -367,6 +248,8 @@ struct LaplacianOp final : OpBase {
         SkeletonMap sk = skeleton_of(m);
         sk.cmask = cmask;
         if constexpr (std::is_same<T, double>::value) {
+            if (m->type != SFEM_AMD_SSHEX8 && g_hex8_patches && m->E >= kPatchMinElements && patches_ready(s))
+                return apply_patches(x, y, s);
             switch (m->type) {
                 case SFEM_AMD_TET4:
                     return tet4_laplacian_apply(m->E, m->idx.p, fff32.p, x, y, s);
@@ -380,6 +263,26 @@ struct LaplacianOp final : OpBase {
             return sshex8_laplacian_apply<float, uint16_t>(m->level, m->E, m->idx.p, fff16.p, m->E, nullptr, Kem.p,
                                                            x, y, part.p, sk, s, ow, g_atomic_skeleton);
         }
+    }
+    // tet4/hex8: the element patches of the mesh and this operator's words in their slot order (first use)
+    bool patches_ready(hipStream_t s) {
+        if (patch_state) return patch_state > 0;
+        if (!may_build_patches(s)) return false;
+        patch_state = -1;
+        const ElementPatches *pt = mesh_cells(m, s);
+        if (!pt || patch_lds_bytes(pt->maxloc, 1, sizeof(double)) > kPatchLdsLimit) return false;
+        bool ok = !ppart.alloc((size_t)pt->nparts + 1) && !fffp.alloc((size_t)6 * m->E) &&
+                  !patch_gather_rows<float>(6, m->E, pt->perm.p, fff32.p, fffp.p, s);
+        if (ok && coeff.p)
+            ok = !coeffp.alloc(m->E) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
+        if (!ok || hipStreamSynchronize(s) != hipSuccess) return false;
+        patch_state = 1;
+        return true;
+    }
+    int apply_patches(const T *x, T *y, hipStream_t s) {
+        const ElementPatches *pt = m->cells.get();
+        if (laplacian_apply_patches(m->nv, patch_view(*pt, m->E), fffp.p, coeffp.p, x, y, ppart.p, s)) return SFEM_FAILURE;
+        return skeleton_gather<T>(patch_boundary(*pt), 1, ppart.p, y, s, 0, 1);
     }
     int diag(void *dv, hipStream_t s) override {
         T *d = (T *)dv;
@@ -536,35 +439,29 @@ struct ElasticityOp final : OpBase {
     // hex8: the element patches of the mesh and this operator's words in their slot order (first use)
     bool patches_ready(hipStream_t s) {
         if (patch_state) return patch_state > 0;
+        if (!may_build_patches(s)) return false;
         patch_state = -1;
-        const ElementPatches *pt = mesh_patches(m);
-        if (!pt || hex8_patch_lds_bytes(pt->maxloc, sizeof(T)) > kPatchLdsLimit) return false;
-        const ptrdiff_t Ep = pt->npatch * ElementPatches::kP;
+        const ElementPatches *pt = mesh_patches(m, s);
+        if (!pt || patch_lds_bytes(pt->maxloc, 3, sizeof(T)) > kPatchLdsLimit) return false;
+        const ptrdiff_t Ep = m->E;
         bool ok = ppart.alloc((size_t)pt->nparts * 3 + 3) == SFEM_SUCCESS;
         if constexpr (std::is_same<T, double>::value)
             ok = ok && !adjp.alloc((size_t)9 * Ep) && !detp.alloc(Ep) &&
-                 !patch_gather_rows<float>(9, m->E, Ep, pt->perm.p, adj.p, adjp.p, s) &&
-                 !patch_gather_rows<float>(1, m->E, Ep, pt->perm.p, det.p, detp.p, s);
+                 !patch_gather_rows<float>(9, m->E, pt->perm.p, adj.p, adjp.p, s) &&
+                 !patch_gather_rows<float>(1, m->E, pt->perm.p, det.p, detp.p, s);
         else
             ok = ok && !adjp16.alloc((size_t)9 * Ep) && !detp16.alloc(Ep) &&
-                 !patch_gather_rows<uint16_t>(9, m->E, Ep, pt->perm.p, adj16.p, adjp16.p, s) &&
-                 !patch_gather_rows<uint16_t>(1, m->E, Ep, pt->perm.p, det16.p, detp16.p, s);
+                 !patch_gather_rows<uint16_t>(9, m->E, pt->perm.p, adj16.p, adjp16.p, s) &&
+                 !patch_gather_rows<uint16_t>(1, m->E, pt->perm.p, det16.p, detp16.p, s);
         if (ok && coeff.p)
-            ok = !coeffp.alloc(Ep) && !patch_gather_rows<float>(1, m->E, Ep, pt->perm.p, coeff.p, coeffp.p, s);
+            ok = !coeffp.alloc(Ep) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
         if (!ok || hipStreamSynchronize(s) != hipSuccess) return false;
         patch_state = 1;
         return true;
     }
     int apply_patches(const void *xv, void *yv, hipStream_t s) {
         const ElementPatches *pt = m->patches.get();
-        PatchView pv;
-        pv.npatch = pt->npatch;
-        pv.maxloc = pt->maxloc;
-        pv.count = pt->count.p;
-        pv.node_off = pt->node_off.p;
-        pv.nodes = pt->nodes.p;
-        pv.bslot = pt->bslot.p;
-        pv.lconn = pt->lconn.p;
+        const PatchView pv = patch_view(*pt, m->E);
         int err;
         if constexpr (std::is_same<T, double>::value)
             err = hex8_elasticity_apply_patches<double, float>(pv, adjp.p, detp.p, coeffp.p, mu, lambda,
@@ -573,11 +470,7 @@ struct ElasticityOp final : OpBase {
             err = hex8_elasticity_apply_patches<float, uint16_t>(pv, adjp16.p, detp16.p, coeffp.p, mu, lambda,
                                                                  (const float *)xv, (float *)yv, ppart.p, s);
         if (err) return err;
-        SkeletonMap sk{};
-        sk.node = pt->boundary.node.p;
-        sk.off = pt->boundary.off.p;
-        sk.n = pt->boundary.n;
-        return skeleton_gather<T>(sk, 3, ppart.p, (T *)yv, s, 0, 1);
+        return skeleton_gather<T>(patch_boundary(*pt), 3, ppart.p, (T *)yv, s, 0, 1);
     }
     int hex8_diag(int block, void *d, hipStream_t s) {
         if constexpr (std::is_same<T, double>::value)

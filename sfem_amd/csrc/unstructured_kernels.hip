@@ -1,4 +1,4 @@
-// gfx950 kernels for tet4 and hex8 meshes: one element per lane.
+// gfx950 kernels for tet4 and hex8 meshes: one element per lane, or a patch of elements per workgroup.
 //
 // Device layout: idx int32 SoA [nv][E] and geometry SoA [k][E] (the layout of the
 // reference's device path, operators/cuda/cu_laplacian.hpp fff_stride), so a wave
@@ -269,112 +269,224 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Patch-wise (ElementPatches): one workgroup per patch of up to kPatch elements.  The patch's nodes
+// Patch-wise (ElementPatches): one workgroup per patch.  The patch's nodes
 // are gathered into LDS once (x), the elements accumulate into LDS (y, LDS atomics), then each patch
 // node is either added to y (the patch's own nodes: no other workgroup touches them) or written to
 // its node-sorted partial slot (nodes shared with other patches; summed by skeleton_gather).  The
 // geometry and coefficient words are stored in patch-slot order, so every read of them coalesces.
 // The LDS accumulator is FP64 for both value types: ds_add_f64 keeps pace with the arithmetic, while
 // ds_add_f32 measured 7x the LDS busy cycles and 100x the LDS wait of the whole FP64 kernel here.
-template <typename T, typename G, int kPatch>
-__global__ void __launch_bounds__(256)
-    hex8_elasticity_patch_kernel(const int32_t *__restrict__ count, const uint16_t *__restrict__ lconn,
-                                 const int32_t *__restrict__ node_off, const int32_t *__restrict__ nodes,
-                                 const int32_t *__restrict__ bslot, const ptrdiff_t Epad, const G *__restrict__ adjp,
-                                 const G *__restrict__ detp, const float *__restrict__ coeffp, const double mu0,
-                                 const double lambda0, const T *__restrict__ x, T *__restrict__ y,
-                                 T *__restrict__ part) {
-    extern __shared__ __align__(16) unsigned char patch_lds[];
-    // workgroups go to the 8 XCDs round-robin: give XCD k the k-th contiguous range of patches, so
-    // neighbouring patches (consecutive in growth order, sharing boundary nodes) meet in one L2
-    const ptrdiff_t b = blockIdx.x, per = gridDim.x / 8, rem = gridDim.x % 8;
-    const int xcd = (int)(b % 8);
-    const ptrdiff_t p = xcd * per + (xcd < rem ? xcd : rem) + b / 8;
-    const int off = node_off[p], nloc = node_off[p + 1] - off;
-    double *sy = reinterpret_cast<double *>(patch_lds);
-    T *sx = reinterpret_cast<T *>(sy + 3 * nloc);
-    // NB patch nodes per thread at a time: their ids, then their x values, each batch issued together
-    constexpr int NB = 4;
-    for (int i0 = threadIdx.x; i0 < nloc; i0 += NB * blockDim.x) {
-        ptrdiff_t gg[NB];
+
+// patch nodes per thread at a time: their ids, then their values, each batch issued together
+constexpr int kPatchBatch = 4;
+template <typename T, int VS>
+__device__ __forceinline__ void patch_gather_x(const int nloc, const int32_t *__restrict__ nodes,
+                                               const T *__restrict__ x, T *__restrict__ sx, double *__restrict__ sy) {
+    for (int i0 = threadIdx.x; i0 < nloc; i0 += kPatchBatch * blockDim.x) {
+        ptrdiff_t gg[kPatchBatch];
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
+        for (int b = 0; b < kPatchBatch; b++) {
             const int i = i0 + b * blockDim.x;
-            gg[b] = nodes[off + (i < nloc ? i : 0)];
+            gg[b] = nodes[i < nloc ? i : 0];
         }
-        T xv[NB][3];
+        T xv[kPatchBatch][VS];
 #pragma unroll
-        for (int b = 0; b < NB; b++)
+        for (int b = 0; b < kPatchBatch; b++)
 #pragma unroll
-            for (int c = 0; c < 3; c++) xv[b][c] = x[gg[b] * 3 + c];
+            for (int c = 0; c < VS; c++) xv[b][c] = x[gg[b] * VS + c];
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
+        for (int b = 0; b < kPatchBatch; b++) {
             const int i = i0 + b * blockDim.x;
             if (i < nloc)
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    sx[i * 3 + c] = xv[b][c];
-                    sy[i * 3 + c] = 0;
+                for (int c = 0; c < VS; c++) {
+                    sx[i * VS + c] = xv[b][c];
+                    sy[i * VS + c] = 0;
                 }
         }
     }
-    __syncthreads();
-    const int cnt = count[p];
-    for (int t = threadIdx.x; t < cnt; t += blockDim.x) {
-        const ptrdiff_t slot = p * kPatch + t;
-        int l[8];
+}
+// the same batches: ids and boundary slots, then the old y (read for every node of the batch: a
+// valid entry, used for the patch's own nodes), then the stores
+template <typename T, int VS>
+__device__ __forceinline__ void patch_scatter_y(const int nloc, const int32_t *__restrict__ nodes,
+                                                const int32_t *__restrict__ bslot, const double *__restrict__ sy,
+                                                T *__restrict__ y, T *__restrict__ part) {
+    for (int i0 = threadIdx.x; i0 < nloc; i0 += kPatchBatch * blockDim.x) {
+        ptrdiff_t gg[kPatchBatch], bb[kPatchBatch];
 #pragma unroll
-        for (int k = 0; k < 8; k++) l[k] = lconn[(p * 8 + k) * kPatch + t];
+        for (int b = 0; b < kPatchBatch; b++) {
+            const int i = i0 + b * blockDim.x, ii = i < nloc ? i : 0;
+            gg[b] = nodes[ii];
+            bb[b] = bslot[ii];
+        }
+        T yo[kPatchBatch][VS];
+#pragma unroll
+        for (int b = 0; b < kPatchBatch; b++)
+#pragma unroll
+            for (int c = 0; c < VS; c++) yo[b][c] = y[gg[b] * VS + c];
+#pragma unroll
+        for (int b = 0; b < kPatchBatch; b++) {
+            const int i = i0 + b * blockDim.x;
+            if (i >= nloc) continue;
+#pragma unroll
+            for (int c = 0; c < VS; c++) {
+                const T v = (T)sy[i * VS + c];
+                if (bb[b] < 0)
+                    y[gg[b] * VS + c] = yo[b][c] + v;
+                else
+                    part[bb[b] * VS + c] = v;
+            }
+        }
+    }
+}
+// the local nodes of a slot's NV corners, four 16-bit ids to a word pair
+template <int NV>
+__device__ __forceinline__ void patch_local_nodes(const uint16_t *__restrict__ lconn, ptrdiff_t E, ptrdiff_t slot,
+                                                  int (&l)[NV]) {
+#pragma unroll
+    for (int q = 0; q < NV / 4; q++) {
+        const ushort4 w = reinterpret_cast<const ushort4 *>(lconn)[q * E + slot];
+        l[4 * q] = w.x, l[4 * q + 1] = w.y, l[4 * q + 2] = w.z, l[4 * q + 3] = w.w;
+    }
+}
+
+template <typename T, typename G>
+__global__ void __launch_bounds__(256)
+    hex8_elasticity_patch_kernel(const PatchView pv, const G *__restrict__ adjp, const G *__restrict__ detp,
+                                 const float *__restrict__ coeffp, const double mu0, const double lambda0,
+                                 const T *__restrict__ x, T *__restrict__ y, T *__restrict__ part) {
+    extern __shared__ __align__(16) unsigned char patch_lds[];
+    const ptrdiff_t p = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const int off = pv.node_off[p], nloc = pv.node_off[p + 1] - off;
+    double *sy = reinterpret_cast<double *>(patch_lds);
+    T *sx = reinterpret_cast<T *>(sy + 3 * nloc);
+    patch_gather_x<T, 3>(nloc, pv.nodes + off, x, sx, sy);
+    __syncthreads();
+    const int first = pv.start[p], cnt = pv.start[p + 1] - first;
+    for (int t = threadIdx.x; t < cnt; t += blockDim.x) {
+        const ptrdiff_t slot = first + t;
+        int l[8];
+        patch_local_nodes<8>(pv.lconn, pv.E, slot, l);
         double a64[9];
 #pragma unroll
-        for (int k = 0; k < 9; k++) a64[k] = load_geom<G>(adjp, k * Epad + slot);
+        for (int k = 0; k < 9; k++) a64[k] = load_geom<G>(adjp, k * pv.E + slot);
         hex8_elasticity_sf_element<T>(
             a64, load_geom<G>(detp, slot), coeffp ? (double)coeffp[slot] : 1.0, mu0, lambda0,
             [&](int n, int d) { return sx[l[n] * 3 + d]; },
             [&](int n, int d, T val) { atomicAdd(&sy[l[n] * 3 + d], (double)val); });
     }
     __syncthreads();
-    // the same batches: ids and boundary slots, then the old y (read for every node of the batch: a
-    // valid entry, used for the patch's own nodes), then the stores
-    for (int i0 = threadIdx.x; i0 < nloc; i0 += NB * blockDim.x) {
-        ptrdiff_t gg[NB], bb[NB];
+    patch_scatter_y<T, 3>(nloc, pv.nodes + off, pv.bslot + off, sy, y, part);
+}
+
+// hex8 Laplacian of one element, sum-factorised as the elasticity element above.  The x-derivative at
+// point (qz, qy, qx) does not depend on qx, so the sums over a direction's own index that the
+// transpose needs act on the derivatives directly: rx = sum_qx t_x = 2 f0 gx + f1 sum_qx gy + f2 sum_qx gz.
+// About 150 operations per element against 600 for the point loop.  f: FFF times coefficient / 8.
+template <typename Load, typename Store>
+__device__ __forceinline__ void hex8_laplacian_sf_element(const double f[6], Load load, Store store) {
+    constexpr int kT[8] = {0, 1, 3, 2, 4, 5, 7, 6};  // hex8 corner n -> iz*4 + iy*2 + ix
+    const double g0 = 0.5 - 0.28867513459481288225, g1 = 0.5 + 0.28867513459481288225;
+    double u[8];
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const int i = i0 + b * blockDim.x, ii = i < nloc ? i : 0;
-            gg[b] = nodes[off + ii];
-            bb[b] = bslot[off + ii];
+    for (int n = 0; n < 8; n++) u[kT[n]] = load(n);
+    double gx[2][2], gy[2][2], gz[2][2];  // [qz][qy], [qz][qx], [qy][qx]
+    sf_interp2<double>(u[1] - u[0], u[3] - u[2], u[5] - u[4], u[7] - u[6], g0, g1, gx);
+    sf_interp2<double>(u[2] - u[0], u[3] - u[1], u[6] - u[4], u[7] - u[5], g0, g1, gy);
+    sf_interp2<double>(u[4] - u[0], u[5] - u[1], u[6] - u[2], u[7] - u[3], g0, g1, gz);
+    double rx[2][2], ry[2][2], rz[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            // (i, j) = (qz, qy), (qz, qx), (qy, qx)
+            rx[i][j] = 2 * f[0] * gx[i][j] + f[1] * (gy[i][0] + gy[i][1]) + f[2] * (gz[j][0] + gz[j][1]);
+            ry[i][j] = 2 * f[3] * gy[i][j] + f[1] * (gx[i][0] + gx[i][1]) + f[4] * (gz[0][j] + gz[1][j]);
+            rz[i][j] = 2 * f[5] * gz[i][j] + f[2] * (gx[0][i] + gx[1][i]) + f[4] * (gy[0][j] + gy[1][j]);
         }
-        T yo[NB][3];
+    double o[8], a00, a01, a10, a11;
+    sf_interp2_t<double>(rx, g0, g1, a00, a01, a10, a11);  // at (iz, iy): +x corner gets +, -x gets -
+    o[1] = a00, o[0] = -a00, o[3] = a01, o[2] = -a01, o[5] = a10, o[4] = -a10, o[7] = a11, o[6] = -a11;
+    sf_interp2_t<double>(ry, g0, g1, a00, a01, a10, a11);  // at (iz, ix)
+    o[2] += a00, o[0] -= a00, o[3] += a01, o[1] -= a01, o[6] += a10, o[4] -= a10, o[7] += a11, o[5] -= a11;
+    sf_interp2_t<double>(rz, g0, g1, a00, a01, a10, a11);  // at (iy, ix)
+    o[4] += a00, o[0] -= a00, o[5] += a01, o[1] -= a01, o[6] += a10, o[2] -= a10, o[7] += a11, o[3] -= a11;
 #pragma unroll
-        for (int b = 0; b < NB; b++)
+    for (int n = 0; n < 8; n++) store(n, o[kT[n]]);
+}
+
+// The Laplacian over patches.  The element-wise kernels are bound by their global FP64 atomics (4 or 8
+// per element), scattered meshes also by the gathers of x; here both stay in LDS.  What bounds this one:
+// latency (two dependent loads before the sweep, two after it) and the ds_add_f64 of the sweep.
+// 1.93M hexahedra: 54 us and 10 us of gather (696 us element-wise); 2.41M shuffled tetrahedra: 36 and 5 us
+// (417 us).
+template <int NV>
+__global__ void __launch_bounds__(256)
+    laplacian_patch_kernel(const PatchView pv, const float *__restrict__ fffp, const float *__restrict__ coeffp,
+                           const double *__restrict__ x, double *__restrict__ y, double *__restrict__ part) {
+    extern __shared__ __align__(16) unsigned char patch_lds[];
+    const ptrdiff_t p = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const int off = pv.node_off[p], nloc = pv.node_off[p + 1] - off;
+    const int first = pv.start[p], cnt = pv.start[p + 1] - first;
+    double *sy = reinterpret_cast<double *>(patch_lds), *sx = sy + nloc;
+    // a thread's elements two at a time, the first two loaded before the gather (absent ones re-read the
+    // patch's first slot and are not added)
+    constexpr int EB = 2;
+    int l[EB][NV];
+    float w[EB][6], c[EB];
+    auto load = [&](int t0) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) yo[b][c] = y[gg[b] * 3 + c];
+        for (int b = 0; b < EB; b++) {
+            const int t = t0 + b * 256 < cnt ? t0 + b * 256 : 0;
+            const ptrdiff_t slot = first + t;
+            patch_local_nodes<NV>(pv.lconn, pv.E, slot, l[b]);
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const int i = i0 + b * blockDim.x;
-            if (i >= nloc) continue;
+            for (int k = 0; k < 6; k++) w[b][k] = fffp[k * pv.E + slot];
+            c[b] = coeffp ? coeffp[slot] : 1.f;
+        }
+    };
+    load(threadIdx.x);
+    patch_gather_x<double, 1>(nloc, pv.nodes + off, x, sx, sy);
+    __syncthreads();
+    for (int t0 = threadIdx.x; t0 < cnt; t0 += EB * 256) {
+        if (t0 != (int)threadIdx.x) load(t0);
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const T v = (T)sy[i * 3 + c];
-                if (bb[b] < 0)
-                    y[gg[b] * 3 + c] = yo[b][c] + v;
-                else
-                    part[bb[b] * 3 + c] = v;
+        for (int b = 0; b < EB; b++) {
+            if (t0 + b * 256 >= cnt) continue;
+            double f[6];
+            if constexpr (NV == 8) {
+#pragma unroll
+                for (int k = 0; k < 6; k++) f[k] = (double)w[b][k] * ((double)c[b] * 0.125);
+                hex8_laplacian_sf_element(
+                    f, [&](int n) { return sx[l[b][n]]; }, [&](int n, double v) { atomicAdd(&sy[l[b][n]], v); });
+            } else {
+#pragma unroll
+                for (int k = 0; k < 6; k++) f[k] = (double)w[b][k];
+                const double u0 = sx[l[b][0]];
+                const double h0 = sx[l[b][1]] - u0, h1 = sx[l[b][2]] - u0, h2 = sx[l[b][3]] - u0;
+                const double t1 = f[0] * h0 + f[1] * h1 + f[2] * h2;
+                const double t2 = f[1] * h0 + f[3] * h1 + f[4] * h2;
+                const double t3 = f[2] * h0 + f[4] * h1 + f[5] * h2;
+                atomicAdd(&sy[l[b][0]], -(t1 + t2 + t3));
+                atomicAdd(&sy[l[b][1]], t1);
+                atomicAdd(&sy[l[b][2]], t2);
+                atomicAdd(&sy[l[b][3]], t3);
             }
         }
     }
+    __syncthreads();
+    patch_scatter_y<double, 1>(nloc, pv.nodes + off, pv.bslot + off, sy, y, part);
 }
 
-// out[k][s] = in[k][perm[s]] (0 where perm[s] < 0): per-element rows in patch-slot order
+// out[k][s] = in[k][perm[s]]: per-element rows in patch-slot order
 template <typename G>
-__global__ void patch_gather_rows_kernel(const int rows, const ptrdiff_t E, const ptrdiff_t Epad,
-                                         const int32_t *__restrict__ perm, const G *__restrict__ in,
-                                         G *__restrict__ out) {
-    for (ptrdiff_t i = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows * Epad;
+__global__ void patch_gather_rows_kernel(const int rows, const ptrdiff_t E, const int32_t *__restrict__ perm,
+                                         const G *__restrict__ in, G *__restrict__ out) {
+    for (ptrdiff_t i = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows * E;
          i += (ptrdiff_t)gridDim.x * blockDim.x) {
-        const ptrdiff_t k = i / Epad, s = i - k * Epad;
-        const int32_t e = perm[s];
-        out[i] = e >= 0 ? in[k * E + e] : G(0);
+        const ptrdiff_t k = i / E, s = i - k * E;
+        out[i] = in[k * E + perm[s]];
     }
 }
 
@@ -548,22 +660,35 @@ template <typename T, typename G>
 int hex8_elasticity_apply_patches(const PatchView &pv, const G *adjp, const G *detp, const float *coeffp, double mu,
                                   double lambda, const T *x, T *y, T *part, hipStream_t s) {
     if (pv.npatch == 0) return SFEM_SUCCESS;
-    const size_t lds = hex8_patch_lds_bytes(pv.maxloc, sizeof(T));
+    const size_t lds = patch_lds_bytes(pv.maxloc, 3, sizeof(T));
     if (lds > kPatchLdsLimit) {
         set_last_error("hex8 elasticity patches: patch node count exceeds the LDS budget");
         return SFEM_FAILURE;
     }
-    hex8_elasticity_patch_kernel<T, G, kPatchElements><<<(unsigned)pv.npatch, 256, lds, s>>>(
-        pv.count, pv.lconn, pv.node_off, pv.nodes, pv.bslot, pv.npatch * kPatchElements, adjp, detp, coeffp, mu,
-        lambda, x, y, part);
+    hex8_elasticity_patch_kernel<T, G><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, adjp, detp, coeffp, mu, lambda, x, y,
+                                                                             part);
+    SFEM_AMD_HIP_CHECK(hipGetLastError());
+    return SFEM_SUCCESS;
+}
+int laplacian_apply_patches(int nv, const PatchView &pv, const float *fffp, const float *coeffp, const double *x,
+                            double *y, double *part, hipStream_t s) {
+    if (pv.npatch == 0) return SFEM_SUCCESS;
+    const size_t lds = patch_lds_bytes(pv.maxloc, 1, sizeof(double));
+    if (lds > kPatchLdsLimit || (nv != 4 && nv != 8)) {
+        set_last_error("Laplacian patches: tet4 or hex8, patch nodes within the LDS budget");
+        return SFEM_FAILURE;
+    }
+    if (nv == 8)
+        laplacian_patch_kernel<8><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, fffp, coeffp, x, y, part);
+    else
+        laplacian_patch_kernel<4><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, fffp, coeffp, x, y, part);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }
 template <typename G>
-int patch_gather_rows(int rows, ptrdiff_t E, ptrdiff_t Epad, const int32_t *perm, const G *in, G *out,
-                      hipStream_t s) {
-    if (rows * Epad == 0) return SFEM_SUCCESS;
-    patch_gather_rows_kernel<G><<<grid_for(rows * Epad), kBlock, 0, s>>>(rows, E, Epad, perm, in, out);
+int patch_gather_rows(int rows, ptrdiff_t E, const int32_t *perm, const G *in, G *out, hipStream_t s) {
+    if (rows * E == 0) return SFEM_SUCCESS;
+    patch_gather_rows_kernel<G><<<grid_for(rows * E), kBlock, 0, s>>>(rows, E, perm, in, out);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }
@@ -573,10 +698,8 @@ template int hex8_elasticity_apply_patches<double, float>(const PatchView &, con
 template int hex8_elasticity_apply_patches<float, uint16_t>(const PatchView &, const uint16_t *, const uint16_t *,
                                                             const float *, double, double, const float *, float *,
                                                             float *, hipStream_t);
-template int patch_gather_rows<float>(int, ptrdiff_t, ptrdiff_t, const int32_t *, const float *, float *,
-                                      hipStream_t);
-template int patch_gather_rows<uint16_t>(int, ptrdiff_t, ptrdiff_t, const int32_t *, const uint16_t *, uint16_t *,
-                                         hipStream_t);
+template int patch_gather_rows<float>(int, ptrdiff_t, const int32_t *, const float *, float *, hipStream_t);
+template int patch_gather_rows<uint16_t>(int, ptrdiff_t, const int32_t *, const uint16_t *, uint16_t *, hipStream_t);
 // FP64 operator on float32 geometry words; FP32 operator on bf16 words
 template int hex8_elasticity_apply<double, float>(ptrdiff_t, const int32_t *, const float *, const float *, double,
                                                   double, const float *, const double *, double *, hipStream_t);

@@ -89,6 +89,49 @@ def test_hex8_laplacian_parity_with_coefficient():
     assert relerr(host(d), do) < RTOL
 
 
+def _isolated(nv, E):
+    """E elements that share no node, in shuffled node order."""
+    return np.random.default_rng(5).permutation(nv * E).reshape(nv, E).astype(np.int32)
+
+
+# element patches from 2^15 elements on: just below and above, ragged last patches, shuffled elements and
+# nodes, the large tet4 patches (2^20), elements without neighbours (a patch each)
+@pytest.mark.parametrize("kind,n,mesh", [("tet4", 17, "box"), ("tet4", 18, "box"), ("tet4", 23, "shuffled"),
+                                         ("tet4", 56, "box"), ("tet4", 0, "isolated"), ("hex8", 31, "box"),
+                                         ("hex8", 32, "box"), ("hex8", 37, "shuffled"), ("hex8", 0, "isolated")])
+@pytest.mark.parametrize("patches", [1, 0])
+def test_laplacian_on_patches(kind, n, mesh, patches):
+    nv = 4 if kind == "tet4" else 8
+    rng = np.random.default_rng(11)
+    if mesh == "isolated":
+        el = _isolated(nv, 1 << 15)
+        N, E = el.size, el.shape[1]
+        fff = rng.uniform(0.1, 1, (E, 6)).astype(np.float32)
+    else:
+        el, pts = skewed_box(n, tet4=kind == "tet4", perturb=0.02 * 6 / n)
+        N, E = pts.shape[1], el.shape[1]
+        fff = O.tet4_fff(el, pts) if kind == "tet4" else O.hex8_fff(el, pts)
+        if mesh == "shuffled":
+            el, q = rng.permutation(N).astype(np.int32)[el], rng.permutation(E)
+            el, fff = np.ascontiguousarray(el[:, q]), np.ascontiguousarray(fff[q])
+    coeff = rng.uniform(0.1, 10, E).astype(np.float32) if kind == "hex8" else None
+    x = rng.uniform(-1, 1, N)
+    yo = rng.uniform(-1, 1, N)
+    y = dev(yo)  # accumulate semantics: y += A x
+    S.set_option("hex8_patches", patches)
+    try:
+        op = S.laplacian(S.Mesh(S.TET4 if kind == "tet4" else S.HEX8, 1, el, N), fff, coeff)
+        op.apply(dev(x), y)
+        S.synchronize()
+    finally:
+        S.set_option("hex8_patches", 1)
+    if kind == "tet4":
+        O.lib.oracle_tet4_laplacian_apply(E, el, fff, x, yo)
+    else:
+        O.lib.oracle_hex8_laplacian_apply(E, el, fff, coeff, x, yo)
+    assert relerr(host(y), yo) < RTOL
+
+
 @pytest.mark.parametrize("L,n", [(1, 3), (2, 3), (3, 2), (4, 3), (5, 2), (6, 2), (8, 3), (10, 1), (12, 1), (16, 2)])
 def test_sshex8_laplacian_parity(L, n):
     mel, mpts = skewed_box(n, perturb=0.02)
