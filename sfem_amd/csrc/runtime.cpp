@@ -39,6 +39,13 @@ hipStream_t library_stream() {
     }
     return streams[dev];
 }
+hipStream_t default_stream() {
+    // an error here says that a blocking stream is being captured
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(nullptr, &st) == hipSuccess) return nullptr;
+    (void)hipGetLastError();
+    return library_stream();
+}
 
 }  // namespace sfem_amd
 
@@ -919,7 +926,8 @@ struct GraphOp final : OpBase {
     int apply_overwrite(const void *x, void *y, hipStream_t s) override { return run(x, y, s, true); }
     // the inner operator's apply (accumulating) or apply_overwrite, replayed from its own capture
     int run(const void *x, void *y, hipStream_t s, bool overwrite) {
-        auto eager = [&] { return overwrite ? inner->apply_overwrite(x, y, s) : inner->apply(x, y, s); };
+        auto on = [&](hipStream_t q) { return overwrite ? inner->apply_overwrite(x, y, q) : inner->apply(x, y, q); };
+        auto eager = [&] { return on(s); };
         Capture &c = cap[(overwrite ? 2 : 0) + (zero_guess ? 1 : 0)];
         const uint64_t now = state_epoch();
         if (c.exec && c.epoch != now) {
@@ -931,14 +939,16 @@ struct GraphOp final : OpBase {
         }
         if (c.calls++ == 0 || failed) return eager();
         if (!c.exec) {
-            if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
+            // the default stream cannot be captured: record on the library's, replay on the default one
+            hipStream_t rec = s ? s : library_stream();
+            if (hipStreamBeginCapture(rec, hipStreamCaptureModeThreadLocal) != hipSuccess) {
                 failed = true;
                 (void)hipGetLastError();
                 return eager();
             }
-            const int err = eager();
+            const int err = on(rec);
             hipGraph_t graph = nullptr;
-            const hipError_t e_end = hipStreamEndCapture(s, &graph);
+            const hipError_t e_end = hipStreamEndCapture(rec, &graph);
             if (err || e_end != hipSuccess || !graph ||
                 hipGraphInstantiate(&c.exec, graph, nullptr, nullptr, 0) != hipSuccess) {
                 if (graph) (void)hipGraphDestroy(graph);
@@ -1920,7 +1930,7 @@ static int block_jacobi_create_t(sfem_amd_op *A, const void *sym, const uint8_t 
     auto P = std::make_shared<BlockInverseOp<T>>();
     P->nb = A->impl->rows() / 3;
     if (P->inv.alloc((size_t)P->nb * 9) ||
-        block_sym_inverse<T>(P->nb, (const T *)sym, mask, omega, P->inv.p, library_stream()))
+        block_sym_inverse<T>(P->nb, (const T *)sym, mask, omega, P->inv.p, as_stream(nullptr)))
         return SFEM_FAILURE;
     auto st = std::make_shared<sfem::StationaryIteration<T>>();
     st->default_init();

@@ -623,6 +623,34 @@ def test_blas_reductions_deterministic_and_accurate():
             assert abs(S.norm2(da) - np.linalg.norm(a)) < 1e-12 * np.linalg.norm(a)
 
 
+def test_calls_without_a_stream_while_a_blocking_stream_is_captured():
+    """No stream means the default stream, which may not be used while a blocking stream is being
+    captured: such calls run on the library's own stream then, at once and outside the capture, which
+    stays valid and replays only what was recorded on its stream."""
+    import ctypes as C
+    hip = C.CDLL(None)  # the HIP runtime that the library has loaded
+    n = 1000
+    a, b = S.DeviceArray(n), S.DeviceArray(n)
+    stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+    S.synchronize()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread-local mode
+    assert S.lib.sfem_amd_blas_values(S.FLOAT64, n, 3.0, C.c_void_p(a.ptr), stream) == 0
+    assert S.lib.sfem_amd_blas_values(S.FLOAT64, n, 5.0, C.c_void_p(b.ptr), None) == 0
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and graph.value
+    S.synchronize()
+    assert np.all(a.numpy() == 0) and np.all(b.numpy() == 5)
+    assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+    b.fill(1.0)
+    for value in (0.0, 2.0, 7.0):
+        a.fill(value)  # the program's own eager work between replays
+        assert hip.hipGraphLaunch(exe, stream) == 0
+        assert hip.hipStreamSynchronize(stream) == 0
+        assert np.all(a.numpy() == 3) and np.all(b.numpy() == 1)
+    assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(stream) == 0
+
+
 @pytest.mark.parametrize("offset", [0, 1, 4])
 def test_fp32_streaming_kernels_aligned_and_not(offset):
     """FP32 axpby, fill, copy and the Chebyshev3 steps take 16 bytes per thread and array when every
