@@ -802,261 +802,243 @@ template int scatter_elements<float>(ptrdiff_t, int, const int32_t *, int, int, 
                                      float *, hipStream_t, bool);
 
 // ------------------------------------------------------------------ fused BF16 MFMA inference
-// One macro element per block (512 threads = 8 waves); the element's
-// activations stay in LDS for all four layers and both signs of f(z) = g(z) - g(-z).  Nodes are
-// processed in tiles of 16 (the MFMA N dimension); per tile and layer:
-//   layer 1 (1 -> 16):  D[co][n]  = sum_{k<32} W1[co][k] z[n + off_k]         one 16x16x32 MFMA
-//   layer 2,3 (16->16): D[co][n] += sum_{pairs p} W[co][ci,off] act[n + off]  14 16x16x32 MFMAs,
-//                       K = 32 = two offsets x 16 input channels; each wave runs three tiles at
-//                       once (three independent accumulation chains)
-//   layer 4 (16 -> 1):  P[k][n]   = sum_ci W4[ci][k] act[ci][n] (16x16x16 MFMAs, 16 offsets k per
-//                       pass, two passes), then out[n] = sum_k P[k][n + off_k] from LDS.
-// Lane layouts (64 lanes, g = lane / 16, c = lane % 16):
-//   16x16x32 A: row c, k = 8g + j (j < 8);  B: column c, k = 8g + j;  D: column c, rows 4g + r
-//   16x16x16 A: row c, k = 4g + j (j < 4);  B: column c, k = 4g + j;  D: as above
-// The input and the activations of layers 1-3 live on the element's grid with a one-point zero
-// halo ((L+3)^3 points), so neighbour reads need no validity tests: one address per tile and a
-// per-pair offset.  Activations are stored post-ReLU in BF16 as two channel planes
-// [half][point][8 channels] (16-byte B reads).  Layer 4's stencil sum reads the unpadded P, with
-// the padding node NXE (P == 0) standing in for missing neighbours.
-typedef short mf_s4 __attribute__((ext_vector_type(4)));
+// One macro element per block of eight waves (two elements for L <= 2), both signs of
+// f(z) = g(z) - g(-z) side by side, the element swept plane by plane in z through all four layers: only
+// a few planes of each layer live in LDS (65 KB at L = 8, two blocks per CU), and a hidden layer's
+// products keep the three output planes that an input plane feeds in registers, so that one read of an
+// operand serves three products.
+//
+// What bounds it: the hidden layers' products (15 per 16 cells, plane and sign at 16 cycles) and their operand
+// reads (5 of 1 KB) take about the same time, 13,000 cycles per element at L = 8.  Whole-element layers (14
+// products for 14 reads, 141 KB of LDS, one block per CU and nothing to overlap a layer's barriers) took
+// 3.14 ms for 32,768 elements of L = 8; this form 1.53 ms (890 TFLOP/s; a large bf16 matrix product
+// reaches 1,190 on the same card), of which layers 1 and 4 take 0.2.
+//
+// A plane is its lines with one halo cell each, LS = L + 2 cells apart, so that the cell after a line's last
+// node is a zero for both neighbours; columns of the matrix tiles are consecutive cells (the halo ones
+// computed and not stored), so every address is a lane's base plus a constant.  Activations are
+// BF16 after the relu, [sign][half of the channels][cell][8]: 16-byte operand reads.
+//   layer 1 (1 -> 16):   D[co][n] = sum_{k < 32} W1[co][k] z[n + off_k]: one 16x16x32 product for both signs
+//   layers 2, 3:         for each dz: D_dz[co][n] += sum W[co][ci, dz dy dx] act[n + dy dx], K = 32 = two of the
+//                        nine (dy, dx) times 16 channels (the tenth is zero)
+//   layer 4 (16 -> 1):   D[(dz, dy)][n] = sum W4[ci, dz dy dx] act[n + dx] for each sign, K = 32 = two dx times
+//                        16 channels (the fourth dx is zero), rows the nine (dz, dy); the difference of the
+//                        signs (formed alike, so f stays exactly odd) goes to a ring in LDS, and
+//                        out = the sum of nine rows of three planes.
+// Waves 0-3 run layers 1 and 2 and the output, waves 4-7 layers 3 and 4 (a hidden layer's weights stay in
+// registers: 15 operands).  In step s: layer 1 plane s, layer 2 takes plane s - 1 and finishes s - 2, layer 3 takes s - 3 and
+// finishes s - 4, layer 4 takes s - 5, and plane s - 7 goes out; every stage reads what the step before wrote:
+// one barrier per step.
+// Lane layouts (64 lanes, g = lane / 16, c = lane % 16), 16x16x32:
+//   A: row c, k = 8g + j (j < 8);  B: column c, k = 8g + j;  D: column c, rows 4g + r
 typedef __bf16 mf_b8 __attribute__((ext_vector_type(8)));
 typedef float mf_f4 __attribute__((ext_vector_type(4)));
 typedef unsigned int mf_u4 __attribute__((ext_vector_type(4)));
 typedef unsigned int mf_u2 __attribute__((ext_vector_type(2)));
-
 typedef __bf16 mf_b2 __attribute__((ext_vector_type(2)));
 typedef float mf_f2 __attribute__((ext_vector_type(2)));
 
-// float -> bf16, round to nearest even: the conversions lower to gfx950's v_cvt_pk_bf16_f32
-// (bf_pack converts two values with one instruction)
-__device__ __forceinline__ __bf16 f2bf(float f) { return (__bf16)f; }
+// two floats -> bf16, round to nearest even (gfx950's v_cvt_pk_bf16_f32)
 __device__ __forceinline__ unsigned bf_pack(float lo, float hi) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector(mf_f2{lo, hi}, mf_b2));
 }
-
-template <int L>
-struct CnnShape {
-    static constexpr int N1 = L + 1;
-    static constexpr int NXE = N1 * N1 * N1;
-    // node tiles of 16 with at least one padding node (node NXE: P[k][NXE] == 0 stands in for the
-    // missing neighbours of the layer-4 stencil sum)
-    static constexpr int T = NXE / 16 + 1;
-    static constexpr int NP = T * 16;
-    // layers 1-3 hold the element on grids with a zero halo, so every node's 27 neighbours are in
-    // range and read without tests: the input on the (L+3)^3 grid, the activations on a grid with
-    // line stride SY and plane stride SZ chosen so that consecutive nodes, also across line and
-    // plane ends, sit one 16-byte row apart mod 8 (eight lanes read all 32 LDS banks)
-    static constexpr int P1 = L + 3;
-    static constexpr int NH = P1 * P1 * P1;
-    static constexpr int SY = L + 9;  // >= L + 3, = L + 1 (mod 8)
-    static constexpr int SZ = P1 * SY + ((((L * SY + L + 1) - P1 * SY) % 8) + 8) % 8;  // = L SY + L + 1 (mod 8)
-    static constexpr int NA = P1 * SZ;
-    static constexpr int THREADS = 512;
-    static constexpr int TPG = 3;  // tiles per wave iteration in the hidden layers
-    // zs [NH] float | actX [2][NA][8] bf16 | actY [2][NA][8] bf16, aliased by P [16][NP] float
-    // (actY is cleared again at the start of each sign)
-    static constexpr size_t ZS = (sizeof(float) * NH + 15) / 16 * 16;
-    static constexpr size_t ACT = 32 * (size_t)NA;
-    static constexpr size_t LDS = ZS + ACT + (ACT > 64 * (size_t)NP ? ACT : 64 * (size_t)NP);
-};
-
-// Neighbour validity as bit tests.  cnn_avail: the directions in which node (x, y, z) has a
-// neighbour (bits x-, x+, y-, y+, z-, z+) and bit 6 for a real node (in); cnn_need(o): the bits offset
-// o requires (bit 7, never available, for the padding offsets o >= 27).  Offset o of the node exists
-// iff (cnn_need(o) & ~cnn_avail) == 0.
-template <int L>
-__device__ __forceinline__ unsigned cnn_avail(int x, int y, int z, bool in) {
-    return (unsigned)(x > 0) | (unsigned)(x < L) << 1 | (unsigned)(y > 0) << 2 | (unsigned)(y < L) << 3 |
-           (unsigned)(z > 0) << 4 | (unsigned)(z < L) << 5 | (unsigned)in << 6;
-}
-__host__ __device__ constexpr unsigned cnn_need(int o) {
-    return o >= 27 ? 128u
-                   : 64u | (o % 3 == 0 ? 1u : 0u) | (o % 3 == 2 ? 2u : 0u) | ((o / 3) % 3 == 0 ? 4u : 0u) |
-                         ((o / 3) % 3 == 2 ? 8u : 0u) | (o / 9 == 0 ? 16u : 0u) | (o / 9 == 2 ? 32u : 0u);
-}
-
-template <int L>
-__device__ __forceinline__ int cnn_shift(int o) {
-    constexpr int N1 = L + 1;
-    return (o / 9 - 1) * N1 * N1 + ((o / 3) % 3 - 1) * N1 + (o % 3 - 1);
-}
-
-// node n = lidx(x, y, z) on a haloed grid with line stride SY and plane stride SZ;
-// cnn_pshift(o): offset o there (0 for the zero-weight padding offsets o >= 27, which then read
-// the node itself)
-template <int L, int SY, int SZ>
-__device__ __forceinline__ int cnn_pad(int n) {
-    constexpr int N1 = L + 1;
-    const int x = n % N1, y = (n / N1) % N1, z = n / (N1 * N1);
-    return (x + 1) + (y + 1) * SY + (z + 1) * SZ;
-}
-template <int SY, int SZ>
-__device__ __forceinline__ int cnn_pshift(int o) {
-    return o >= 27 ? 0 : (o / 9 - 1) * SZ + ((o / 3) % 3 - 1) * SY + (o % 3 - 1);
-}
-
-// 4 channels (4g .. 4g+3) of grid point q, as stored from an MFMA D fragment
-__device__ __forceinline__ unsigned short *act_quad(unsigned short *a, int NA, int q, int g) {
-    return a + (g >> 1) * NA * 8 + q * 8 + 4 * (g & 1);
-}
-
 __device__ __forceinline__ mf_u2 relu_pack(const mf_f4 &acc, float sg) {
     mf_u2 o2;
     o2[0] = bf_pack(fmaxf(sg * acc[0], 0.f), fmaxf(sg * acc[1], 0.f));
     o2[1] = bf_pack(fmaxf(sg * acc[2], 0.f), fmaxf(sg * acc[3], 0.f));
     return o2;
 }
+__device__ __forceinline__ mf_f4 mf_mma(const mf_u4 &a, const mf_u4 &b, const mf_f4 &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_b8, a), __builtin_bit_cast(mf_b8, b), c, 0, 0,
+                                                   0);
+}
 
 template <int L>
-__global__ void __launch_bounds__(512, 2) cnn_infer_kernel(const ptrdiff_t E, const unsigned short *__restrict__ W16,
-                                                           const float *__restrict__ zin, float *__restrict__ out) {
-    using S = CnnShape<L>;
-    constexpr int NP = S::NP, NH = S::NH, NA = S::NA, P1 = S::P1, SY = S::SY, SZ = S::SZ, TPG = S::TPG,
-                  NB = (S::NXE + S::THREADS - 1) / S::THREADS;
-    extern __shared__ __align__(16) unsigned char cnn_smem[];
-    float *zs = (float *)cnn_smem;
-    unsigned short *actX = (unsigned short *)(cnn_smem + S::ZS);
-    unsigned short *actY = actX + 16 * NA;
-    float *P = (float *)actY;
-    const ptrdiff_t e = blockIdx.x;
-    if (e >= E) return;  // uniform per block
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = S::THREADS / 64;
-    const int g = lane >> 4, c = lane & 15;
+struct CnnShape {
+    static constexpr int N1 = L + 1, NXE = N1 * N1 * N1, LS = L + 2, REAL = N1 * LS;
+    static constexpr int TS = (REAL + 15) / 16;                  // tiles of a plane and sign
+    static constexpr int WS = TS >= 2 ? 2 : 1, EPB = 2 / WS;     // waves per sign; elements per block
+    static constexpr int TW = (TS + WS - 1) / WS;                // tiles per wave
+    static constexpr int COLS = 16 * WS * TW;
+    // cells of a plane with the halo around the columns' neighbourhoods; cell p is stored at p + LS + 1
+    static constexpr int CELLS = (COLS + 2 * (LS + 1) + 7) / 8 * 8;
+    static constexpr int HALF = CELLS * 16, SIGN = 2 * HALF, PLANE = 2 * SIGN, BUF = EPB * PLANE;  // bytes
+    // the input: planes PS cells apart, sharing their halo lines
+    static constexpr int PS = (L + 2) * LS, OFFZ = PS + LS + 1;
+    static constexpr int ZN = (L * PS + COLS - 1 + 2 * OFFZ + 1 + 7) / 8 * 8;
+    // layer 4's rows of a plane: a zero line on both sides; rows 4 (mod 8) words apart (bank spread of the
+    // stores' row groups); a ring of four planes
+    static constexpr int DROW = (REAL + 2 * LS + 7) / 8 * 8 + 4, DPLANE = 9 * DROW;
+    static constexpr int STEPS = L + 8, THREADS = 512;
+    static constexpr size_t LDS = (size_t)6 * BUF + sizeof(float) * 4 * EPB * DPLANE + 3 * 64 * 16 + 2 * (size_t)EPB * ZN;
+};
 
-    // the input on its haloed grid; actX zeroed (the layers write only the interior points, so its
-    // halo stays zero for both signs)
-    {
-        // all of this thread's input loads at once (halo and tail points read the element's first
-        // value, a valid address, and store zero)
-        constexpr int NBI = (NH + S::THREADS - 1) / S::THREADS;
-        float zv[NBI];
+// The nine (dy, dx) of a hidden layer as five pairs, (dy, -1) with (dy, 0), then (-1, 1) with (0, 1) and
+// nothing with (1, 1): the second of a pair lies one cell, or one line, after the first, so a lane needs two
+// addresses and constant offsets.
+//
+// One input plane through a hidden layer.  a, b: the lane's addresses for the first three and the last two
+// pairs; o: its store address.  acc[d][h]: output plane zi - 1 + d of tile h.
+template <int L>
+__device__ __forceinline__ void cnn_hidden(const unsigned char *__restrict__ a, const unsigned char *__restrict__ b,
+                                           unsigned char *__restrict__ o, const int zi, const mf_u4 (&w)[15],
+                                           const bool (&real)[CnnShape<L>::TW], mf_f4 (&acc)[3][CnnShape<L>::TW]) {
+    constexpr int TW = CnnShape<L>::TW, LS = CnnShape<L>::LS;
+    if (zi <= L) {
 #pragma unroll
-        for (int b = 0; b < NBI; b++) {
-            const int q = tid + b * S::THREADS;
-            const int px = q % P1 - 1, py = (q / P1) % P1 - 1, pz = q / (P1 * P1) - 1;
-            const bool in = q < NH && (unsigned)px <= (unsigned)L && (unsigned)py <= (unsigned)L &&
-                            (unsigned)pz <= (unsigned)L;
-            const float v = zin[(size_t)e * S::NXE + (in ? (pz * S::N1 + py) * S::N1 + px : 0)];
-            zv[b] = in ? v : 0.f;
-        }
+        for (int p = 0; p < 5; p++) {
+            const unsigned char *q = p < 3 ? a + 16 * ((p - 1) * LS - 1) : b + 16 * (p == 3 ? 1 - LS : 1);
+            mf_u4 x[TW];
 #pragma unroll
-        for (int b = 0; b < NBI; b++) {
-            const int q = tid + b * S::THREADS;
-            if (q < NH) zs[q] = zv[b];
+            for (int h = 0; h < TW; h++) x[h] = *(const mf_u4 *)(q + 256 * h);
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int h = 0; h < TW; h++) acc[d][h] = mf_mma(w[(2 - d) * 5 + p], x[h], acc[d][h]);
         }
     }
-    for (int i = tid; i < 2 * NA; i += S::THREADS) ((mf_u4 *)actX)[i] = mf_u4{0u, 0u, 0u, 0u};
-    // weights in lane order: layer 1 [64][8], layers 2-3 [14][64][8], layer 4 [2][64][4]
-    const mf_u4 w1 = *(const mf_u4 *)(W16 + lane * 8);
-    int sh1[8];  // layer 1: lane group g gathers offsets 8g .. 8g+7
+    if (zi >= 1)
 #pragma unroll
-    for (int j = 0; j < 8; j++) sh1[j] = cnn_pshift<P1, P1 * P1>(8 * g + j);
-    const bool hi = (g >> 1) != 0;  // hidden layers: lane groups 2, 3 take the pair's second offset
-    float gplus[NB];
+        for (int h = 0; h < TW; h++)
+            if (real[h]) *(mf_u2 *)(o + 256 * h) = relu_pack(acc[0][h], 1.f);
+#pragma unroll
+    for (int h = 0; h < TW; h++) {
+        acc[0][h] = acc[1][h];
+        acc[1][h] = acc[2][h];
+        acc[2][h] = mf_f4{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+template <int L>
+__global__ void __launch_bounds__(512, 4) cnn_infer_kernel(const ptrdiff_t E, const unsigned short *__restrict__ W16,
+                                                           const float *__restrict__ zin, float *__restrict__ out) {
+    using S = CnnShape<L>;
+    constexpr int N1 = S::N1, LS = S::LS, TW = S::TW, EPB = S::EPB;
+    extern __shared__ __align__(16) unsigned char cnn_smem[];
+    unsigned char *A1 = cnn_smem, *A2 = A1 + 2 * S::BUF, *A3 = A2 + 2 * S::BUF;
+    float *D = (float *)(A3 + 2 * S::BUF);
+    mf_u4 *WS14 = (mf_u4 *)(D + 4 * EPB * S::DPLANE);
+    unsigned short *zs = (unsigned short *)(WS14 + 3 * 64);
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = wave & 3;
+    const ptrdiff_t e0 = (ptrdiff_t)blockIdx.x * EPB;
+
+    // zero planes and rows (the stages write real nodes only), the input as bf16 in its halo layout
+    for (int i = tid; i < (int)((6 * S::BUF + 16 * EPB * S::DPLANE) / 16); i += S::THREADS)
+        ((mf_u4 *)cnn_smem)[i] = mf_u4{0u, 0u, 0u, 0u};
+    for (int i = tid; i < EPB * S::ZN; i += S::THREADS) {
+        const int el = i / S::ZN, q = i - el * S::ZN - (LS + 1);  // q = (z + 1) PS + y LS + x
+        const int z = (q + S::PS) / S::PS - 2, r = (q + S::PS) % S::PS, y = r / LS, x = r % LS;
+        const bool in = z >= 0 && z <= L && y <= L && x <= L && e0 + el < E;
+        const float v = zin[(size_t)(in ? e0 + el : e0) * S::NXE + (in ? (z * N1 + y) * N1 + x : 0)];
+        zs[i] = in ? (unsigned short)bf_pack(v, 0.f) : (unsigned short)0;
+    }
+
+    // the A operands of layers 1 and 4, read back where they are used
+    for (int i = tid; i < 64 * 3; i += S::THREADS)
+        WS14[i] = *(const mf_u4 *)(W16 + (i < 64 ? i * 8 : 512 + 2 * 7680 + (i - 64) * 8));
+
+    // this wave's tiles in the hidden layers
+    const int el = EPB == 1 ? 0 : w4 >> 1, sign = EPB == 1 ? w4 >> 1 : w4 & 1;
+    const int p0 = (EPB == 1 ? (w4 & 1) * TW * 16 : 0) + c;
+    const int base = el * S::PLANE + sign * S::SIGN + (p0 + LS + 1) * 16;
+    const int ha = base + (g & 1) * S::HALF + (g >> 1) * 16, hb = base + (g & 1) * S::HALF + (g >> 1) * 16 * LS;
+    const int store = base + (g >> 1) * S::HALF + 8 * (g & 1);
+    bool real[TW];
+#pragma unroll
+    for (int h = 0; h < TW; h++) real[h] = p0 + 16 * h < S::REAL && (p0 + 16 * h) % LS <= L;
+    mf_u4 w[15];
+    const unsigned short *wl = W16 + 512 + (wave >> 2) * 7680;
+#pragma unroll
+    for (int i = 0; i < 15; i++) w[i] = *(const mf_u4 *)(wl + (i * 64 + lane) * 8);
+    mf_f4 acc[3][TW];
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int h = 0; h < TW; h++) acc[d][h] = mf_f4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
 
-    for (int sign = 0; sign < 2; sign++) {
-        const float sg = sign ? -1.f : 1.f;
-        // ---- layer 1: zs -> actX; actY (P of the previous sign) cleared for layer 2
-        for (int i = tid; i < 2 * NA; i += S::THREADS) ((mf_u4 *)actY)[i] = mf_u4{0u, 0u, 0u, 0u};
-        for (int t = wave; t < S::T; t += nw) {
-            const int n = t * 16 + c;
-            const bool real = n < S::NXE;
-            const int qz = cnn_pad<L, P1, P1 * P1>(real ? n : 0);
-            mf_b8 b;
+    if (wave < 4) {
+        // layer 1's gathers: lane groups 0-2 take plane dz = g - 1 without its last offset (dy, dx) = (1, 1),
+        // group 3 the three last ones: one address and constant offsets, but for three slots
+        const int zc = S::OFFZ + c, za = zc + (g < 3 ? g - 1 : 0) * S::PS;
+        int zb[3];
 #pragma unroll
-            for (int j = 0; j < 8; j++) b[j] = f2bf(zs[qz + sh1[j]]);
-            mf_f4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_b8, w1), b, acc, 0, 0, 0);
-            if (real) *(mf_u2 *)act_quad(actX, NA, cnn_pad<L, SY, SZ>(n), g) = relu_pack(acc, sg);
-        }
-        __syncthreads();
-        // ---- layers 2 and 3: actX -> actY -> actX
-#pragma unroll 1
-        for (int layer = 0; layer < 2; layer++) {
-            const unsigned short *ain = layer ? actY : actX;
-            unsigned short *aout = layer ? actX : actY;
-            const unsigned short *wl = W16 + 512 + layer * 7168;
-            mf_u4 w[14];
+        for (int j = 0; j < 3; j++) zb[j] = g < 3 ? za - LS + j - 1 : zc + (j - 1) * S::PS + LS + 1;
+        for (int s = 0; s < S::STEPS; s++) {
+            if (s <= L)
+                for (int t = w4; t < EPB * S::TS; t += 4) {
+                    const int le = EPB == 1 ? 0 : t / S::TS, p = (t - le * S::TS) * 16;
+                    const unsigned short *q = zs + le * S::ZN + s * S::PS + p;
+                    mf_u4 b;
 #pragma unroll
-            for (int p = 0; p < 14; p++) w[p] = *(const mf_u4 *)(wl + (p * 64 + lane) * 8);
-            // byte addresses: the lane's channel plane plus 16 bytes per grid point
-            const unsigned char *plane = (const unsigned char *)(ain + (g & 1) * NA * 8);
-            for (int t = TPG * wave; t < S::T; t += TPG * nw) {
-                int q[TPG], qb[TPG];
-                bool real[TPG];
-                mf_f4 acc[TPG];
-#pragma unroll
-                for (int h = 0; h < TPG; h++) {
-                    const int n = (t + h) * 16 + c;
-                    real[h] = n < S::NXE;
-                    q[h] = cnn_pad<L, SY, SZ>(real[h] ? n : 0);
-                    qb[h] = q[h] * 16;
-                    acc[h] = mf_f4{0.f, 0.f, 0.f, 0.f};
+                    for (int j = 0; j < 4; j++) {
+                        const int k0 = 2 * j, k1 = 2 * j + 1;
+                        const unsigned lo = k0 < 3 ? q[zb[k0 < 3 ? k0 : 0]] : q[za + (k0 / 3 - 1) * LS + k0 % 3 - 1];
+                        const unsigned hi = k1 < 3 ? q[zb[k1 < 3 ? k1 : 0]] : q[za + (k1 / 3 - 1) * LS + k1 % 3 - 1];
+                        b[j] = lo | hi << 16;
+                    }
+                    const mf_f4 a = mf_mma(WS14[lane], b, mf_f4{0.f, 0.f, 0.f, 0.f});
+                    unsigned char *o = A1 + (s & 1) * S::BUF + le * S::PLANE + (g >> 1) * S::HALF +
+                                       (p + c + LS + 1) * 16 + 8 * (g & 1);
+                    if (p + c < S::REAL && (p + c) % LS <= L) {
+                        *(mf_u2 *)o = relu_pack(a, 1.f);
+                        *(mf_u2 *)(o + S::SIGN) = relu_pack(a, -1.f);
+                    }
                 }
+            if (s >= 1 && s <= L + 2) {
+                const unsigned char *in = A1 + ((s - 1) & 1) * S::BUF;
+                cnn_hidden<L>(in + ha, in + hb, A2 + (s & 1) * S::BUF + store, s - 1, w, real, acc);
+            }
+            if (s >= 7) {
+                // plane s - 7 from the rows of planes s - 8, s - 7, s - 6
+                const int z = s - 7;
+                for (int i = tid; i < EPB * S::REAL; i += 256) {
+                    const int le = EPB == 1 ? 0 : i / S::REAL, p = i - le * S::REAL, y = p / LS, x = p - y * LS;
+                    if (x > L || e0 + le >= E) continue;
+                    float v = 0.f;
 #pragma unroll
-                for (int p = 0; p < 14; p++) {
-                    const int shb = 16 * (hi ? cnn_pshift<SY, SZ>(2 * p + 1) : cnn_pshift<SY, SZ>(2 * p));
-                    mf_u4 bv[TPG];
+                    for (int dz = -1; dz <= 1; dz++) {
+                        if (z + dz < 0 || z + dz > L) continue;
+                        const float *r = D + (((z + dz) & 3) * EPB + le) * S::DPLANE + LS + p + (dz + 1) * 3 * S::DROW;
 #pragma unroll
-                    for (int h = 0; h < TPG; h++) bv[h] = *(const mf_u4 *)(plane + qb[h] + shb);
-#pragma unroll
-                    for (int h = 0; h < TPG; h++)
-                        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_b8, w[p]),
-                                                                          __builtin_bit_cast(mf_b8, bv[h]), acc[h], 0,
-                                                                          0, 0);
+                        for (int dy = -1; dy <= 1; dy++) v += r[(dy + 1) * S::DROW + dy * LS];
+                    }
+                    out[(size_t)(e0 + le) * S::NXE + (z * N1 + y) * N1 + x] = v;
                 }
-#pragma unroll
-                for (int h = 0; h < TPG; h++)
-                    if (real[h]) *(mf_u2 *)act_quad(aout, NA, q[h], g) = relu_pack(acc[h], 1.f);
             }
-            __syncthreads();
+            lds_barrier();
         }
-        // ---- layer 4 in two passes of 16 offsets: P[r][n] = sum_ci W4[ci][16 pass + r] act[ci][n],
-        // then v[n] += sum_r P[r][n + off_{16 pass + r}]
-        float v[NB];
+    } else {
+        for (int s = 0; s < S::STEPS; s++) {
+            if (s >= 5 && s <= L + 5) {
+                // plane s - 5 of layer 4's rows
+                const mf_u4 wa = WS14[64 + lane], wb = WS14[128 + lane];
+                for (int t = w4; t < EPB * S::TS; t += 4) {
+                    const int le = EPB == 1 ? 0 : t / S::TS, p = (t - le * S::TS) * 16 + c;
+                    // dx = -1 and 0, then 1 and none (the lanes g >= 2 read dx = 1 there too)
+                    const unsigned char *q = A3 + ((s - 1) & 1) * S::BUF + le * S::PLANE + (g & 1) * S::HALF +
+                                             (p + LS + (g >> 1)) * 16;
+                    const unsigned char *q1 = q + (g < 2 ? 32 : 16);
+                    mf_f4 d[2];
 #pragma unroll
-        for (int i = 0; i < NB; i++) v[i] = 0.f;
-#pragma unroll
-        for (int pass = 0; pass < 2; pass++) {
-            const mf_u2 w4 = *(const mf_u2 *)(W16 + 512 + 2 * 7168 + pass * 256 + lane * 4);
-            for (int t = wave; t < S::T; t += nw) {
-                const int n = t * 16 + c;
-                const bool real = n < S::NXE;
-                const mf_u2 ld = *(const mf_u2 *)act_quad(actX, NA, cnn_pad<L, SY, SZ>(real ? n : 0), g);
-                const mf_u2 bv = real ? ld : mf_u2{0u, 0u};  // padding nodes: P[r][n] = 0
-                mf_f4 a = {0.f, 0.f, 0.f, 0.f};
-                a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(mf_s4, w4), __builtin_bit_cast(mf_s4, bv),
-                                                               a, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; r++) P[(4 * g + r) * NP + n] = a[r];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < NB; i++) {
-                const int n = tid + i * S::THREADS;
-                if (n < S::NXE) {
-                    const unsigned na = ~cnn_avail<L>(n % S::N1, (n / S::N1) % S::N1, n / (S::N1 * S::N1), true);
-                    // missing neighbours add P[r][NXE] == 0 (the padding node's product)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int k = 16 * pass + r;
-                        if (k < 27) v[i] += P[r * NP + ((cnn_need(k) & na) == 0 ? n + cnn_shift<L>(k) : S::NXE)];
+                    for (int sn = 0; sn < 2; sn++) {
+                        d[sn] = mf_mma(wa, *(const mf_u4 *)(q + sn * S::SIGN), mf_f4{0.f, 0.f, 0.f, 0.f});
+                        d[sn] = mf_mma(wb, *(const mf_u4 *)(q1 + sn * S::SIGN), d[sn]);
+                    }
+                    const mf_f4 a = d[0] - d[1];
+                    float *o = D + (((s - 5) & 3) * EPB + le) * S::DPLANE + LS + p + 4 * g * S::DROW;
+                    if (p < S::REAL) {
+                        if (g < 3) o[0] = a[0];
+                        if (g < 2) o[S::DROW] = a[1], o[2 * S::DROW] = a[2], o[3 * S::DROW] = a[3];
                     }
                 }
             }
-            __syncthreads();  // P is rewritten by the next pass / sign
-        }
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const int n = tid + i * S::THREADS;
-            if (n < S::NXE) {
-                if (sign == 0)
-                    gplus[i] = v[i];
-                else
-                    out[(size_t)e * S::NXE + n] = gplus[i] - v[i];
+            if (s >= 3 && s <= L + 4) {
+                const unsigned char *in = A2 + ((s - 1) & 1) * S::BUF;
+                cnn_hidden<L>(in + ha, in + hb, A3 + (s & 1) * S::BUF + store, s - 3, w, real, acc);
             }
+            lds_barrier();
         }
     }
 }
@@ -1064,13 +1046,9 @@ __global__ void __launch_bounds__(512, 2) cnn_infer_kernel(const ptrdiff_t E, co
 template <int L>
 static int launch_cnn_infer(ptrdiff_t E, const uint16_t *W16, const float *z, float *out, hipStream_t s) {
     using S = CnnShape<L>;
-    static bool attr = false;
-    if (!attr) {
-        SFEM_AMD_HIP_CHECK(
-            hipFuncSetAttribute((const void *)cnn_infer_kernel<L>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::LDS));
-        attr = true;
-    }
-    cnn_infer_kernel<L><<<(unsigned)E, S::THREADS, S::LDS, s>>>(E, (const unsigned short *)W16, z, out);
+    if (raise_lds_limit<cnn_infer_kernel<L>>(S::LDS)) return SFEM_FAILURE;
+    cnn_infer_kernel<L><<<(unsigned)((E + S::EPB - 1) / S::EPB), S::THREADS, S::LDS, s>>>(E, (const unsigned short *)W16, z,
+                                                                                         out);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }

@@ -38,7 +38,7 @@ int scatter_elements(ptrdiff_t E, int nxe, const int32_t *idx, int bs, int comp,
                      const float *val, T *vec, hipStream_t s, bool channels = false);
 // fused BF16 MFMA inference (hidden 16, 4 layers, L <= 8); W16: bf16 weights of the 4 layers in
 // MFMA lane order (kCnnPackedWeights entries, see cnn_pack_weights)
-constexpr int kCnnPackedWeights = 512 + 2 * 7168 + 512;
+constexpr int kCnnPackedWeights = 512 + 2 * 7680 + 1024;
 void cnn_pack_weights(const float *W, uint16_t *packed);
 int cnn_infer_mfma(int L, ptrdiff_t E, const uint16_t *W16, const float *z, float *out, hipStream_t s);
 }  // namespace sfem_amd

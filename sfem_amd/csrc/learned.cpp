@@ -71,27 +71,33 @@ int forward_f(sfem_amd_cnn *c, int L, ptrdiff_t E, const float *z, float *out, h
 
 namespace sfem_amd {
 // Weights [layer][Cout][Cin][27] (hidden 16, 4 layers) -> BF16 in the lane order of the fused
-// inference kernel: layer 1 [64 lanes][8], layers 2-3 [14 offset pairs][64][8], layer 4 [2][64][4].
+// inference kernel's A operands, [64 lanes][8] each (row lane % 16, group lane / 16): layer 1; layers
+// 2-3 [dz][five pairs of (dy, dx)] with k = (offset of the pair, channel); layer 4 [two
+// pairs of dx], rows (dz, dy), k = (dx of the pair, channel).
 void cnn_pack_weights(const float *W, uint16_t *packed) {
     const float *W1 = W, *W2 = W + 432, *W3 = W + 432 + 6912, *W4 = W + 432 + 2 * 6912;
     uint16_t *o = packed;
     for (int lane = 0; lane < 64; lane++)
         for (int j = 0; j < 8; j++) {
-            const int co = lane % 16, k = 8 * (lane / 16) + j;
+            // groups 0-2: the plane dz without its last offset; group 3: the three last ones
+            const int co = lane % 16, g = lane / 16, k = g < 3 ? 9 * g + j : (j < 3 ? 9 * j + 8 : 27);
             *o++ = to_bf16(k < 27 ? W1[co * 27 + k] : 0.f);
         }
     for (const float *Wl : {W2, W3})
-        for (int p = 0; p < 14; p++)
-            for (int lane = 0; lane < 64; lane++)
-                for (int j = 0; j < 8; j++) {
-                    const int co = lane % 16, g = lane / 16, off = 2 * p + g / 2, ci = 8 * (g % 2) + j;
-                    *o++ = to_bf16(off < 27 ? Wl[(co * 16 + ci) * 27 + off] : 0.f);
-                }
-    for (int h = 0; h < 2; h++)
+        for (int dz = 0; dz < 3; dz++)
+            for (int p = 0; p < 5; p++)
+                for (int lane = 0; lane < 64; lane++)
+                    for (int j = 0; j < 8; j++) {
+                        // (dy, dx) as dy * 3 + dx of each pair's members (9: none)
+                        constexpr int pair[5][2] = {{0, 1}, {3, 4}, {6, 7}, {2, 5}, {9, 8}};
+                        const int co = lane % 16, g = lane / 16, off = pair[p][g / 2], ci = 8 * (g % 2) + j;
+                        *o++ = to_bf16(off < 9 ? Wl[(co * 16 + ci) * 27 + dz * 9 + off] : 0.f);
+                    }
+    for (int i = 0; i < 2; i++)
         for (int lane = 0; lane < 64; lane++)
-            for (int j = 0; j < 4; j++) {
-                const int k = 16 * h + lane % 16, ci = 4 * (lane / 16) + j;
-                *o++ = to_bf16(k < 27 ? W4[ci * 27 + k] : 0.f);
+            for (int j = 0; j < 8; j++) {
+                const int row = lane % 16, g = lane / 16, ci = 8 * (g % 2) + j, dx = 2 * i + g / 2;
+                *o++ = to_bf16(row < 9 && dx < 3 ? W4[ci * 27 + row * 3 + dx] : 0.f);
             }
 }
 }  // namespace sfem_amd
@@ -134,7 +140,6 @@ int sfem_amd_cnn_create_channels(int channels, int hidden, int layers, const flo
     SFEM_AMD_HIP_CHECK(hipMemset(c->v.p, 0, sizeof(float) * off));
     for (int l = 0; l < layers; l++) c->acts.push_back(new DevArray<float>());
     if (c->ws.alloc(514)) return SFEM_FAILURE;
-    SFEM_AMD_HIP_CHECK(hipHostMalloc((void **)&c->host, 2 * sizeof(double) + sizeof(float) * off));
     *out = c.release();
     return SFEM_SUCCESS;
 }
@@ -188,6 +193,8 @@ int sfem_amd_cnn_loss_grad(sfem_amd_cnn *c, int L, ptrdiff_t E, const float *z, 
     hipStream_t s = as_stream(stream);
     const size_t nxe = nxe_of(L), n = (size_t)E * c->io * nxe;
     const int nblocks = cnn_weight_partials(2 * E);
+    if (!c->host)  // networks that only infer have no use for it
+        SFEM_AMD_HIP_CHECK(hipHostMalloc((void **)&c->host, 2 * sizeof(double) + sizeof(float) * c->nparams));
     if (ensure(c->diff, n) || ensure(c->dpm, 2 * n) || ensure(c->part, (size_t)nblocks * c->nparams))
         return SFEM_FAILURE;
     if (forward_g(c, L, E, z, s)) return SFEM_FAILURE;
