@@ -5,8 +5,6 @@
 //
 // Layouts: activations [E][C][nxe] float (node index = lidx), weights [Cout][Cin][27] with
 // offset k = (dz+1)*9 + (dy+1)*3 + (dx+1).
-#include <atomic>
-
 #include "cnn_kernels.hpp"
 #include "common.hpp"
 
@@ -570,21 +568,6 @@ __global__ void scatter_elements_kernel(const ptrdiff_t E, const int nxe, const 
 }
 
 // ------------------------------------------------------------------ launchers
-// Dynamic LDS above the default 64 KB needs the function attribute, once per function and device.
-template <auto Fn>
-static int raise_lds_limit(size_t bytes) {
-    static std::atomic<uint64_t> done{0};
-    if (bytes <= 64 * 1024) return SFEM_SUCCESS;
-    int dev = 0;
-    SFEM_AMD_HIP_CHECK(hipGetDevice(&dev));
-    const uint64_t bit = 1ull << (dev & 63);
-    if (done.load(std::memory_order_acquire) & bit) return SFEM_SUCCESS;
-    SFEM_AMD_HIP_CHECK(
-        hipFuncSetAttribute((const void *)Fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    done.fetch_or(bit, std::memory_order_acq_rel);
-    return SFEM_SUCCESS;
-}
-
 // Blocks on whole elements once the batch alone fills the GPU (two blocks on each of 256 CUs); below,
 // blocks on 64 nodes (convolutions) or a quarter of the nodes (weight gradients) of an element.
 constexpr ptrdiff_t kConvFull = 512;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <cstdio>
@@ -145,17 +146,17 @@ __host__ __device__ inline int hierarchical_level_index(int L, const int *levels
 }
 
 // 1-D Q1 integrals on [0,1]: mass, stiffness, and C[i][j] = int psi_i' psi_j.
-__host__ __device__ inline double q1_mass(int i, int j) { return i == j ? 1.0 / 3.0 : 1.0 / 6.0; }
-__host__ __device__ inline double q1_stiff(int i, int j) { return i == j ? 1.0 : -1.0; }
-__host__ __device__ inline double q1_mixed(int i, int /*j*/) { return i ? 0.5 : -0.5; }
+__host__ __device__ constexpr inline double q1_mass(int i, int j) { return i == j ? 1.0 / 3.0 : 1.0 / 6.0; }
+__host__ __device__ constexpr inline double q1_stiff(int i, int j) { return i == j ? 1.0 : -1.0; }
+__host__ __device__ constexpr inline double q1_mixed(int i, int /*j*/) { return i ? 0.5 : -0.5; }
 
 // I_ab(i,j) = int_{[0,1]^3} d_a phi_i d_b phi_j for hex8 corners i, j
-__host__ __device__ inline double q1_grad_integral(int a, int b, int i, int j) {
+__host__ __device__ constexpr inline double q1_grad_integral(int a, int b, int i, int j) {
     const int bi[3] = {hex8_cx(i), hex8_cy(i), hex8_cz(i)};
     const int bj[3] = {hex8_cx(j), hex8_cy(j), hex8_cz(j)};
     double r = 1.0;
     for (int d = 0; d < 3; d++) {
-        double t;
+        double t = 0;
         if (d == a && d == b)
             t = q1_stiff(bi[d], bj[d]);
         else if (d == a)
@@ -266,6 +267,22 @@ inline unsigned grid_for(ptrdiff_t n, int block = kBlock, unsigned cap = 1u << 2
     if (g < 1) g = 1;
     if (g > (ptrdiff_t)cap) g = cap;
     return (unsigned)g;
+}
+
+
+// Dynamic LDS above the default 64 KB needs the function attribute, once per function and device.
+template <auto Fn>
+static int raise_lds_limit(size_t bytes) {
+    static std::atomic<uint64_t> done{0};
+    if (bytes <= 64 * 1024) return SFEM_SUCCESS;
+    int dev = 0;
+    SFEM_AMD_HIP_CHECK(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_acquire) & bit) return SFEM_SUCCESS;
+    SFEM_AMD_HIP_CHECK(
+        hipFuncSetAttribute((const void *)Fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    done.fetch_or(bit, std::memory_order_acq_rel);
+    return SFEM_SUCCESS;
 }
 
 }  // namespace sfem_amd

@@ -25,7 +25,7 @@ __device__ __forceinline__ void atomic_add(T *p, T v) {
 constexpr int round64(int n) { return ((n + 63) / 64) * 64; }
 
 template <int L>
-struct LapShape {
+struct LapShape {  // the diagonal kernel: a thread per x-line
     static constexpr int N1 = L + 1;
     static constexpr int NXE = N1 * N1 * N1;
     static constexpr int LINES = N1 * N1;
@@ -33,14 +33,34 @@ struct LapShape {
     static constexpr int BLOCK = round64(EPB * LINES);
 };
 
-// Computes the 8x8 sub-element matrices of the block's macro elements into sK.
-template <int L, int EPB, int BLOCK, typename G>
+// Entry (i, j) of the 8x8 Laplacian sub-element matrix as a combination of the six FFF words
+// (hex8_laplacian_entry with the integrals evaluated at compile time).
+struct LapEntryTable {
+    double c[64][6];
+    constexpr LapEntryTable() : c() {
+        for (int ij = 0; ij < 64; ij++) {
+            int q = 0;
+            for (int a = 0; a < 3; a++)
+                for (int b = a; b < 3; b++)
+                    c[ij][q++] = q1_grad_integral(a, b, ij / 8, ij % 8) +
+                                 (a == b ? 0.0 : q1_grad_integral(b, a, ij / 8, ij % 8));
+        }
+    }
+};
+__constant__ LapEntryTable lap_entry_table = LapEntryTable();
+
+// Computes the 8x8 sub-element matrices of the block's macro elements into sK (BLOCK is a multiple of
+// 64: a thread has one entry (i, j) of every fourth element or so, and loads its six coefficients once).
+template <int L, int EPB, int BLOCK, typename G, typename T>
 __device__ __forceinline__ void lap_block_matrices(ptrdiff_t E, ptrdiff_t e0, const G *__restrict__ fff,
                                                    ptrdiff_t fstride, const float *__restrict__ coeff,
-                                                   const double *__restrict__ Kem, double (*sK)[64]) {
+                                                   const double *__restrict__ Kem, T (*sK)[64]) {
     const double h = 1.0 / L;
-    for (int k = threadIdx.x; k < EPB * 64; k += BLOCK) {
-        const int le = k >> 6, ij = k & 63;
+    const int ij = threadIdx.x & 63;
+    double t[6];
+#pragma unroll
+    for (int q = 0; q < 6; q++) t[q] = lap_entry_table.c[ij][q];
+    for (int le = threadIdx.x >> 6; le < EPB; le += BLOCK / 64) {
         const ptrdiff_t e = e0 + le;
         double v = 0;
         if (e < E && Kem) {
@@ -48,361 +68,204 @@ __device__ __forceinline__ void lap_block_matrices(ptrdiff_t E, ptrdiff_t e0, co
             // (operators/stencil/sshex8_stencil_element_matrix_apply.cpp:10-78)
             v = Kem[e * 64 + ij];
         } else if (e < E) {
-            double f[6];
-            const double c = (coeff ? (double)coeff[e] : 1.0) * h;
 #pragma unroll
-            for (int q = 0; q < 6; q++) f[q] = load_geom<G>(fff, q * fstride + e) * c;
-            v = hex8_laplacian_entry(f, ij >> 3, ij & 7);
+            for (int q = 0; q < 6; q++) v += load_geom<G>(fff, q * fstride + e) * t[q];
+            v *= (coeff ? (double)coeff[e] : 1.0) * h;
         }
-        sK[le][ij] = v;
+        sK[le][ij] = (T)v;
     }
 }
 
-// y += A x for the sshex8 Laplacian.  One thread per x-line (y,z) of a macro element;
-// the line's node values sit in LDS, a 3x3x3 register window slides along x.  The
-// node's stencil is split into S_a (micro elements whose lower x-corner is the node) and
-// S_b (upper x-corner), each masked by which y/z micro elements exist inside the macro
-// element, so x = 0 and x = L (skeleton) need no divergent code: the whole wave is at
-// the same x.  Interior nodes are owned by one macro element: their y values are loaded
-// together with x (before the barrier), so the sweep only stores.
-// Skeleton nodes are shared: their element contributions go to the element's slots of
-// `part` (plain stores, no atomics) and skeleton_gather_kernel sums them per node in a
-// fixed order, so the result is bitwise reproducible.
+// Skeleton slot of each local node, -1 for interior ones.
+template <int L>
+struct LapSlotTable {
+    int16_t v[nxe_of(L)];
+    constexpr LapSlotTable() : v() {
+        for (int z = 0; z <= L; z++)
+            for (int y = 0; y <= L; y++)
+                for (int x = 0; x <= L; x++) v[lidx(L, x, y, z)] = (int16_t)sk_slot(L, x, y, z);
+    }
+};
+template <int L>
+__constant__ LapSlotTable<L> lap_slot_table = LapSlotTable<L>();
+
+// Elements per block of the apply: about 256 lines, fewer at the small levels, whose meshes are the coarse
+// ones of a hierarchy (level 2 on 4,096 elements: 147 blocks of 256 threads left a third of the CUs idle).
+template <int L>
+struct LapApply {
+    static constexpr int N1 = L + 1, NXE = N1 * N1 * N1, LINES = N1 * N1;
+    static constexpr int WANT = LINES <= 16 ? 64 : LINES <= 25 ? 128 : 256;
+    static constexpr int EPB = LINES >= WANT ? 1 : WANT / LINES, BLOCK = round64(EPB * LINES);
+    static constexpr int SLOTS = EPB * NXE, PER_THREAD = (SLOTS + BLOCK - 1) / BLOCK;
+    template <typename T>
+    static constexpr size_t lds_bytes() {
+        return ((size_t)EPB * 64 + (size_t)SLOTS * 2) * sizeof(T);
+    }
+};
+
+// y += A x for the sshex8 Laplacian, in three phases around LDS:
+//   1. the block's node slots, consecutive threads on consecutive slots of the element-major connectivity,
+//      whose ids run in long consecutive stretches: id, then x (to LDS) and the old y (interior nodes,
+//      accumulating) or the skeleton slot position (both kept in registers), each as one batch of loads;
+//   2. a thread per x-line (y, z) sweeps it: the nine lines around it are read once per x, and each column
+//      feeds the three outputs x - 1, x, x + 1 (27 products in three chains).  S[d] is the stencil's
+//      column at dx = d - 1, masked by which micro elements exist in y and z; the node's own column is the
+//      sum of the lower and the upper micro elements' parts, of which x = 0 and x = L see one: the whole
+//      wave is at the same x, so there is no divergent code;
+//   3. per slot again: interior nodes store their y; skeleton nodes, shared with other elements, store the
+//      element's contribution to its slot of `part` (plain stores, no atomics), and
+//      skeleton_gather_kernel sums them per node in a fixed order: bitwise reproducible.  part == null:
+//      added to y with atomics instead.
+// What bounds it: instruction issue (about 1,600 per wave at L = 8, 243 of them the sweep's products) and the
+// latency of the two dependent loads and of the stores around it.  The former kernel (a thread per line
+// loading and storing its own nodes, so that each access touched 36 lines, 36 products per node and 222
+// registers in FP64) took 33 us in FP64 for 16^3 elements of L = 8 and 170 us in FP32 for 32^3 (there staged
+// through LDS too, with its loads behind branches); this one 23 and 115 us.
 template <typename T, typename G, int L>
-__global__ void __launch_bounds__(LapShape<L>::BLOCK)
+__global__ void __launch_bounds__(LapApply<L>::BLOCK)
     sshex8_laplacian_apply_kernel(const ptrdiff_t E, const int32_t *__restrict__ idx, const G *__restrict__ fff,
                                   const ptrdiff_t fstride, const float *__restrict__ coeff,
                                   const double *__restrict__ Kem, const T *__restrict__ x, T *__restrict__ y,
                                   T *__restrict__ part, const int32_t *__restrict__ sk_pos, const int overwrite) {
-    using S = LapShape<L>;
-    constexpr int N1 = S::N1, NXE = S::NXE, LINES = S::LINES, EPB = S::EPB, NSK = sk_count(L);
-    __shared__ T su[EPB][NXE];
-    __shared__ double sK[EPB][64];
-
-    const int tid = threadIdx.x;
-    const int le = tid / LINES;
-    const int line = tid - le * LINES;
-    const int yy = line % N1, zz = line / N1;
-    const ptrdiff_t e0 = xcd_contiguous_block(blockIdx.x, gridDim.x) * EPB;
-    const ptrdiff_t e = e0 + le;
-    const bool active = (le < EPB) && (e < E);
-
-    const bool skl = sk_line(L, yy, zz);
-    int32_t gid[N1];
-    T old[N1];  // y of the interior nodes of an interior line, loaded early
-    if (active) {
-        const int32_t *row = idx + e * NXE + lidx(L, 0, yy, zz);
-#pragma unroll
-        for (int i = 0; i < N1; i++) gid[i] = row[i];
-#pragma unroll
-        for (int i = 0; i < N1; i++) su[le][lidx(L, i, yy, zz)] = x[gid[i]];
-        if (!skl) {
-#pragma unroll
-            for (int i = 1; i < L; i++) old[i] = overwrite ? T(0) : y[gid[i]];
-        }
-    }
-    lap_block_matrices<L, EPB, S::BLOCK, G>(E, e0, fff, fstride, coeff, Kem, sK);
-    __syncthreads();
-    if (!active) return;
-
-    // masked stencil halves: [dz+1][dy+1][dx'] with dx' = dx (S_a, dx in {0,1}) or dx+1 (S_b)
-    T Sa[3][3][2], Sb[3][3][2];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int b = 0; b < 3; b++)
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                Sa[a][b][c] = 0;
-                Sb[a][b][c] = 0;
-            }
-    const double *K = sK[le];
-#pragma unroll
-    for (int cz = 0; cz < 2; cz++) {
-        const bool okz = cz ? (zz > 0) : (zz < L);
-#pragma unroll
-        for (int cy = 0; cy < 2; cy++) {
-            const bool oky = cy ? (yy > 0) : (yy < L);
-            const double m = (okz && oky) ? 1.0 : 0.0;
-#pragma unroll
-            for (int dz = -cz; dz <= 1 - cz; dz++)
-#pragma unroll
-                for (int dy = -cy; dy <= 1 - cy; dy++) {
-                    const int ra = hex8_corner(0, cy, cz), rb = hex8_corner(1, cy, cz);
-#pragma unroll
-                    for (int dx = 0; dx < 2; dx++) {
-                        Sa[dz + 1][dy + 1][dx] += (T)(m * K[ra * 8 + hex8_corner(dx, cy + dy, cz + dz)]);
-                        Sb[dz + 1][dy + 1][dx] += (T)(m * K[rb * 8 + hex8_corner(dx, cy + dy, cz + dz)]);
-                    }
-                }
-        }
-    }
-
-    // sliding window: w[s][dz+1][dy+1], s = 0: x-1, 1: x, 2: x+1
-    const int yl = yy > 0 ? yy - 1 : 0, yh = yy < L ? yy + 1 : L;
-    const int zl = zz > 0 ? zz - 1 : 0, zh = zz < L ? zz + 1 : L;
-    const int ys[3] = {yl, yy, yh}, zs[3] = {zl, zz, zh};
-    const T *u = su[le];
-    T w[3][3][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            w[0][a][b] = 0;
-            w[1][a][b] = u[lidx(L, 0, ys[b], zs[a])];
-            w[2][a][b] = u[lidx(L, 1, ys[b], zs[a])];
-        }
-
-    // part positions of this line's skeleton nodes (all L+1 on a skeleton line, else x = 0, L);
-    // part == null: skeleton contributions are added to y atomically instead (accumulating apply)
-    const int32_t *pp = sk_pos + e * NSK + sk_line_base(L, yy, zz);
-    int32_t ppos[N1];
-    if (part) {
-        if (skl) {
-#pragma unroll
-            for (int i = 0; i <= L; i++) ppos[i] = pp[i];
-        } else {
-            ppos[0] = pp[0];
-            ppos[L] = pp[1];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i <= L; i++) {
-        T v = 0;
-        if (i < L) {
-#pragma unroll
-            for (int a = 0; a < 3; a++)
-#pragma unroll
-                for (int b = 0; b < 3; b++) {
-                    v = fma(Sa[a][b][0], w[1][a][b], v);
-                    v = fma(Sa[a][b][1], w[2][a][b], v);
-                }
-        }
-        if (i > 0) {
-#pragma unroll
-            for (int a = 0; a < 3; a++)
-#pragma unroll
-                for (int b = 0; b < 3; b++) {
-                    v = fma(Sb[a][b][0], w[0][a][b], v);
-                    v = fma(Sb[a][b][1], w[1][a][b], v);
-                }
-        }
-        if (skl || i == 0 || i == L) {
-            if (part)
-                part[ppos[i]] = v;
-            else
-                atomic_add(&y[gid[i]], v);
-        } else {
-            y[gid[i]] = old[i] + v;
-        }
-        // slide
-        if (i < L) {
-#pragma unroll
-            for (int a = 0; a < 3; a++)
-#pragma unroll
-                for (int b = 0; b < 3; b++) {
-                    w[0][a][b] = w[1][a][b];
-                    w[1][a][b] = w[2][a][b];
-                    w[2][a][b] = (i + 2 <= L) ? u[lidx(L, i + 2 <= L ? i + 2 : L, ys[b], zs[a])] : T(0);
-                }
-        }
-    }
-
-}
-
-// The same operator with the block's memory traffic staged through LDS (levels whose block
-// tile fits in 64 KB).  A thread per x-line makes each of the line's loads and stores a
-// 64-lane access spread over ~30 cache lines (lanes one line apart); here the block's node
-// slots are read and written with consecutive threads on consecutive slots of the
-// element-major connectivity, whose ids run in long consecutive stretches, instead:
-//   1. per slot: its id, x, and the old y (interior nodes, accumulating) or the skeleton slot
-//      position, into LDS (one unrolled batch of loads per thread);
-//   2. the line sweep of the kernel above, from LDS x into the LDS results (each node has one
-//      line thread, so no two threads touch a result);
-//   3. per slot: interior nodes store their y, skeleton nodes their partial (or, without
-//      partials, add to y atomically).
-template <int L>
-struct LapStagedShape {
-    static constexpr int N1 = L + 1, NXE = N1 * N1 * N1, LINES = N1 * N1;
-    static constexpr int EPB = LapShape<L>::EPB, BLOCK = LapShape<L>::BLOCK;
-    static constexpr int SLOTS = EPB * NXE, PER_THREAD = (SLOTS + BLOCK - 1) / BLOCK;
-    template <typename T>
-    static constexpr size_t lds_bytes() {
-        return (size_t)SLOTS * (2 * sizeof(T) + sizeof(int32_t)) + (size_t)EPB * 64 * sizeof(double);
-    }
-};
-
-// Used for FP32 vectors: at 113 VGPRs the staged kernel runs 4 waves per SIMD and beats the
-// line-thread loads (L=8 on 32^3: 165 vs 189 us); in FP64 both kernels hold ~200 VGPRs (2 waves
-// per SIMD, the window and the masked stencil halves) and the three phases of the staged one
-// overlap worse (280 vs 242 us), so FP64 keeps the line-thread kernel.
-template <typename T, int L>
-constexpr bool lap_staged_used() {
-    return std::is_same<T, float>::value && LapStagedShape<L>::template lds_bytes<T>() <= 64 * 1024;
-}
-
-template <typename T, typename G, int L>
-__global__ void __launch_bounds__(LapShape<L>::BLOCK)
-    sshex8_laplacian_apply_staged_kernel(const ptrdiff_t E, const int32_t *__restrict__ idx, const G *__restrict__ fff,
-                                         const ptrdiff_t fstride, const float *__restrict__ coeff,
-                                         const double *__restrict__ Kem, const T *__restrict__ x, T *__restrict__ y,
-                                         T *__restrict__ part, const int32_t *__restrict__ sk_pos,
-                                         const int overwrite) {
-    using S = LapStagedShape<L>;
-    constexpr int N1 = S::N1, NXE = S::NXE, LINES = S::LINES, EPB = S::EPB, NSK = sk_count(L);
-    __shared__ T su[EPB][NXE];      // x of the block's nodes
-    __shared__ T sy[EPB][NXE];      // old y (interior, accumulating) or 0, then the results
-    __shared__ int32_t st[EPB][NXE];  // store target: node id (interior; skeleton without partials) or slot position
-    __shared__ double sK[EPB][64];
+    using S = LapApply<L>;
+    constexpr int N1 = S::N1, NXE = S::NXE, LINES = S::LINES, EPB = S::EPB, NSK = sk_count(L), PT = S::PER_THREAD;
+    extern __shared__ __align__(16) unsigned char lap_lds[];
+    T(*sK)[64] = reinterpret_cast<T(*)[64]>(lap_lds);
+    T *su = &sK[EPB][0], *sy = su + S::SLOTS;
 
     const int tid = threadIdx.x;
     const ptrdiff_t e0 = xcd_contiguous_block(blockIdx.x, gridDim.x) * EPB;
-    const ptrdiff_t nslots = (E - e0 < EPB ? E - e0 : EPB) * (ptrdiff_t)NXE;
-    T *su0 = &su[0][0], *sy0 = &sy[0][0];
-    int32_t *st0 = &st[0][0];
+    const int nslots = (int)(E - e0 < EPB ? E - e0 : EPB) * NXE;
 
-    // 1. ids, then x and old y or slot positions, of this thread's slots
+    // 1. No load waits behind a branch: slots past the end re-read the block's first one (and are not stored),
+    // skeleton slots read the old y, and interior ones a slot position, at one address for all
+    int32_t tg[PT];  // where the result goes: node id, or position in part
+    T yo[PT];
+    unsigned skel = 0;
     {
-        int32_t id[S::PER_THREAD];
+        int16_t sl[PT];
 #pragma unroll
-        for (int k = 0; k < S::PER_THREAD; k++) {
-            const int sl = tid + k * S::BLOCK;
-            id[k] = sl < nslots ? idx[e0 * NXE + sl] : 0;
+        for (int k = 0; k < PT; k++) {
+            const int i = tid + k * S::BLOCK, ii = i < nslots ? i : 0;
+            tg[k] = idx[e0 * NXE + ii];
+            sl[k] = lap_slot_table<L>.v[ii % NXE];
+            skel |= (sl[k] >= 0 ? 1u : 0u) << k;
         }
-        T xv[S::PER_THREAD], yv[S::PER_THREAD];
-        int32_t tg[S::PER_THREAD];
+        T xv[PT];
+        const int32_t one = __builtin_amdgcn_readfirstlane(tg[0]);
 #pragma unroll
-        for (int k = 0; k < S::PER_THREAD; k++) {
-            const int sl = tid + k * S::BLOCK;
-            const int le = sl / NXE, n = sl - le * NXE;
-            const int cx = n % N1, cy = (n / N1) % N1, cz = n / (N1 * N1);
-            const int slot = sk_slot(L, cx, cy, cz);
-            const bool ok = sl < nslots;
-            xv[k] = ok ? x[id[k]] : T(0);
-            yv[k] = (ok && slot < 0 && !overwrite) ? y[id[k]] : T(0);
-            tg[k] = (ok && slot >= 0 && part) ? sk_pos[(e0 + le) * NSK + slot] : id[k];
+        for (int k = 0; k < PT; k++) xv[k] = x[tg[k]];
+        if (overwrite) {
+#pragma unroll
+            for (int k = 0; k < PT; k++) yo[k] = T(0);
+        } else {
+#pragma unroll
+            for (int k = 0; k < PT; k++) yo[k] = y[sl[k] >= 0 ? one : tg[k]];
         }
+        if (part) {
 #pragma unroll
-        for (int k = 0; k < S::PER_THREAD; k++) {
-            const int sl = tid + k * S::BLOCK;
-            if (sl < S::SLOTS) {
-                su0[sl] = xv[k];
-                sy0[sl] = yv[k];
-                st0[sl] = tg[k];
+            for (int k = 0; k < PT; k++) {
+                const int i = tid + k * S::BLOCK, ii = i < nslots ? i : 0;
+                const int32_t p = sk_pos[sl[k] >= 0 ? (e0 + ii / NXE) * NSK + sl[k] : e0 * NSK];
+                tg[k] = sl[k] >= 0 ? p : tg[k];
             }
+        }
+#pragma unroll
+        for (int k = 0; k < PT; k++) {
+            const int i = tid + k * S::BLOCK;
+            if (i < S::SLOTS) su[i] = xv[k];
         }
     }
     lap_block_matrices<L, EPB, S::BLOCK, G>(E, e0, fff, fstride, coeff, Kem, sK);
     __syncthreads();
 
-    // 2. the line sweep
+    // 2.
     const int le = tid / LINES, line = tid - le * LINES;
-    const int yy = line % N1, zz = line / N1;
     if (le < EPB && e0 + le < E) {
-        T Sa[3][3][2], Sb[3][3][2];
+        const int yy = line % N1, zz = line / N1;
+        const T *K = sK[le];
+        // the parts of the stencil: lower micro elements (the node is their lower x corner) at dx = 0, 1, upper ones
+        // at dx = -1, 0
+        T lo0[9], lo1[9], up0[9], up1[9];
+        auto column = [&](int cx, int dx, T(&c)[9]) {
 #pragma unroll
-        for (int a = 0; a < 3; a++)
+            for (int k = 0; k < 9; k++) c[k] = T(0);
 #pragma unroll
-            for (int b = 0; b < 3; b++)
+            for (int cz = 0; cz < 2; cz++)
 #pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    Sa[a][b][c] = 0;
-                    Sb[a][b][c] = 0;
-                }
-        const double *K = sK[le];
+                for (int cy = 0; cy < 2; cy++) {
+                    const T m = (cz ? zz > 0 : zz < L) && (cy ? yy > 0 : yy < L) ? T(1) : T(0);
 #pragma unroll
-        for (int cz = 0; cz < 2; cz++) {
-            const bool okz = cz ? (zz > 0) : (zz < L);
+                    for (int dz = -cz; dz <= 1 - cz; dz++)
 #pragma unroll
-            for (int cy = 0; cy < 2; cy++) {
-                const bool oky = cy ? (yy > 0) : (yy < L);
-                const double m = (okz && oky) ? 1.0 : 0.0;
-#pragma unroll
-                for (int dz = -cz; dz <= 1 - cz; dz++)
-#pragma unroll
-                    for (int dy = -cy; dy <= 1 - cy; dy++) {
-                        const int ra = hex8_corner(0, cy, cz), rb = hex8_corner(1, cy, cz);
-#pragma unroll
-                        for (int dx = 0; dx < 2; dx++) {
-                            Sa[dz + 1][dy + 1][dx] += (T)(m * K[ra * 8 + hex8_corner(dx, cy + dy, cz + dz)]);
-                            Sb[dz + 1][dy + 1][dx] += (T)(m * K[rb * 8 + hex8_corner(dx, cy + dy, cz + dz)]);
+                        for (int dy = -cy; dy <= 1 - cy; dy++) {
+                            T &e = c[(dz + 1) * 3 + dy + 1];
+                            e = fma(m, K[hex8_corner(cx, cy, cz) * 8 + hex8_corner(cx + dx, cy + dy, cz + dz)], e);
                         }
-                    }
-            }
-        }
-        const int yl = yy > 0 ? yy - 1 : 0, yh = yy < L ? yy + 1 : L;
-        const int zl = zz > 0 ? zz - 1 : 0, zh = zz < L ? zz + 1 : L;
-        const int ys[3] = {yl, yy, yh}, zs[3] = {zl, zz, zh};
-        const T *__restrict__ u = su[le];
-        T *__restrict__ out = sy[le];
-        T res[N1];
-        T w[3][3][3];
+                }
+        };
+        column(0, 0, lo0);
+        column(0, 1, lo1);
+        column(1, -1, up0);
+        // lines around this one (clamped: their coefficients are zero where they do not exist)
+        int at[9];
 #pragma unroll
         for (int a = 0; a < 3; a++)
 #pragma unroll
             for (int b = 0; b < 3; b++) {
-                w[0][a][b] = 0;
-                w[1][a][b] = u[lidx(L, 0, ys[b], zs[a])];
-                w[2][a][b] = u[lidx(L, 1, ys[b], zs[a])];
+                const int z = zz + a - 1, q = yy + b - 1;
+                at[a * 3 + b] = le * NXE + lidx(L, 0, q < 0 ? 0 : (q > L ? L : q), z < 0 ? 0 : (z > L ? L : z));
             }
+        T *out = sy + le * NXE + line * N1;
+        T u[9], prev = T(0), cur = T(0), next = T(0);
+        auto dot = [&](const T(&c)[9], T v) {
 #pragma unroll
-        for (int i = 0; i <= L; i++) {
-            T v = 0;
-            if (i < L) {
+            for (int k = 0; k < 9; k++) v = fma(c[k], u[k], v);
+            return v;
+        };
 #pragma unroll
-                for (int a = 0; a < 3; a++)
+        for (int k = 0; k < 9; k++) u[k] = su[at[k]];
+        prev = dot(lo0, T(0));
+        cur = dot(up0, T(0));
+        column(1, 0, up1);
 #pragma unroll
-                    for (int b = 0; b < 3; b++) {
-                        v = fma(Sa[a][b][0], w[1][a][b], v);
-                        v = fma(Sa[a][b][1], w[2][a][b], v);
-                    }
-            }
-            if (i > 0) {
+        for (int k = 0; k < 9; k++) lo0[k] += up1[k];  // the interior nodes' own column
 #pragma unroll
-                for (int a = 0; a < 3; a++)
+        for (int i = 1; i < L; i++) {
 #pragma unroll
-                    for (int b = 0; b < 3; b++) {
-                        v = fma(Sb[a][b][0], w[0][a][b], v);
-                        v = fma(Sb[a][b][1], w[1][a][b], v);
-                    }
-            }
-            res[i] = v;
-            if (i < L) {
-#pragma unroll
-                for (int a = 0; a < 3; a++)
-#pragma unroll
-                    for (int b = 0; b < 3; b++) {
-                        w[0][a][b] = w[1][a][b];
-                        w[1][a][b] = w[2][a][b];
-                        w[2][a][b] = (i + 2 <= L) ? u[lidx(L, i + 2 <= L ? i + 2 : L, ys[b], zs[a])] : T(0);
-                    }
-            }
+            for (int k = 0; k < 9; k++) u[k] = su[at[k] + i];
+            out[i - 1] = dot(lo1, prev);
+            prev = dot(lo0, cur);
+            cur = dot(up0, T(0));
         }
-        // the line's results after the sweep (no LDS store inside it, so the window may be re-read)
 #pragma unroll
-        for (int i = 0; i <= L; i++) {
-            const int n = lidx(L, i, yy, zz);
-            out[n] += res[i];
-        }
+        for (int k = 0; k < 9; k++) u[k] = su[at[k] + L];
+        out[L - 1] = dot(lo1, prev);
+        column(1, 0, up1);
+        out[L] = dot(up1, cur);
     }
     __syncthreads();
 
-    // 3. the stores
+    // 3.
+    T v[PT];
 #pragma unroll
-    for (int k = 0; k < S::PER_THREAD; k++) {
-        const int sl = tid + k * S::BLOCK;
-        if (sl < nslots) {
-            const int n = sl % NXE;
-            const int cx = n % N1, cy = (n / N1) % N1, cz = n / (N1 * N1);
-            const bool skel = sk_slot(L, cx, cy, cz) >= 0;
-            const T v = sy0[sl];
-            const int32_t t = st0[sl];
-            if (!skel)
-                y[t] = v;
-            else if (part)
-                part[t] = v;
+    for (int k = 0; k < PT; k++) {
+        const int i = tid + k * S::BLOCK;
+        v[k] = sy[i < S::SLOTS ? i : 0];
+        if (!((skel >> k) & 1u)) v[k] += yo[k];
+    }
+    if (part) {
+#pragma unroll
+        for (int k = 0; k < PT; k++)
+            if (tid + k * S::BLOCK < nslots) ((skel >> k) & 1u ? part : y)[tg[k]] = v[k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < PT; k++) {
+            if (tid + k * S::BLOCK >= nslots) continue;
+            if ((skel >> k) & 1u)
+                atomic_add(&y[tg[k]], v[k]);
             else
-                atomic_add(&y[t], v);
+                y[tg[k]] = v[k];
         }
     }
 }
@@ -1374,14 +1237,12 @@ int sshex8_laplacian_apply(int L, ptrdiff_t E, const int32_t *idx, const G *fff,
     switch (L) {
 #define CASE(LV)                                                                                                  \
     case LV: {                                                                                                    \
-        using Sh = LapShape<LV>;                                                                                  \
+        using Sh = LapApply<LV>;                                                                                  \
         const unsigned grid = (unsigned)((E + Sh::EPB - 1) / Sh::EPB);                                            \
-        if constexpr (lap_staged_used<T, LV>())                                                                   \
-            sshex8_laplacian_apply_staged_kernel<T, G, LV><<<grid, Sh::BLOCK, 0, s>>>(                            \
-                E, idx, fff, fstride, coeff, Kem, x, y, part, sk.pos, overwrite);                                 \
-        else                                                                                                      \
-            sshex8_laplacian_apply_kernel<T, G, LV><<<grid, Sh::BLOCK, 0, s>>>(E, idx, fff, fstride, coeff, Kem, x, y, \
-                                                                                 part, sk.pos, overwrite);        \
+        constexpr size_t lds = Sh::template lds_bytes<T>();                                                       \
+        if (raise_lds_limit<sshex8_laplacian_apply_kernel<T, G, LV>>(lds)) return SFEM_FAILURE;                   \
+        sshex8_laplacian_apply_kernel<T, G, LV><<<grid, Sh::BLOCK, lds, s>>>(E, idx, fff, fstride, coeff, Kem, x, y, \
+                                                                             part, sk.pos, overwrite);            \
         break;                                                                                                    \
     }
         SFEM_AMD_SSHEX8_LEVELS(CASE)
