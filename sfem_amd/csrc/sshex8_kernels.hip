@@ -297,55 +297,61 @@ struct MfmaAcc<float> {
 // operator's y = x there), or to zero without cx (a restriction onto constrained dofs), instead.
 // With a Chebyshev step (cs.p != null, overwriting apply): the node's product t feeds the step
 // (p and x updated there, y not written).
-template <typename T, int BS>
+// A thread takes CT of a node's BS components: one of three in FP64, where a wave's loads then run over
+// consecutive words (10.4M nodes: 323 us against 366 for all three in turn), all of them in FP32, whose
+// 12-byte nodes gain less from that than the threefold offset loads cost (5.7M nodes: 107 against 121 us).
+template <typename T, int BS, int CT>
 __global__ void skeleton_gather_kernel(const ptrdiff_t n, const int32_t *__restrict__ node,
                                        const int32_t *__restrict__ off, const int32_t *__restrict__ ent,
                                        const T *__restrict__ part, T *__restrict__ y, const int overwrite,
                                        const uint8_t *__restrict__ cmask, const T *cx, const ChebStep<T> cs) {
     // the first NU partials of a node (face nodes have 2, edge nodes 4) are loaded together with its
     // old value, right after its offsets: two memory round trips per node instead of one per partial
-    constexpr int NU = 4;
-    for (ptrdiff_t t = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (ptrdiff_t)gridDim.x * blockDim.x) {
+    constexpr int NU = 4, PER = BS / CT;
+    for (ptrdiff_t i = (ptrdiff_t)blockIdx.x * blockDim.x + threadIdx.x; i < n * PER;
+         i += (ptrdiff_t)gridDim.x * blockDim.x) {
+        const ptrdiff_t t = i / PER;
+        const int c0 = (int)(i - t * PER) * CT;
         const int j0 = off[t], j1 = off[t + 1];
-        const ptrdiff_t g = (ptrdiff_t)node[t] * BS;
-        const unsigned cm = cmask ? cmask[t] : 0u;
-        T acc[BS], yo[BS];
+        const ptrdiff_t g = (ptrdiff_t)node[t] * BS + c0;
+        const unsigned cm = cmask ? (unsigned)cmask[t] >> c0 : 0u;
+        T acc[CT], yo[CT];
 #pragma unroll
-        for (int c = 0; c < BS; c++) acc[c] = yo[c] = 0;
+        for (int c = 0; c < CT; c++) acc[c] = yo[c] = 0;
         if (!ent) {
             // absent slots re-read the node's first partial (a valid index: every skeleton node has
             // one) and are zeroed after the load, so that no load waits behind a branch
-            T pv[NU][BS];
+            T pv[NU][CT];
 #pragma unroll
             for (int k = 0; k < NU; k++) {
-                const ptrdiff_t q = (ptrdiff_t)(j0 + k < j1 ? j0 + k : j0) * BS;
+                const ptrdiff_t q = (ptrdiff_t)(j0 + k < j1 ? j0 + k : j0) * BS + c0;
 #pragma unroll
-                for (int c = 0; c < BS; c++) pv[k][c] = part[q + c];
+                for (int c = 0; c < CT; c++) pv[k][c] = part[q + c];
             }
             if (!overwrite)
 #pragma unroll
-                for (int c = 0; c < BS; c++) yo[c] = y[g + c];
+                for (int c = 0; c < CT; c++) yo[c] = y[g + c];
             // in slot order, as the loop below (adding the zeros of absent slots leaves the sum's
             // words unchanged: it starts at +0 and never becomes -0)
 #pragma unroll
             for (int k = 0; k < NU; k++)
 #pragma unroll
-                for (int c = 0; c < BS; c++) acc[c] += j0 + k < j1 ? pv[k][c] : T(0);
+                for (int c = 0; c < CT; c++) acc[c] += j0 + k < j1 ? pv[k][c] : T(0);
             for (int j = j0 + NU; j < j1; j++)
 #pragma unroll
-                for (int c = 0; c < BS; c++) acc[c] += part[(ptrdiff_t)j * BS + c];
+                for (int c = 0; c < CT; c++) acc[c] += part[(ptrdiff_t)j * BS + c0 + c];
         } else {
             if (!overwrite)
 #pragma unroll
-                for (int c = 0; c < BS; c++) yo[c] = y[g + c];
+                for (int c = 0; c < CT; c++) yo[c] = y[g + c];
             for (int j = j0; j < j1; j++) {
-                const ptrdiff_t q = (ptrdiff_t)ent[j] * BS;
+                const ptrdiff_t q = (ptrdiff_t)ent[j] * BS + c0;
 #pragma unroll
-                for (int c = 0; c < BS; c++) acc[c] += part[q + c];
+                for (int c = 0; c < CT; c++) acc[c] += part[q + c];
             }
         }
 #pragma unroll
-        for (int c = 0; c < BS; c++) {
+        for (int c = 0; c < CT; c++) {
             const T v = ((cm >> c) & 1u) ? (cx ? cx[g + c] : T(0)) : (overwrite ? acc[c] : yo[c] + acc[c]);
             if (cs.p) {
                 const T pi = cheb3_direction<T>(cs.first ? T(0) : cs.p[g + c], cs.rhs[g + c], v, cs.beta, cs.dinv, g + c,
@@ -600,6 +606,55 @@ struct ElMfma {
     static constexpr int WPE = 4 / EPB;                  // waves per macro element
 };
 
+// The nodes k = tid + 256 i of a block's macro elements, for the matrix-core kernels: ids, then x, the old y
+// (interior nodes of an accumulating apply; 0 otherwise) and the skeleton slot positions as one batch.  No
+// load waits behind a branch: absent nodes re-read the block's first one, and a node that needs no old y (or
+// no slot position) reads at one address for all such lanes.  gid -1: absent; pos -1: interior.
+template <typename T, int L, typename Lay, int EPB, int NPT>
+__device__ __forceinline__ void el_load_nodes(const ptrdiff_t E, const ptrdiff_t e0, const int32_t *__restrict__ idx,
+                                              const int32_t *__restrict__ sk_pos, const T *x, const T *y,
+                                              const int overwrite, int32_t (&gid)[NPT], int32_t (&pos)[NPT],
+                                              int (&lds)[NPT], T (&xv)[NPT][3], T (&yv)[NPT][3]) {
+    constexpr int NXE = nxe_of(L), NSK = sk_count(L);
+    const int tid = threadIdx.x;
+    const int n = (int)(E - e0 < EPB ? E - e0 : EPB) * NXE;
+    int slot[NPT];
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        const int k = tid + 256 * i;
+        gid[i] = idx[e0 * NXE + (k < n ? k : 0)];
+        slot[i] = sk_slot_table<L, Lay>.v[k % NXE];
+        lds[i] = sk_slot_table<L, Lay>.lds[k % NXE];
+    }
+    const int32_t one = __builtin_amdgcn_readfirstlane(gid[0]);
+#pragma unroll
+    for (int i = 0; i < NPT; i++)
+#pragma unroll
+        for (int ci = 0; ci < 3; ci++) xv[i][ci] = x[(ptrdiff_t)gid[i] * 3 + ci];
+    if (!overwrite) {
+#pragma unroll
+        for (int i = 0; i < NPT; i++)
+#pragma unroll
+            for (int ci = 0; ci < 3; ci++) yv[i][ci] = y[(ptrdiff_t)(slot[i] < 0 ? gid[i] : one) * 3 + ci];
+    }
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        const int k = tid + 256 * i;
+        pos[i] = sk_pos[slot[i] < 0 || k >= n ? e0 * NSK : (e0 + k / NXE) * NSK + slot[i]];
+    }
+#pragma unroll
+    for (int i = 0; i < NPT; i++) {
+        const bool ok = tid + 256 * i < n;
+#pragma unroll
+        for (int ci = 0; ci < 3; ci++) {
+            xv[i][ci] = ok ? xv[i][ci] : T(0);
+            yv[i][ci] = ok && slot[i] < 0 && !overwrite ? yv[i][ci] : T(0);
+        }
+        gid[i] = ok ? gid[i] : -1;
+        pos[i] = ok && slot[i] >= 0 ? pos[i] : -1;
+    }
+}
+
 typedef __bf16 el_b8 __attribute__((ext_vector_type(8)));
 typedef float el_f4 __attribute__((ext_vector_type(4)));
 
@@ -674,44 +729,6 @@ __global__ void __launch_bounds__(256)
     const int c = lane & 15, g = lane >> 4;
     const ptrdiff_t e0 = xcd_contiguous_block(blockIdx.x, gridDim.x) * EPB;
 
-    // node k = tid + 256 i of the block: ids first, then all values at once; interior nodes
-    // start from their y (accumulate), skeleton nodes from 0
-    int32_t gid[NPT], pos[NPT];  // node ids; node-sorted skeleton slots (-1: interior)
-    int lds[NPT];                // LDS positions
-    float xk[NPT][3];            // x of the node (the Chebyshev step updates interior ones)
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int k = tid + 256 * i, le = k / NXE;
-        gid[i] = (k < EPB * NXE && e0 + le < E) ? idx[e0 * NXE + k] : -1;
-    }
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int k = tid + 256 * i, le = k / NXE, v = k - le * NXE;
-        const int slot = sk_slot_table<L>.v[v];
-        lds[i] = sk_slot_table<L>.lds[v];
-        const bool interior = slot < 0;
-        pos[i] = (gid[i] >= 0 && !interior) ? sk_pos[(e0 + le) * NSK + slot] : -1;
-        float xv[3] = {0, 0, 0}, yv[3] = {0, 0, 0};
-        if (gid[i] >= 0) {
-            const float *xp = x + (ptrdiff_t)gid[i] * 3;
-            const float *yp = y + (ptrdiff_t)gid[i] * 3;
-#pragma unroll
-            for (int ci = 0; ci < 3; ci++) {
-                xv[ci] = xp[ci];
-                if (interior && !overwrite) yv[ci] = yp[ci];
-            }
-        }
-        if (k < EPB * NXE) {
-#pragma unroll
-            for (int ci = 0; ci < 3; ci++) {
-                sx[le][ci][v] = el_split_pack(xv[ci]);
-                sy[le][ci][lds[i]] = yv[ci];
-            }
-        }
-#pragma unroll
-        for (int ci = 0; ci < 3; ci++) xk[i][ci] = xv[ci];
-    }
-
     // A operands (this wave's macro element): tile tt holds K rows 16tt + c, columns 8g + j
     const int le = wave / WPE, wsub = wave - le * WPE;
     const ptrdiff_t e = e0 + le;
@@ -725,6 +742,25 @@ __global__ void __launch_bounds__(256)
             alo[tt] = __builtin_bit_cast(el_b8, ak[(2 * tt + 1) * 64]);
         }
     }
+    int32_t gid[NPT], pos[NPT];  // node ids; node-sorted skeleton slots (-1: interior)
+    int lds[NPT];                // LDS positions
+    float xk[NPT][3];            // x of the node (the Chebyshev step updates interior ones)
+    {
+        float yv[NPT][3];
+        el_load_nodes<float, L, Y, EPB, NPT>(E, e0, idx, sk_pos, x, y, overwrite, gid, pos, lds, xk, yv);
+#pragma unroll
+        for (int i = 0; i < NPT; i++) {
+            const int k = tid + 256 * i, le2 = k / NXE, v = k - le2 * NXE;
+            if (k < EPB * NXE) {
+#pragma unroll
+                for (int ci = 0; ci < 3; ci++) {
+                    sx[le2][ci][v] = el_split_pack(xk[i][ci]);
+                    sy[le2][ci][lds[i]] = yv[i][ci];
+                }
+            }
+        }
+    }
+
     __syncthreads();
 
     // Tiles of 16 micro elements of one colour: wave wsub takes tiles wsub, wsub + WPE, ...  Lane
@@ -858,40 +894,7 @@ __global__ void __launch_bounds__(256)
     const int c = lane & 15, g = lane >> 4;
     const ptrdiff_t e0 = xcd_contiguous_block(blockIdx.x, gridDim.x) * EPB;
 
-    int32_t gid[NPT], pos[NPT];  // node ids; node-sorted skeleton slots (-1: interior)
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int k = tid + 256 * i, le = k / NXE;
-        gid[i] = (k < EPB * NXE && e0 + le < E) ? idx[e0 * NXE + k] : -1;
-    }
-    int lds[NPT];  // LDS positions
-#pragma unroll
-    for (int i = 0; i < NPT; i++) {
-        const int k = tid + 256 * i, le = k / NXE, v = k - le * NXE;
-        const int slot = sk_slot_table<L, Y>.v[v];
-        lds[i] = sk_slot_table<L, Y>.lds[v];
-        const bool interior = slot < 0;
-        pos[i] = (gid[i] >= 0 && !interior) ? sk_pos[(e0 + le) * NSK + slot] : -1;
-        double xv[3] = {0, 0, 0}, yv[3] = {0, 0, 0};
-        if (gid[i] >= 0) {
-            const double *xp = x + (ptrdiff_t)gid[i] * 3;
-            const double *yp = y + (ptrdiff_t)gid[i] * 3;
-#pragma unroll
-            for (int ci = 0; ci < 3; ci++) {
-                xv[ci] = xp[ci];
-                if (interior && !overwrite) yv[ci] = yp[ci];
-            }
-        }
-        if (k < EPB * NXE) {
-#pragma unroll
-            for (int ci = 0; ci < 3; ci++) {
-                sx[le][ci][lds[i]] = xv[ci];
-                sy[le][ci][lds[i]] = yv[ci];
-            }
-        }
-    }
-
-    // A: tile tt, step s holds K[16tt + c][4s + g]
+    // A: tile tt, step s holds K[16tt + c][4s + g] (rows past the 24 re-read the last one and are zeroed)
     const int le = wave / WPE, wsub = wave - le * WPE;
     const ptrdiff_t e = e0 + le;
     const bool active = e < E;
@@ -901,8 +904,26 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
         for (int s = 0; s < 6; s++) {
             const int row = 16 * tt + c;
-            a[tt][s] = (active && row < 24) ? Kall[(e >> kshift) * 576 + row * 24 + 4 * s + g] : 0.0;
+            const double v = Kall[((active ? e : e0) >> kshift) * 576 + (row < 24 ? row : 23) * 24 + 4 * s + g];
+            a[tt][s] = row < 24 ? v : 0.0;
         }
+    int32_t gid[NPT], pos[NPT];  // node ids; node-sorted skeleton slots (-1: interior)
+    int lds[NPT];                // LDS positions
+    {
+        double xv[NPT][3], yv[NPT][3];
+        el_load_nodes<double, L, Y, EPB, NPT>(E, e0, idx, sk_pos, x, y, overwrite, gid, pos, lds, xv, yv);
+#pragma unroll
+        for (int i = 0; i < NPT; i++) {
+            const int k = tid + 256 * i, le2 = k / NXE;
+            if (k < EPB * NXE) {
+#pragma unroll
+                for (int ci = 0; ci < 3; ci++) {
+                    sx[le2][ci][lds[i]] = xv[i][ci];
+                    sy[le2][ci][lds[i]] = yv[i][ci];
+                }
+            }
+        }
+    }
     __syncthreads();
 
 #pragma unroll 1
@@ -1212,12 +1233,13 @@ int skeleton_gather(const SkeletonMap &sk, int bs, const T *part, T *y, hipStrea
     if (node_sorted < 0) node_sorted = bs == 1;
     const int32_t *ent = node_sorted ? nullptr : sk.ent;
     const uint8_t *cm = sk.cmask;
+    constexpr int CT = std::is_same<T, double>::value ? 1 : 3;
     if (bs == 1)
-        skeleton_gather_kernel<T, 1>
+        skeleton_gather_kernel<T, 1, 1>
                 <<<grid_for(sk.n), kBlock, 0, s>>>(sk.n, sk.node, sk.off, ent, part, y, overwrite, cm, cx, cs);
     else if (bs == 3)
-        skeleton_gather_kernel<T, 3>
-                <<<grid_for(sk.n), kBlock, 0, s>>>(sk.n, sk.node, sk.off, ent, part, y, overwrite, cm, cx, cs);
+        skeleton_gather_kernel<T, 3, CT><<<grid_for(sk.n * (3 / CT)), kBlock, 0, s>>>(sk.n, sk.node, sk.off, ent, part, y,
+                                                                                    overwrite, cm, cx, cs);
     else {
         set_last_error("skeleton_gather: block size must be 1 or 3");
         return SFEM_FAILURE;
