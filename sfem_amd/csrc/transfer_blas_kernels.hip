@@ -92,93 +92,126 @@ __global__ void sshex8_restrict_kernel(const ptrdiff_t E, const int Lf, const in
     }
 }
 
-// LDS-staged variants, one macro element per block.
+__device__ __forceinline__ double mean(double a, double b) { return fma(0.5, a, 0.5 * b); }
+
+// LDS-staged variants, one macro element per block.  The level pairs of the usual hierarchies are template
+// parameters (LF > 0): with run-time levels the kernels spend most of their time on integer and FP64
+// divisions (coordinates, weights); other pairs run the LF = 0 form.  4,096 elements of level 8 to 4, FP64:
+// restriction 20.9 -> 15.3 us; prolongation 18.7 -> 17.8 us (about 55 MB of traffic; bound by its three
+// dependent loads); 512 elements, FP32 vectors of 3: 8.0 -> 7.7 and 7.7 -> 7.2 us.
 // Prolongation: the element's coarse values are staged in LDS once, then every owned fine node
 // interpolates from LDS (the per-node variant above re-reads up to 8 coarse values and their ids
 // from memory for every fine node).
-template <typename T, int VS>
-__global__ void __launch_bounds__(256) sshex8_prolongate_lds_kernel(const ptrdiff_t E, const int Lf, const int Lc,
+template <typename T, int VS, bool ADD, int LF, int LC>
+__global__ void __launch_bounds__(1024) sshex8_prolongate_lds_kernel(const ptrdiff_t E, const int Lf_, const int Lc_,
                                                                     const int32_t *__restrict__ idx,
                                                                     const uint8_t *__restrict__ own,
                                                                     const T *__restrict__ from, T *__restrict__ to,
-                                                                    const uint8_t *__restrict__ keep, const int add) {
+                                                                    const uint8_t *__restrict__ keep) {
     extern __shared__ double tr_smem[];
     const ptrdiff_t e = blockIdx.x;
     if (e >= E) return;  // uniform per block
+    const int Lf = LF ? LF : Lf_, Lc = LF ? LC : Lc_;
     const int N1 = Lf + 1, nxe = N1 * N1 * N1, s = Lf / Lc, C1 = Lc + 1, cnxe = C1 * C1 * C1;
     const int32_t *row = idx + e * nxe;
-    // NB nodes per thread at a time (coarse nodes here, fine nodes below): their ids, then their values
+    const uint8_t *ow = own + e * nxe;
+    // NB fine nodes per thread at a time: their owner flags and ids, then (adding) their keep flags
+    // and old values, each batch of loads issued together (unowned nodes read valid entries they
+    // do not use); the first batch is on its way while the coarse values are staged
     constexpr int NB = 4;
-    for (int c0 = threadIdx.x; c0 < cnxe; c0 += NB * blockDim.x) {
-        ptrdiff_t cg[NB];
+    uint8_t o[NB];
+    ptrdiff_t gg[NB];
+    unsigned km[NB];
+    T old[NB][VS];
+    auto load_ids = [&](int v0) {
 #pragma unroll
         for (int b = 0; b < NB; b++) {
+            const int v = v0 + b * blockDim.x;
+            const bool in = v < nxe;
+            o[b] = ow[in ? v : 0];
+            if (!in) o[b] = 0;
+            gg[b] = row[in ? v : 0];
+        }
+    };
+    auto load_old = [&]() {
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            km[b] = (ADD && keep) ? keep[gg[b]] : 0u;
+#pragma unroll
+            for (int d = 0; d < VS; d++) old[b][d] = ADD ? to[gg[b] * VS + d] : T(0);
+        }
+    };
+    load_ids(threadIdx.x);
+    // coarse nodes: NC per thread at a time, their ids, then their values
+    constexpr int NC = LF && LC <= 6 ? 1 : 4;
+    for (int c0 = threadIdx.x; c0 < cnxe; c0 += NC * blockDim.x) {
+        ptrdiff_t cg[NC];
+#pragma unroll
+        for (int b = 0; b < NC; b++) {
             const int c = c0 + b * blockDim.x, cc = c < cnxe ? c : 0;
             const int X = cc % C1, Y = (cc / C1) % C1, Z = cc / (C1 * C1);
             cg[b] = row[lidx(Lf, X * s, Y * s, Z * s)];
         }
-        T fv[NB][VS];
+        T fv[NC][VS];
 #pragma unroll
-        for (int b = 0; b < NB; b++)
+        for (int b = 0; b < NC; b++)
 #pragma unroll
             for (int d = 0; d < VS; d++) fv[b][d] = from[cg[b] * VS + d];
+        if (c0 == (int)threadIdx.x) load_old();
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
+        for (int b = 0; b < NC; b++) {
             const int c = c0 + b * blockDim.x;
             if (c < cnxe)
 #pragma unroll
                 for (int d = 0; d < VS; d++) tr_smem[c * VS + d] = (double)fv[b][d];
         }
     }
+    if ((int)threadIdx.x >= cnxe) load_old();
     __syncthreads();
-    const uint8_t *ow = own + e * nxe;
-    // NB fine nodes per thread at a time: their owner flags and ids, then (adding) their keep flags
-    // and old values, each batch of loads issued together (unowned nodes read valid entries they
-    // do not use)
     for (int v0 = threadIdx.x; v0 < nxe; v0 += NB * blockDim.x) {
-        uint8_t o[NB];
-        ptrdiff_t gg[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const int v = v0 + b * blockDim.x;
-            const bool in = v < nxe;
-            o[b] = in ? ow[v] : 0;
-            gg[b] = row[in ? v : 0];
-        }
-        unsigned km[NB];
-        T old[NB][VS];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            km[b] = (add && keep) ? keep[gg[b]] : 0u;
-#pragma unroll
-            for (int d = 0; d < VS; d++) old[b][d] = add ? to[gg[b] * VS + d] : T(0);
+        if (v0 != (int)threadIdx.x) {
+            load_ids(v0);
+            load_old();
         }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             if (!o[b]) continue;
             const int v = v0 + b * blockDim.x;
             const int x = v % N1, y = (v / N1) % N1, z = v / (N1 * N1);
-            int cx = x / s, cy = y / s, cz = z / s;
-            if (cx == Lc) cx--;
-            if (cy == Lc) cy--;
-            if (cz == Lc) cz--;
-            const double tx = (double)(x - cx * s) / s, ty = (double)(y - cy * s) / s, tz = (double)(z - cz * s) / s;
             double acc[VS];
+            if constexpr (LF > 0 && LF == 2 * LC) {
+                // halving: averages of the coarse nodes at and after x / 2, per direction (the same node twice on
+                // even coordinates: the average is then exact), without weights or branches
+                const double *src = tr_smem + lidx(LC, x >> 1, y >> 1, z >> 1) * VS;
+                const int dx = (x & 1) * VS, dy = (y & 1) * (LC + 1) * VS, dz = (z & 1) * (LC + 1) * (LC + 1) * VS;
 #pragma unroll
-            for (int d = 0; d < VS; d++) acc[d] = 0;
+                for (int d = 0; d < VS; d++) {
+                    const double *q = src + d;
+                    acc[d] = mean(mean(mean(q[0], q[dx]), mean(q[dy], q[dy + dx])),
+                                  mean(mean(q[dz], q[dz + dx]), mean(q[dz + dy], q[dz + dy + dx])));
+                }
+            } else {
+                int cx = x / s, cy = y / s, cz = z / s;
+                if (cx == Lc) cx--;
+                if (cy == Lc) cy--;
+                if (cz == Lc) cz--;
+                const double tx = (double)(x - cx * s) / s, ty = (double)(y - cy * s) / s, tz = (double)(z - cz * s) / s;
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const int bx = hex8_cx(k), by = hex8_cy(k), bz = hex8_cz(k);
-                const double w = (bx ? tx : 1 - tx) * (by ? ty : 1 - ty) * (bz ? tz : 1 - tz);
-                if (w == 0) continue;
-                const double *src = tr_smem + lidx(Lc, cx + bx, cy + by, cz + bz) * VS;
+                for (int d = 0; d < VS; d++) acc[d] = 0;
 #pragma unroll
-                for (int d = 0; d < VS; d++) acc[d] += w * src[d];
+                for (int k = 0; k < 8; k++) {
+                    const int bx = hex8_cx(k), by = hex8_cy(k), bz = hex8_cz(k);
+                    const double w = (bx ? tx : 1 - tx) * (by ? ty : 1 - ty) * (bz ? tz : 1 - tz);
+                    if (w == 0) continue;
+                    const double *src = tr_smem + lidx(Lc, cx + bx, cy + by, cz + bz) * VS;
+#pragma unroll
+                    for (int d = 0; d < VS; d++) acc[d] += w * src[d];
+                }
             }
             const ptrdiff_t g = gg[b];
 #pragma unroll
             for (int d = 0; d < VS; d++) {
-                if (!add)
+                if (!ADD)
                     to[g * VS + d] = (T)acc[d];
                 else if (!((km[b] >> d) & 1u))
                     to[g * VS + d] = old[b][d] + (T)acc[d];
@@ -192,8 +225,8 @@ __global__ void __launch_bounds__(256) sshex8_prolongate_lds_kernel(const ptrdif
 // the element (owned by it alone) are updated in place; coarse skeleton nodes store their
 // element contribution (scalar: node-sorted position pos[e][slot]; vector: element-major slot)
 // for the skeleton gather.  No atomics, deterministic.
-template <typename T, int VS>
-__global__ void __launch_bounds__(256) sshex8_restrict_lds_kernel(const ptrdiff_t E, const int Lf, const int Lc,
+template <typename T, int VS, int LF, int LC>
+__global__ void __launch_bounds__(1024) sshex8_restrict_lds_kernel(const ptrdiff_t E, const int Lf_, const int Lc_,
                                                                   const int32_t *__restrict__ idx,
                                                                   const uint16_t *__restrict__ count,
                                                                   const T *__restrict__ from, T *__restrict__ to,
@@ -203,6 +236,7 @@ __global__ void __launch_bounds__(256) sshex8_restrict_lds_kernel(const ptrdiff_
     extern __shared__ double tr_smem[];
     const ptrdiff_t e = blockIdx.x;
     if (e >= E) return;  // uniform per block
+    const int Lf = LF ? LF : Lf_, Lc = LF ? LC : Lc_;
     const int N1 = Lf + 1, nxe = N1 * N1 * N1, s = Lf / Lc, C1 = Lc + 1, cnxe = C1 * C1 * C1;
     const int nskc = sk_count(Lc);
     const int32_t *row = idx + e * nxe;
@@ -342,15 +376,37 @@ int sshex8_restrict(ptrdiff_t E, int Lf, int Lc, const int32_t *idx, const uint1
 
 size_t sshex8_transfer_lds_bytes(int L, int vs) { return sizeof(double) * (size_t)nxe_of(L) * vs; }
 
+// A thread per fine node up to 256; where the elements are too few to fill the GPU, up to 1,024 threads each
+// (one element of level 16, restriction: 11.5 us with 256 threads and run-time levels, 7.1 us now).  Fewer than
+// 256 for the levels below 8, whose other threads would only wait.
+static unsigned transfer_block(ptrdiff_t E, int Lf) {
+    const int want = (nxe_of(Lf) + 63) / 64 * 64, most = E < 256 ? 1024 : 256;
+    return (unsigned)(want < most ? want : most);
+}
+#define SFEM_AMD_TRANSFER_LEVELS(X) X(2, 1) X(4, 2) X(8, 4) X(16, 8) X(12, 6) X(0, 0)
+
+template <typename T, int VS, bool ADD>
+static void prolongate_lds(ptrdiff_t E, int Lf, int Lc, const int32_t *idx, const uint8_t *own, const T *from, T *to,
+                           hipStream_t s, const uint8_t *keep) {
+    const size_t lds = sshex8_transfer_lds_bytes(Lc, VS);
+    const unsigned block = transfer_block(E, Lf);
+#define CASE(F, C)                                                                                                  \
+    if (F == 0 || (Lf == F && Lc == C)) {                                                                           \
+        sshex8_prolongate_lds_kernel<T, VS, ADD, F, C><<<(unsigned)E, block, lds, s>>>(E, Lf, Lc, idx, own, from, to, keep); \
+        return;                                                                                                     \
+    }
+    SFEM_AMD_TRANSFER_LEVELS(CASE)
+#undef CASE
+}
+
 template <typename T>
 int sshex8_prolongate_lds(ptrdiff_t E, int Lf, int Lc, const int32_t *idx, const uint8_t *own, int vs, const T *from,
                           T *to, hipStream_t s, const uint8_t *keep, int add) {
     if (E == 0) return SFEM_SUCCESS;
-    const size_t lds = sshex8_transfer_lds_bytes(Lc, vs);
     if (vs == 1)
-        sshex8_prolongate_lds_kernel<T, 1><<<(unsigned)E, 256, lds, s>>>(E, Lf, Lc, idx, own, from, to, keep, add);
+        (add ? prolongate_lds<T, 1, true> : prolongate_lds<T, 1, false>)(E, Lf, Lc, idx, own, from, to, s, keep);
     else if (vs == 3)
-        sshex8_prolongate_lds_kernel<T, 3><<<(unsigned)E, 256, lds, s>>>(E, Lf, Lc, idx, own, from, to, keep, add);
+        (add ? prolongate_lds<T, 3, true> : prolongate_lds<T, 3, false>)(E, Lf, Lc, idx, own, from, to, s, keep);
     else if (!add)
         return sshex8_prolongate<T>(E, Lf, Lc, idx, own, vs, from, to, s);
     else {
@@ -361,17 +417,29 @@ int sshex8_prolongate_lds(ptrdiff_t E, int Lf, int Lc, const int32_t *idx, const
     return SFEM_SUCCESS;
 }
 
+template <typename T, int VS>
+static void restrict_lds(ptrdiff_t E, int Lf, int Lc, const int32_t *idx, const uint16_t *count, const T *from, T *to,
+                         T *part, const int32_t *cpos, hipStream_t s, int overwrite) {
+    const size_t lds = sshex8_transfer_lds_bytes(Lf, VS);
+    const unsigned block = transfer_block(E, Lf);
+#define CASE(F, C)                                                                                             \
+    if (F == 0 || (Lf == F && Lc == C)) {                                                                      \
+        sshex8_restrict_lds_kernel<T, VS, F, C><<<(unsigned)E, block, lds, s>>>(E, Lf, Lc, idx, count, from, to, part, \
+                                                                               cpos, overwrite);               \
+        return;                                                                                                \
+    }
+    SFEM_AMD_TRANSFER_LEVELS(CASE)
+#undef CASE
+}
+
 template <typename T>
 int sshex8_restrict_lds(ptrdiff_t E, int Lf, int Lc, const int32_t *idx, const uint16_t *count, int vs, const T *from,
                         T *to, T *part, const int32_t *cpos, hipStream_t s, int overwrite) {
     if (E == 0) return SFEM_SUCCESS;
-    const size_t lds = sshex8_transfer_lds_bytes(Lf, vs);
     if (vs == 1)
-        sshex8_restrict_lds_kernel<T, 1>
-                <<<(unsigned)E, 256, lds, s>>>(E, Lf, Lc, idx, count, from, to, part, cpos, overwrite);
+        restrict_lds<T, 1>(E, Lf, Lc, idx, count, from, to, part, cpos, s, overwrite);
     else if (vs == 3)
-        sshex8_restrict_lds_kernel<T, 3>
-                <<<(unsigned)E, 256, lds, s>>>(E, Lf, Lc, idx, count, from, to, part, cpos, overwrite);
+        restrict_lds<T, 3>(E, Lf, Lc, idx, count, from, to, part, cpos, s, overwrite);
     else {
         set_last_error("sshex8_restrict_lds: vector size 1 or 3");
         return SFEM_FAILURE;

@@ -514,6 +514,32 @@ def test_transfers_level16_parity(vs):
         assert relerr(host(r).astype(np.float64), ro) < tol
 
 
+# level pairs of their own kernel (one element: the widest block; 343: more than a block per CU) and others
+@pytest.mark.parametrize("Lf,Lc,n", [(4, 2, 1), (4, 2, 7), (8, 4, 1), (8, 4, 7), (12, 6, 1), (16, 8, 1), (6, 3, 2),
+                                     (8, 2, 2), (12, 4, 1), (6, 2, 1)])
+@pytest.mark.parametrize("vs", [1, 3])
+def test_transfers_by_level_pair(Lf, Lc, n, vs):
+    mel, mpts = skewed_box(n, perturb=0.02)
+    el, pts = O.sshex8_refine(Lf, mel, mpts)
+    E, nf = mel.shape[1], pts.shape[1]
+    fine = S.Mesh(S.SSHEX8, Lf, el, nf)
+    coarse = fine.derefine(Lc)
+    ec = O.derefine(Lf, Lc, el)
+    nc = coarse.nnodes
+    rng = np.random.default_rng(Lf * 31 + Lc)
+    xc, xf = rng.uniform(-1, 1, nc * vs), rng.uniform(-1, 1, nf * vs)
+    yo, ro = np.zeros(nf * vs), np.zeros(nc * vs)
+    O.lib.oracle_sshex8_prolongate(E, Lc, ec, Lf, el, vs, xc, yo)
+    O.lib.oracle_sshex8_restrict(E, Lf, el, O.incidence(el, nf), Lc, ec, vs, xf, ro)
+    for rt, dt, tol in ((S.FLOAT64, np.float64, RTOL), (S.FLOAT32, np.float32, 1e-6)):
+        y, r = zeros(nf * vs, dt), zeros(nc * vs, dt)
+        S.prolongation(coarse, fine, vs, real_type=rt).apply(dev(xc, dt), y)
+        S.restriction(fine, coarse, vs, real_type=rt).apply(dev(xf, dt), r)
+        S.synchronize()
+        assert relerr(host(y).astype(np.float64), yo) < tol
+        assert relerr(host(r).astype(np.float64), ro) < tol
+
+
 def test_constrained_operator_copies_dofs():
     L = 4
     mel, mpts = skewed_box(2)
