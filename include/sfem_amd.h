@@ -65,7 +65,8 @@ const char *sfem_amd_last_error(void);
  * summation order differs.  "hex8_patches" (default 1): tet4 and hex8 applies on meshes of at least
  * 2^15 elements run on element patches (512 or 2,048 elements grown over shared nodes, accumulated in
  * LDS, patch-boundary nodes summed in a fixed order; the partition is made by a mesh's first apply, on
- * the host); 0 runs one element per lane with atomics.
+ * the host), and the overwriting applies inside solvers on smaller hex8 meshes node by node; 0 runs one
+ * element per lane with atomics.
  * "mixed_cg" (default 1): flexible CGs created afterwards around a bridged FP32 preconditioner keep
  * z in FP32 (see sfem_amd_cg_create; the same iterates); 0 runs them through the bridge's casts. */
 int sfem_amd_set_option(const char *name, int value);

@@ -90,8 +90,11 @@ struct OpBase {
     // it can be set there, see apply_constrained); null otherwise
     virtual const sfem_amd_mesh *gather_mesh(hipStream_t) { return nullptr; }
     virtual int block_size() const { return 1; }
-    // y (+)= A x with the rows flagged in cmask (per entry of gather_mesh's skeleton, bit per
-    // component) set to x instead; overwrite: y is output only
+    // operators whose overwriting apply writes every node in one pass: Dirichlet rows as a byte per mesh node
+    // (bit per component) in apply_constrained (overwriting only), in place of gather_mesh's skeleton entries
+    virtual bool masks_nodes(hipStream_t) { return false; }
+    // y (+)= A x with the rows flagged in cmask (per entry of gather_mesh's skeleton or, with masks_nodes,
+    // per node; bit per component) set to x instead; overwrite: y is output only
     virtual int apply_constrained(const void *, void *, const uint8_t *, int, hipStream_t) {
         set_last_error("constrained gather not available for this operator");
         return SFEM_FAILURE;
@@ -147,6 +150,11 @@ struct ElementPatches {
     SkeletonStore boundary;          // the shared nodes: node (ascending), off (partial ranges)
     ptrdiff_t nparts{0};             // partial entries
 };
+// The corners of a mesh by node: node g has corners ent[off[g]] .. ent[off[g + 1] - 1], a corner being
+// element * nv + local node, elements ascending.
+struct NodeElements {
+    DevArray<int32_t> off, ent;
+};
 }  // namespace sfem_amd
 
 struct sfem_amd_op {
@@ -169,6 +177,8 @@ struct sfem_amd_mesh {
     mutable std::map<int, std::unique_ptr<sfem_amd_mesh>> sub;
     // tet4/hex8: element patches (lazy, mesh_patches and mesh_cells)
     mutable std::unique_ptr<sfem_amd::ElementPatches> patches, cells;
+    // hex8: the elements around each node (lazy, mesh_node_elements)
+    mutable std::unique_ptr<sfem_amd::NodeElements> around;
 };
 
 namespace sfem_amd {
@@ -210,5 +220,8 @@ const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t 
 const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
 const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
 bool may_build_patches(hipStream_t s);
+// The corners of a tet4/hex8 mesh by node, built by the first call outside a capture; null where they are not
+// available (the element-wise kernels run then).
+const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s);
 sfem_amd_op *wrap_op(std::shared_ptr<OpBase> o);
 }  // namespace sfem_amd

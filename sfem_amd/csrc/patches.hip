@@ -10,6 +10,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <mutex>
 #include <climits>
 #include <vector>
 
@@ -539,6 +540,49 @@ const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
     if (work()) return nullptr;
     m->patches = std::move(pt);
     return m->patches.get();
+}
+
+// Operators on one mesh may run their first applies in several threads: one of them builds.
+static std::mutex &build_mutex() {
+    static std::mutex mtx;
+    return mtx;
+}
+
+// ---------------------------------------------------------------- corners by node
+__global__ void corners_kernel(const ptrdiff_t n, const ptrdiff_t E, const int nv, const int32_t *__restrict__ idx,
+                               int32_t *__restrict__ node, int32_t *__restrict__ corner, int32_t *__restrict__ count) {
+    GRID_LOOP(i, n) {
+        const ptrdiff_t e = i / nv;
+        const int32_t g = idx[(i - e * nv) * E + e];
+        node[i] = g;
+        corner[i] = (int32_t)i;
+        atomicAdd(&count[g], 1);
+    }
+}
+const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(build_mutex());
+    if (m->around) return m->around.get();
+    if (!may_build_patches(s)) return nullptr;
+    const ptrdiff_t E = m->E, N = m->nnodes, n = E * m->nv;
+    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)n >= 2147483647.0 || N >= 2147483646) return nullptr;
+    auto ne = std::make_unique<NodeElements>();
+    auto work = [&]() -> int {
+        Scratch sc;
+        DevArray<int32_t> node, corner, snode, count;
+        if (node.alloc(n) || corner.alloc(n) || snode.alloc(n) || count.alloc(N + 1) || ne->off.alloc(N + 1) ||
+            ne->ent.alloc(n))
+            return SFEM_FAILURE;
+        LAUNCH(fill_kernel<int32_t>, N + 1, 0, count.p);
+        LAUNCH(corners_kernel, n, E, m->nv, m->idx.p, node.p, corner.p, count.p);
+        if (sc.exclusive_sum(count.p, ne->off.p, N + 1, s) ||
+            sc.sort(node.p, snode.p, corner.p, ne->ent.p, n, bits_for(N), s))
+            return SFEM_FAILURE;
+        SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
+        return SFEM_SUCCESS;
+    };
+    if (work()) return nullptr;
+    m->around = std::move(ne);
+    return m->around.get();
 }
 
 bool may_build_patches(hipStream_t s) {

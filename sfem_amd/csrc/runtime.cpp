@@ -214,6 +214,14 @@ static SkeletonMap patch_boundary(const ElementPatches &pt) {
     return sk;
 }
 
+// Small hex8 meshes: the corner lists of the node-by-node kernel (option hex8_patches covers this form too), null
+// where it does not apply.  It serves the overwriting forms, whose caller owns y (in a solver); apply keeps the
+// atomic kernel, with which several streams may add into one y.
+static const NodeElements *node_form(const sfem_amd_mesh *m, hipStream_t s) {
+    if (m->type != SFEM_AMD_HEX8 || !g_hex8_patches || m->E >= kPatchMinElements) return nullptr;
+    return mesh_node_elements(m, s);
+}
+
 // ----------------------------------------------------------------- Laplacian
 template <typename T>
 struct LaplacianOp final : OpBase {
@@ -232,13 +240,16 @@ struct LaplacianOp final : OpBase {
 
     int apply(const void *xv, void *yv, hipStream_t s) override { return apply_impl(xv, yv, s, 0); }
     int apply_overwrite(const void *xv, void *yv, hipStream_t s) override {
+        if (masks_nodes(s)) return apply_impl(xv, yv, s, 1);
         if (m->type != SFEM_AMD_SSHEX8) return OpBase::apply_overwrite(xv, yv, s);
         if (mesh_skeleton(m, 0)) return SFEM_FAILURE;
         if (!skeleton_covers(m)) return OpBase::apply_overwrite(xv, yv, s);
         return apply_impl(xv, yv, s, 1);
     }
+    bool masks_nodes(hipStream_t s) override { return std::is_same<T, double>::value && node_form(m, s) != nullptr; }
     const sfem_amd_mesh *gather_mesh(hipStream_t) override { return m->type == SFEM_AMD_SSHEX8 ? m : nullptr; }
     int apply_constrained(const void *xv, void *yv, const uint8_t *cmask, int ow, hipStream_t s) override {
+        if (ow && masks_nodes(s)) return apply_impl(xv, yv, s, 1, cmask);
         if (m->type != SFEM_AMD_SSHEX8 || mesh_skeleton(m, 0)) return SFEM_FAILURE;
         if (ow && !skeleton_covers(m)) {
             if (fill_zero(yv, (size_t)rows() * sizeof(T), s)) return SFEM_FAILURE;
@@ -255,6 +266,9 @@ struct LaplacianOp final : OpBase {
         SkeletonMap sk = skeleton_of(m);
         sk.cmask = cmask;
         if constexpr (std::is_same<T, double>::value) {
+            if (const NodeElements *ne = ow ? node_form(m, s) : nullptr)
+                return hex8_laplacian_apply_nodes(m->nnodes, m->E, ne->off.p, ne->ent.p, m->idx.p, fff32.p, coeff.p, x,
+                                                  y, cmask, s);
             if (m->type != SFEM_AMD_SSHEX8 && g_hex8_patches && m->E >= kPatchMinElements && patches_ready(s))
                 return apply_patches(x, y, s);
             switch (m->type) {
@@ -362,7 +376,9 @@ struct ElasticityOp final : OpBase {
         return Ls ? mesh_subblocks(m, Ls, s) : m;
     }
     int apply(const void *xv, void *yv, hipStream_t s) override { return apply_impl(xv, yv, s, 0); }
+    bool masks_nodes(hipStream_t s) override { return node_form(m, s) != nullptr; }
     int apply_overwrite(const void *xv, void *yv, hipStream_t s) override {
+        if (masks_nodes(s)) return apply_impl(xv, yv, s, 1);
         if (m->type != SFEM_AMD_SSHEX8) return OpBase::apply_overwrite(xv, yv, s);
         const sfem_amd_mesh *wm = work_mesh(s);
         if (!wm || mesh_skeleton(wm, 0)) return SFEM_FAILURE;
@@ -374,6 +390,7 @@ struct ElasticityOp final : OpBase {
         return m->type == SFEM_AMD_SSHEX8 ? work_mesh(s) : nullptr;
     }
     int apply_constrained(const void *xv, void *yv, const uint8_t *cmask, int ow, hipStream_t s) override {
+        if (ow && masks_nodes(s)) return apply_impl(xv, yv, s, 1, cmask);
         const sfem_amd_mesh *wm = m->type == SFEM_AMD_SSHEX8 ? work_mesh(s) : nullptr;
         if (!wm || mesh_skeleton(wm, 0)) return SFEM_FAILURE;
         if (ow && !skeleton_covers(wm)) {
@@ -403,6 +420,16 @@ struct ElasticityOp final : OpBase {
     int apply_impl(const void *xv, void *yv, hipStream_t s, int ow, const uint8_t *cmask = nullptr,
                    const ChebStep<T> *cs = nullptr) {
         if (m->type == SFEM_AMD_HEX8) {
+            if (const NodeElements *ne = ow ? node_form(m, s) : nullptr) {
+                if constexpr (std::is_same<T, double>::value)
+                    return hex8_elasticity_apply_nodes<double, float>(m->nnodes, m->E, ne->off.p, ne->ent.p, m->idx.p,
+                                                                      adj.p, det.p, mu, lambda, coeff.p,
+                                                                      (const double *)xv, (double *)yv, cmask, s);
+                else
+                    return hex8_elasticity_apply_nodes<float, uint16_t>(m->nnodes, m->E, ne->off.p, ne->ent.p, m->idx.p,
+                                                                        adj16.p, det16.p, mu, lambda, coeff.p,
+                                                                        (const float *)xv, (float *)yv, cmask, s);
+            }
             if (g_hex8_patches && m->E >= kPatchMinElements && patches_ready(s)) return apply_patches(xv, yv, s);
             if constexpr (std::is_same<T, double>::value)
                 return hex8_elasticity_apply<double, float>(m->E, m->idx.p, adj.p, det.p, mu, lambda, coeff.p,
@@ -522,33 +549,52 @@ struct ConstrainedOp final : OpBase {
     std::shared_ptr<OpBase> inner;
     DevArray<int32_t> dofs;
     // the constrained dofs as flags on the inner sshex8 operator's skeleton entries, when every
-    // one is a skeleton (macro-element boundary) dof: its gather then writes y = x there
-    DevArray<uint8_t> cmask;
-    int cmask_state{0};  // 0: not yet built, 1: in use, -1: not applicable (separate copy)
-    bool fused(hipStream_t s) {
+    // one is a skeleton (macro-element boundary) dof: its gather then writes y = x there; or as flags on the
+    // nodes of an operator that writes every node in one pass (masks_nodes)
+    DevArray<uint8_t> cmask, nmask;
+    int cmask_state{0}, nmask_state{0};  // 0: not yet built, 1: in use, -1: not applicable (separate copy)
+    // the flags for the inner operator's present form (library options may change it), null: separate copy
+    const uint8_t *mask(hipStream_t s, bool overwrite) {
+        if (inner->masks_nodes(s)) {
+            if (!overwrite) return nullptr;
+            if (nmask_state == 0 && may_build_patches(s)) nmask_state = build_nmask() ? -1 : 1;
+            return nmask_state > 0 ? nmask.p : nullptr;
+        }
         if (cmask_state == 0) {
             cmask_state = -1;
             if (!build_cmask(s)) cmask_state = 1;
             (void)hipGetLastError();
         }
-        return cmask_state > 0;
+        return cmask_state > 0 ? cmask.p : nullptr;
     }
     int build_cmask(hipStream_t s) {
         const sfem_amd_mesh *gm = inner->gather_mesh(s);
         if (!gm || mesh_skeleton(gm, 0)) return SFEM_FAILURE;
         return skeleton_dof_mask(skeleton_of(gm), inner->block_size(), dofs, cmask, s);
     }
+    int build_nmask() {
+        const int bs = inner->block_size();
+        if (bs > 8) return SFEM_FAILURE;
+        std::vector<int32_t> d(dofs.n);
+        if (!d.empty() &&
+            hipMemcpy(d.data(), dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) != hipSuccess)
+            return SFEM_FAILURE;
+        std::vector<uint8_t> k((size_t)(inner->rows() / bs), 0);
+        for (const int32_t q : d)
+            if (q >= 0 && (size_t)(q / bs) < k.size()) k[(size_t)(q / bs)] |= (uint8_t)(1u << (q % bs));
+        return nmask.upload(k.data(), k.size());
+    }
     int apply(const void *x, void *y, hipStream_t s) override {
-        if (fused(s)) return inner->apply_constrained(x, y, cmask.p, 0, s);
+        if (const uint8_t *k = mask(s, false)) return inner->apply_constrained(x, y, k, 0, s);
         if (inner->apply(x, y, s)) return SFEM_FAILURE;
         return copy_constrained(x, y, s);
     }
     int apply_overwrite(const void *x, void *y, hipStream_t s) override {
-        if (fused(s)) return inner->apply_constrained(x, y, cmask.p, 1, s);
+        if (const uint8_t *k = mask(s, true)) return inner->apply_constrained(x, y, k, 1, s);
         if (inner->apply_overwrite(x, y, s)) return SFEM_FAILURE;
         return copy_constrained(x, y, s);
     }
-    bool cheb3_fusable(hipStream_t s) override { return fused(s) && inner->cheb3_fusable(s); }
+    bool cheb3_fusable(hipStream_t s) override { return mask(s, false) && inner->cheb3_fusable(s); }
     int cheb3_step(void *x, const void *rhs, const void *dinv, void *p, double alpha, double beta, int first,
                    const uint8_t *, hipStream_t s) override {
         return inner->cheb3_step(x, rhs, dinv, p, alpha, beta, first, cmask.p, s);

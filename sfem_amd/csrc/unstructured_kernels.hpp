@@ -45,6 +45,15 @@ int hex8_elasticity_apply_patches(const PatchView &pv, const G *adjp, const G *d
 // out[k][s] = in[k][perm[s]] for k < rows, s < E
 template <typename G>
 int patch_gather_rows(int rows, ptrdiff_t E, const int32_t *perm, const G *in, G *out, hipStream_t s);
+// hex8 applies node by node (small meshes): y = A x over all N nodes, off/ent the corners by node
+// (NodeElements); mask (nullable, bit per component of each node): y = x there instead
+int hex8_laplacian_apply_nodes(ptrdiff_t N, ptrdiff_t E, const int32_t *off, const int32_t *ent, const int32_t *idx,
+                               const float *fff, const float *coeff, const double *x, double *y, const uint8_t *mask,
+                               hipStream_t s);
+template <typename T, typename G>
+int hex8_elasticity_apply_nodes(ptrdiff_t N, ptrdiff_t E, const int32_t *off, const int32_t *ent, const int32_t *idx,
+                                const G *adj, const G *det, double mu, double lambda, const float *coeff, const T *x,
+                                T *y, const uint8_t *mask, hipStream_t s);
 template <typename T, typename G>
 int hex8_elasticity_diag(ptrdiff_t E, const int32_t *idx, const G *adj, const G *det, double mu, double lambda,
                          const float *coeff, int block, T *d, hipStream_t s);

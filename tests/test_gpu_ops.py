@@ -265,6 +265,62 @@ def test_hex8_elasticity_parity(n, patches):
     assert relerr(host(d), do) < RTOL
 
 
+# One Chebyshev step on rhs = 0 moves x along A x: the overwriting, constrained apply of small hex8 meshes (node by
+# node, or element by element with the option off) against the oracle.  "random": nodes with many more than eight
+# corners, corners that share a node, nodes without any.
+@pytest.mark.parametrize("mesh", [1, 2, 7, "isolated", "random"])
+@pytest.mark.parametrize("rt,bs", [(S.FLOAT64, 1), (S.FLOAT64, 3), (S.FLOAT32, 3)])
+@pytest.mark.parametrize("patches", [1, 0])
+def test_hex8_overwriting_constrained_apply(mesh, rt, bs, patches):
+    rng = np.random.default_rng(23)
+    if isinstance(mesh, int):
+        el, pts = skewed_box(mesh, perturb=0.01)
+        N = pts.shape[1]
+        adj, det = O.hex8_adj_det(el, pts)
+        fff = O.hex8_fff(el, pts)
+    else:
+        el = _isolated(8, 37) if mesh == "isolated" else rng.integers(0, 40, (8, 50)).astype(np.int32)
+        N = el.size if mesh == "isolated" else 45
+        one_el, one_pts = skewed_box(1, perturb=0.0)
+        adj, det = O.hex8_adj_det(one_el, one_pts)
+        fff = O.hex8_fff(one_el, one_pts)
+        E = el.shape[1]
+        adj, det, fff = (np.ascontiguousarray(np.repeat(a, E, axis=0)) for a in (adj, det, fff))
+    E = el.shape[1]
+    coeff = rng.uniform(0.1, 10, E).astype(np.float32)
+    mu, lam = O.lame(1.0, 0.3)
+    x = rng.uniform(-1, 1, N * bs)
+    nodes = np.unique(rng.integers(0, N, max(1, N // 4))).astype(np.int32)
+    m = S.Mesh(S.HEX8, 1, el, N)
+    dt, comps = np.float64, [0]
+    if bs == 1:
+        op = S.laplacian(m, fff, coeff)
+    else:
+        comps = [0, 2]
+        if rt == S.FLOAT32:
+            dt, adj, det = np.float32, bf16_round(adj), bf16_round(det)
+        op = S.linear_elasticity(m, adj, det, mu, lam, coeff, real_type=rt)
+    S.set_option("hex8_patches", patches)
+    try:
+        step = S.graph_op(S.cheb3(S.constrained(op, nodes, bs, comps if bs > 1 else None), max_it=1))
+        zero, y = zeros(N * bs, dt), dev(x, dt)
+        for _ in range(4):  # eager, captured, replayed
+            x = host(y).astype(np.float64)
+            step.apply(zero, y)
+            S.synchronize()
+            d = x - host(y).astype(np.float64)
+            ao = np.zeros(N * bs)
+            if bs == 1:
+                O.lib.oracle_hex8_laplacian_apply(E, el, fff, coeff, x, ao)
+            else:
+                O.lib.oracle_hex8_elasticity_apply(E, el, adj, det, mu, lam, coeff, x, ao)
+            for c in comps:
+                ao[nodes * bs + c] = x[nodes * bs + c]
+            assert relerr(d * (ao @ d) / (d @ d), ao) < (RTOL if dt == np.float64 else 1e-5)
+    finally:
+        S.set_option("hex8_patches", 1)
+
+
 @pytest.mark.parametrize("n,patches", [(6, 1), (40, 1), (40, 0)])
 def test_hex8_elasticity_fp32_bf16_error_stated(n, patches):
     """FP32 hex8 elasticity (bf16 adjugate and determinant words, FP32 sum-factorised arithmetic):
