@@ -64,7 +64,7 @@ const char *sfem_amd_last_error(void);
  * 2 the stencil form (levels 2-6, 8, 10, 12, 16).  Both give the reference's operator; the
  * summation order differs.  "hex8_patches" (default 1): tet4 and hex8 applies on meshes of at least
  * 2^15 elements run on element patches (512 or 2,048 elements grown over shared nodes, accumulated in
- * LDS, patch-boundary nodes summed in a fixed order; the partition is made by a mesh's first apply, on
+ * LDS and added to y with atomics; the partition is made by a mesh's first apply, the elasticity's on
  * the host), and the overwriting applies inside solvers on smaller hex8 meshes node by node; 0 runs one
  * element per lane with atomics.
  * "mixed_cg" (default 1): flexible CGs created afterwards around a bridged FP32 preconditioner keep

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -134,10 +135,8 @@ struct SkeletonStore {
 };
 
 // The elements of a tet4/hex8 mesh grouped into patches of neighbouring elements (patches.hip).  A patch
-// kernel gathers the patch's nodes once into LDS, accumulates its elements there, adds the nodes that
-// belong to this patch alone straight into y, and writes the others (the patch boundary) to
-// partials in node-sorted order, which skeleton_gather sums per node in patch order.  A slot is a position
-// in the patch order of the elements.
+// kernel gathers the patch's nodes once into LDS, accumulates its elements there and adds them to y.  A slot
+// is a position in the patch order of the elements.
 struct ElementPatches {
     ptrdiff_t npatch{0};
     int maxloc{0};                   // largest node count of a patch
@@ -146,9 +145,6 @@ struct ElementPatches {
     DevArray<uint16_t> lconn;        // [nv / 4][E][4] local node of each slot's corners
     DevArray<int32_t> node_off;      // [npatch + 1] ranges of the patch node lists
     DevArray<int32_t> nodes;         // mesh node of each patch node, ascending in a patch
-    DevArray<int32_t> bslot;         // its partial position (node-sorted), -1 for a patch's own node
-    SkeletonStore boundary;          // the shared nodes: node (ascending), off (partial ranges)
-    ptrdiff_t nparts{0};             // partial entries
 };
 // The corners of a mesh by node: node g has corners ent[off[g]] .. ent[off[g + 1] - 1], a corner being
 // element * nv + local node, elements ascending.
@@ -192,14 +188,16 @@ extern bool g_atomic_skeleton;
 // (option "elasticity_form")
 extern int g_elasticity_form;
 // tet4/hex8 applies on element patches (option "hex8_patches", default on) for meshes of at
-// least kPatchMinElements elements; off: one element per lane with atomics.  The line lies where the two
-// Laplacians cross (back-to-back applies, element-wise / patches): hex8 13,824 elements 8.1 / 11.4 us,
-// 32,768 14.8 / 11.5, 262,144 94 / 17; tet4 16,464 5.6 / 7.5 us, 34,992 8.9 / 8.2, 279,936 48 / 10.
+// least kPatchMinElements elements; off: one element per lane with atomics.  Back-to-back applies, element-wise /
+// patches: hex8 Laplacian 8,000 elements 6.8 / 8.2 us, 13,824 8.1 / 7.8, 32,768 15.1 / 7.9, 262,144 94 / 11;
+// tet4 6,000 5.5 / 5.2 us, 16,464 5.7 / 4.4, 34,992 9.0 / 4.8, 279,936 48 / 6.5; FP64 hex8 elasticity 8,000
+// 10 / 13 us, 13,824 17 / 14, 32,768 33 / 15.  The line lies above the crossing (about 12,000 elements)
+// because making the patches costs the first apply about 3 ms, at 2^14 elements over 500 applies' gain.
 extern bool g_hex8_patches;
 constexpr ptrdiff_t kPatchMinElements = (ptrdiff_t)1 << 15;
 // elements per cell of mesh_cells: at least kPatchElements, then as many as leave kCellsWanted cells, at
 // most kCellHexes or kCellTets (flat around these: 1.93M hexahedra at 384, 512, 768, 1,024 elements a cell
-// 104, 103, 107, 103 us an apply with its zero fill; 2.41M tetrahedra at 1,024 to 3,072 75 to 77 us)
+// within 4% of each other; 2.41M tetrahedra at 1,024 to 3,072 within 3%)
 constexpr ptrdiff_t kCellsWanted = 1024, kCellHexes = 512, kCellTets = 2048;
 // Host-side state that a captured HIP graph depends on (library options, switch selections, CNN
 // weights) changes the state epoch; graph-replaying operators re-capture when it moved.
@@ -220,6 +218,9 @@ const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t 
 const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
 const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
 bool may_build_patches(hipStream_t s);
+// Held while lists of a mesh or words of an operator in their order are made: operators on one mesh, or
+// one operator, may run their first applies in several threads.
+std::recursive_mutex &patch_mutex();
 // The corners of a tet4/hex8 mesh by node, built by the first call outside a capture; null where they are not
 // available (the element-wise kernels run then).
 const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s);

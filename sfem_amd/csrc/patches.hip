@@ -10,7 +10,6 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
-#include <mutex>
 #include <climits>
 #include <vector>
 
@@ -106,16 +105,15 @@ __global__ void corner_keys_kernel(const ptrdiff_t n, const ptrdiff_t E, const i
 __global__ void key_heads_kernel(const ptrdiff_t n, const uint64_t *__restrict__ key, int32_t *__restrict__ head) {
     GRID_LOOP(i, n) head[i] = i == 0 || key[i] != key[i - 1];
 }
-// patch node lists and their ranges; the number of patches that use each node
+// patch node lists and their ranges
 __global__ void node_lists_kernel(const ptrdiff_t n, const int nbits, const uint64_t *__restrict__ key,
                                   const int32_t *__restrict__ incl, int32_t *__restrict__ nodes,
-                                  int32_t *__restrict__ node_off, int32_t *__restrict__ used) {
+                                  int32_t *__restrict__ node_off) {
     GRID_LOOP(i, n) {
         const uint64_t k = key[i];
         if (i == 0 || k != key[i - 1]) {
             const int32_t u = incl[i] - 1, g = (int32_t)(k & (((uint64_t)1 << nbits) - 1));
             nodes[u] = g;
-            atomicAdd(&used[g], 1);
             if (i == 0 || (k >> nbits) != (key[i - 1] >> nbits)) node_off[k >> nbits] = u;
         }
         if (i == n - 1) node_off[(k >> nbits) + 1] = incl[i];
@@ -134,35 +132,6 @@ __global__ void local_nodes_kernel(const ptrdiff_t n, const ptrdiff_t E, const i
 __global__ void list_sizes_kernel(const ptrdiff_t n, const int32_t *__restrict__ off, int32_t *__restrict__ size) {
     GRID_LOOP(i, n) size[i] = off[i + 1] - off[i];
 }
-__global__ void shared_counts_kernel(const ptrdiff_t n, const int32_t *__restrict__ used, int32_t *__restrict__ parts,
-                                     int32_t *__restrict__ flag) {
-    GRID_LOOP(g, n) {
-        parts[g] = used[g] > 1 ? used[g] : 0;
-        flag[g] = used[g] > 1;
-    }
-}
-// the shared nodes (ascending) with their partial ranges
-__global__ void shared_nodes_kernel(const ptrdiff_t n, const int32_t *__restrict__ used, const int32_t *__restrict__ parts,
-                                    const int32_t *__restrict__ rank, int32_t *__restrict__ node,
-                                    int32_t *__restrict__ off) {
-    GRID_LOOP(g, n) {
-        if (used[g] > 1) {
-            node[rank[g]] = (int32_t)g;
-            off[rank[g]] = parts[g];
-        }
-        if (g == n - 1) off[rank[g] + (used[g] > 1)] = parts[g] + (used[g] > 1 ? used[g] : 0);
-    }
-}
-// entry u of the lists, j-th in node order (patches ascending within a node) -> its partial slot
-__global__ void partial_slots_kernel(const ptrdiff_t n, const int32_t *__restrict__ sorted_node,
-                                     const int32_t *__restrict__ entry, const int32_t *__restrict__ used,
-                                     const int32_t *__restrict__ first, const int32_t *__restrict__ parts,
-                                     int32_t *__restrict__ bslot) {
-    GRID_LOOP(j, n) {
-        const int32_t g = sorted_node[j];
-        bslot[entry[j]] = used[g] > 1 ? parts[g] + ((int32_t)j - first[g]) : -1;
-    }
-}
 
 // label: element -> group (device, destroyed); groups become patches of at most cap elements
 int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label, int cap, ElementPatches &pt,
@@ -170,7 +139,7 @@ int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label
     const int nv = m->nv;
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * nv;
     Scratch sc;
-    DevArray<int32_t> a, b, head, incl, pos, spos, used;
+    DevArray<int32_t> a, b, head, incl, pos, spos;
     // elements by group, ascending ids within one (consecutive slots are consecutive elements wherever the
     // mesh allows)
     if (a.alloc(E) || b.alloc(E) || head.alloc(n) || incl.alloc(n) || pt.perm.alloc(E)) return SFEM_FAILURE;
@@ -191,7 +160,7 @@ int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label
     // patch node lists, ascending, and local numbering
     const int nbits = bits_for(N);
     DevArray<uint64_t> key, skey;
-    if (key.alloc(n) || skey.alloc(n) || pos.alloc(n) || spos.alloc(n) || used.alloc(N) || pt.lconn.alloc(n))
+    if (key.alloc(n) || skey.alloc(n) || pos.alloc(n) || spos.alloc(n) || pt.lconn.alloc(n))
         return SFEM_FAILURE;
     LAUNCH(corner_keys_kernel, n, E, nv, nbits, pt.perm.p, b.p, m->idx.p, key.p, pos.p);
     if (sc.sort(key.p, skey.p, pos.p, spos.p, n, nbits + bits_for(np), s)) return SFEM_FAILURE;
@@ -199,9 +168,8 @@ int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label
     if (sc.inclusive_sum(head.p, incl.p, n, s)) return SFEM_FAILURE;
     int32_t total = 0;
     if (fetch(incl.p + n - 1, &total, s)) return SFEM_FAILURE;
-    if (pt.nodes.alloc(total) || pt.bslot.alloc(total)) return SFEM_FAILURE;
-    LAUNCH(fill_kernel<int32_t>, N, 0, used.p);
-    LAUNCH(node_lists_kernel, n, nbits, skey.p, incl.p, pt.nodes.p, pt.node_off.p, used.p);
+    if (pt.nodes.alloc(total)) return SFEM_FAILURE;
+    LAUNCH(node_lists_kernel, n, nbits, skey.p, incl.p, pt.nodes.p, pt.node_off.p);
     LAUNCH(local_nodes_kernel, n, E, nbits, skey.p, spos.p, incl.p, pt.node_off.p, pt.lconn.p);
     LAUNCH(list_sizes_kernel, (ptrdiff_t)np, pt.node_off.p, head.p);
     if (sc.run([&](void *t, size_t &bytes) { return hipcub::DeviceReduce::Max(t, bytes, head.p, incl.p, (int)np, s); }))
@@ -213,25 +181,6 @@ int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label
         return SFEM_FAILURE;
     }
     pt.maxloc = maxloc;
-    // the nodes that several patches share, and the partial slots
-    DevArray<int32_t> parts, first, flag, rank, snode, entry;
-    if (parts.alloc(N) || first.alloc(N) || flag.alloc(N) || rank.alloc(N) || snode.alloc(total) || entry.alloc(total))
-        return SFEM_FAILURE;
-    LAUNCH(shared_counts_kernel, N, used.p, parts.p, flag.p);
-    if (sc.exclusive_sum(used.p, first.p, N, s) || sc.exclusive_sum(flag.p, rank.p, N, s)) return SFEM_FAILURE;
-    int32_t last[2];
-    if (fetch(rank.p + N - 1, &last[0], s) || fetch(flag.p + N - 1, &last[1], s)) return SFEM_FAILURE;
-    const ptrdiff_t nb = (ptrdiff_t)last[0] + last[1];
-    if (sc.exclusive_sum(parts.p, flag.p, N, s)) return SFEM_FAILURE;  // flag: partial offsets from here on
-    if (pt.boundary.node.alloc(nb) || pt.boundary.off.alloc(nb + 1)) return SFEM_FAILURE;
-    pt.boundary.n = nb;
-    LAUNCH(shared_nodes_kernel, N, used.p, flag.p, rank.p, pt.boundary.node.p, pt.boundary.off.p);
-    int32_t nparts = 0;
-    if (fetch(pt.boundary.off.p + nb, &nparts, s)) return SFEM_FAILURE;
-    pt.nparts = nparts;
-    LAUNCH(iota_kernel, (ptrdiff_t)total, pos.p);
-    if (sc.sort(pt.nodes.p, snode.p, pos.p, entry.p, total, nbits, s)) return SFEM_FAILURE;
-    LAUNCH(partial_slots_kernel, (ptrdiff_t)total, snode.p, entry.p, used.p, first.p, flag.p, pt.bslot.p);
     SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
     return SFEM_SUCCESS;
 }
@@ -542,12 +491,6 @@ const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
     return m->patches.get();
 }
 
-// Operators on one mesh may run their first applies in several threads: one of them builds.
-static std::mutex &build_mutex() {
-    static std::mutex mtx;
-    return mtx;
-}
-
 // ---------------------------------------------------------------- corners by node
 __global__ void corners_kernel(const ptrdiff_t n, const ptrdiff_t E, const int nv, const int32_t *__restrict__ idx,
                                int32_t *__restrict__ node, int32_t *__restrict__ corner, int32_t *__restrict__ count) {
@@ -560,7 +503,7 @@ __global__ void corners_kernel(const ptrdiff_t n, const ptrdiff_t E, const int n
     }
 }
 const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
-    std::lock_guard<std::mutex> lock(build_mutex());
+    std::lock_guard<std::recursive_mutex> lock(patch_mutex());
     if (m->around) return m->around.get();
     if (!may_build_patches(s)) return nullptr;
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * m->nv;
@@ -583,6 +526,11 @@ const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
     if (work()) return nullptr;
     m->around = std::move(ne);
     return m->around.get();
+}
+
+std::recursive_mutex &patch_mutex() {
+    static std::recursive_mutex m;
+    return m;
 }
 
 bool may_build_patches(hipStream_t s) {

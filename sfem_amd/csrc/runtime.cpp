@@ -202,16 +202,8 @@ static PatchView patch_view(const ElementPatches &pt, ptrdiff_t E) {
     pv.start = pt.start.p;
     pv.node_off = pt.node_off.p;
     pv.nodes = pt.nodes.p;
-    pv.bslot = pt.bslot.p;
     pv.lconn = pt.lconn.p;
     return pv;
-}
-static SkeletonMap patch_boundary(const ElementPatches &pt) {
-    SkeletonMap sk{};
-    sk.node = pt.boundary.node.p;
-    sk.off = pt.boundary.off.p;
-    sk.n = pt.boundary.n;
-    return sk;
 }
 
 // Small hex8 meshes: the corner lists of the node-by-node kernel (option hex8_patches covers this form too), null
@@ -231,9 +223,8 @@ struct LaplacianOp final : OpBase {
     DevArray<float> coeff;
     DevArray<T> part;  // sshex8: skeleton contributions [E][sk_count(L)]
     DevArray<double> Kem;  // sshex8 stored sub-element matrices [E][64] (instead of the FFF)
-    // tet4/hex8 on element patches: the words in patch-slot order, shared-node partials
+    // tet4/hex8 on element patches: the words in patch-slot order
     DevArray<float> fffp, coeffp;
-    DevArray<double> ppart;
     int patch_state{0};  // 0 not yet tried, 1 ready, -1 not applicable
     int real_type() const override { return std::is_same<T, double>::value ? SFEM_AMD_FLOAT64 : SFEM_AMD_FLOAT32; }
     ptrdiff_t rows() const override { return m->nnodes; }
@@ -287,12 +278,13 @@ struct LaplacianOp final : OpBase {
     }
     // tet4/hex8: the element patches of the mesh and this operator's words in their slot order (first use)
     bool patches_ready(hipStream_t s) {
+        std::lock_guard<std::recursive_mutex> lock(patch_mutex());
         if (patch_state) return patch_state > 0;
         if (!may_build_patches(s)) return false;
         patch_state = -1;
         const ElementPatches *pt = mesh_cells(m, s);
         if (!pt || patch_lds_bytes(pt->maxloc, 1, sizeof(double)) > kPatchLdsLimit) return false;
-        bool ok = !ppart.alloc((size_t)pt->nparts + 1) && !fffp.alloc((size_t)6 * m->E) &&
+        bool ok = !fffp.alloc((size_t)6 * m->E) &&
                   !patch_gather_rows<float>(6, m->E, pt->perm.p, fff32.p, fffp.p, s);
         if (ok && coeff.p)
             ok = !coeffp.alloc(m->E) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
@@ -302,8 +294,7 @@ struct LaplacianOp final : OpBase {
     }
     int apply_patches(const T *x, T *y, hipStream_t s) {
         const ElementPatches *pt = m->cells.get();
-        if (laplacian_apply_patches(m->nv, patch_view(*pt, m->E), fffp.p, coeffp.p, x, y, ppart.p, s)) return SFEM_FAILURE;
-        return skeleton_gather<T>(patch_boundary(*pt), 1, ppart.p, y, s, 0, 1);
+        return laplacian_apply_patches(m->nv, patch_view(*pt, m->E), fffp.p, coeffp.p, x, y, s);
     }
     int diag(void *dv, hipStream_t s) override {
         T *d = (T *)dv;
@@ -330,10 +321,9 @@ struct ElasticityOp final : OpBase {
     const sfem_amd_mesh *m{nullptr};
     DevArray<float> adj, det, coeff;  // hex8: SoA [9][E], [E]
     DevArray<uint16_t> adj16, det16;  // hex8, FP32 operator: the same words rounded to bf16
-    // hex8 on element patches: geometry and coefficient words in patch-slot order, shared-node partials
+    // hex8 on element patches: geometry and coefficient words in patch-slot order
     DevArray<float> adjp, detp, coeffp;
     DevArray<uint16_t> adjp16, detp16;
-    DevArray<T> ppart;
     int patch_state{0};  // 0 not yet tried, 1 ready, -1 not applicable
     DevArray<double> K;               // sshex8: per-macro 24x24 matrices
     DevArray<float> K32;              // sshex8, FP32 operator: K rounded to float
@@ -472,19 +462,20 @@ struct ElasticityOp final : OpBase {
     }
     // hex8: the element patches of the mesh and this operator's words in their slot order (first use)
     bool patches_ready(hipStream_t s) {
+        std::lock_guard<std::recursive_mutex> lock(patch_mutex());
         if (patch_state) return patch_state > 0;
         if (!may_build_patches(s)) return false;
         patch_state = -1;
         const ElementPatches *pt = mesh_patches(m, s);
         if (!pt || patch_lds_bytes(pt->maxloc, 3, sizeof(T)) > kPatchLdsLimit) return false;
         const ptrdiff_t Ep = m->E;
-        bool ok = ppart.alloc((size_t)pt->nparts * 3 + 3) == SFEM_SUCCESS;
+        bool ok;
         if constexpr (std::is_same<T, double>::value)
-            ok = ok && !adjp.alloc((size_t)9 * Ep) && !detp.alloc(Ep) &&
+            ok = !adjp.alloc((size_t)9 * Ep) && !detp.alloc(Ep) &&
                  !patch_gather_rows<float>(9, m->E, pt->perm.p, adj.p, adjp.p, s) &&
                  !patch_gather_rows<float>(1, m->E, pt->perm.p, det.p, detp.p, s);
         else
-            ok = ok && !adjp16.alloc((size_t)9 * Ep) && !detp16.alloc(Ep) &&
+            ok = !adjp16.alloc((size_t)9 * Ep) && !detp16.alloc(Ep) &&
                  !patch_gather_rows<uint16_t>(9, m->E, pt->perm.p, adj16.p, adjp16.p, s) &&
                  !patch_gather_rows<uint16_t>(1, m->E, pt->perm.p, det16.p, detp16.p, s);
         if (ok && coeff.p)
@@ -496,15 +487,12 @@ struct ElasticityOp final : OpBase {
     int apply_patches(const void *xv, void *yv, hipStream_t s) {
         const ElementPatches *pt = m->patches.get();
         const PatchView pv = patch_view(*pt, m->E);
-        int err;
         if constexpr (std::is_same<T, double>::value)
-            err = hex8_elasticity_apply_patches<double, float>(pv, adjp.p, detp.p, coeffp.p, mu, lambda,
-                                                               (const double *)xv, (double *)yv, ppart.p, s);
+            return hex8_elasticity_apply_patches<double, float>(pv, adjp.p, detp.p, coeffp.p, mu, lambda,
+                                                                (const double *)xv, (double *)yv, s);
         else
-            err = hex8_elasticity_apply_patches<float, uint16_t>(pv, adjp16.p, detp16.p, coeffp.p, mu, lambda,
-                                                                 (const float *)xv, (float *)yv, ppart.p, s);
-        if (err) return err;
-        return skeleton_gather<T>(patch_boundary(*pt), 3, ppart.p, (T *)yv, s, 0, 1);
+            return hex8_elasticity_apply_patches<float, uint16_t>(pv, adjp16.p, detp16.p, coeffp.p, mu, lambda,
+                                                                  (const float *)xv, (float *)yv, s);
     }
     int hex8_diag(int block, void *d, hipStream_t s) {
         if constexpr (std::is_same<T, double>::value)

@@ -270,14 +270,18 @@ __global__ void __launch_bounds__(256)
 }
 
 // Patch-wise (ElementPatches): one workgroup per patch.  The patch's nodes
-// are gathered into LDS once (x), the elements accumulate into LDS (y, LDS atomics), then each patch
-// node is either added to y (the patch's own nodes: no other workgroup touches them) or written to
-// its node-sorted partial slot (nodes shared with other patches; summed by skeleton_gather).  The
+// are gathered into LDS once (x), the elements accumulate into LDS (y, LDS atomics), then every patch
+// node is added to y with a global atomic, consecutive lanes on consecutive entries of y: nodes that
+// several patches share need no further pass.  (Shared nodes written to partials instead, summed by a
+// gather kernel, the others added without atomics: 73 against 52 us at 1.93M hexahedra, Laplacian; 176
+// against 133 us at 2.10M, FP64 elasticity (FP32 103 against 85), where a lane per node with its three components apart
+// takes 244 us.)  It also lets several streams apply one operator, or add into one y.  The
 // geometry and coefficient words are stored in patch-slot order, so every read of them coalesces.
 // The LDS accumulator is FP64 for both value types: ds_add_f64 keeps pace with the arithmetic, while
 // ds_add_f32 measured 7x the LDS busy cycles and 100x the LDS wait of the whole FP64 kernel here.
 
-// patch nodes per thread at a time: their ids, then their values, each batch issued together
+// patch nodes per thread at a time: their ids, then their values, each batch issued together (an entry per
+// thread as in patch_add_y: 155 us an elasticity apply)
 constexpr int kPatchBatch = 4;
 template <typename T, int VS>
 __device__ __forceinline__ void patch_gather_x(const int nloc, const int32_t *__restrict__ nodes,
@@ -306,37 +310,22 @@ __device__ __forceinline__ void patch_gather_x(const int nloc, const int32_t *__
         }
     }
 }
-// the same batches: ids and boundary slots, then the old y (read for every node of the batch: a
-// valid entry, used for the patch's own nodes), then the stores
+// entries (node, component) per thread at a time
 template <typename T, int VS>
-__device__ __forceinline__ void patch_scatter_y(const int nloc, const int32_t *__restrict__ nodes,
-                                                const int32_t *__restrict__ bslot, const double *__restrict__ sy,
-                                                T *__restrict__ y, T *__restrict__ part) {
-    for (int i0 = threadIdx.x; i0 < nloc; i0 += kPatchBatch * blockDim.x) {
-        ptrdiff_t gg[kPatchBatch], bb[kPatchBatch];
+__device__ __forceinline__ void patch_add_y(const int nloc, const int32_t *__restrict__ nodes,
+                                            const double *__restrict__ sy, T *__restrict__ y) {
+    const int n = nloc * VS;
+    for (int i0 = threadIdx.x; i0 < n; i0 += kPatchBatch * blockDim.x) {
+        ptrdiff_t gg[kPatchBatch];
 #pragma unroll
         for (int b = 0; b < kPatchBatch; b++) {
-            const int i = i0 + b * blockDim.x, ii = i < nloc ? i : 0;
-            gg[b] = nodes[ii];
-            bb[b] = bslot[ii];
+            const int i = i0 + b * blockDim.x < n ? i0 + b * blockDim.x : 0, node = i / VS;
+            gg[b] = (ptrdiff_t)nodes[node] * VS + (i - node * VS);
         }
-        T yo[kPatchBatch][VS];
-#pragma unroll
-        for (int b = 0; b < kPatchBatch; b++)
-#pragma unroll
-            for (int c = 0; c < VS; c++) yo[b][c] = y[gg[b] * VS + c];
 #pragma unroll
         for (int b = 0; b < kPatchBatch; b++) {
             const int i = i0 + b * blockDim.x;
-            if (i >= nloc) continue;
-#pragma unroll
-            for (int c = 0; c < VS; c++) {
-                const T v = (T)sy[i * VS + c];
-                if (bb[b] < 0)
-                    y[gg[b] * VS + c] = yo[b][c] + v;
-                else
-                    part[bb[b] * VS + c] = v;
-            }
+            if (i < n) atomicAdd(&y[gg[b]], (T)sy[i]);
         }
     }
 }
@@ -355,7 +344,7 @@ template <typename T, typename G>
 __global__ void __launch_bounds__(256)
     hex8_elasticity_patch_kernel(const PatchView pv, const G *__restrict__ adjp, const G *__restrict__ detp,
                                  const float *__restrict__ coeffp, const double mu0, const double lambda0,
-                                 const T *__restrict__ x, T *__restrict__ y, T *__restrict__ part) {
+                                 const T *__restrict__ x, T *__restrict__ y) {
     extern __shared__ __align__(16) unsigned char patch_lds[];
     const ptrdiff_t p = xcd_contiguous_block(blockIdx.x, gridDim.x);
     const int off = pv.node_off[p], nloc = pv.node_off[p + 1] - off;
@@ -377,7 +366,7 @@ __global__ void __launch_bounds__(256)
             [&](int n, int d, T val) { atomicAdd(&sy[l[n] * 3 + d], (double)val); });
     }
     __syncthreads();
-    patch_scatter_y<T, 3>(nloc, pv.nodes + off, pv.bslot + off, sy, y, part);
+    patch_add_y<T, 3>(nloc, pv.nodes + off, sy, y);
 }
 
 // hex8 Laplacian of one element, sum-factorised as the elasticity element above.  The x-derivative at
@@ -418,13 +407,12 @@ __device__ __forceinline__ void hex8_laplacian_sf_element(const double f[6], Loa
 
 // The Laplacian over patches.  The element-wise kernels are bound by their global FP64 atomics (4 or 8
 // per element), scattered meshes also by the gathers of x; here both stay in LDS.  What bounds this one:
-// latency (two dependent loads before the sweep, two after it) and the ds_add_f64 of the sweep.
-// 1.93M hexahedra: 54 us and 10 us of gather (696 us element-wise); 2.41M shuffled tetrahedra: 36 and 5 us
-// (417 us).
+// latency (two dependent loads before the sweep, one after it) and the ds_add_f64 of the sweep.
+// 1.93M hexahedra: 47 us (696 us element-wise); 2.41M shuffled tetrahedra: 41 us (417 us).
 template <int NV>
 __global__ void __launch_bounds__(256)
     laplacian_patch_kernel(const PatchView pv, const float *__restrict__ fffp, const float *__restrict__ coeffp,
-                           const double *__restrict__ x, double *__restrict__ y, double *__restrict__ part) {
+                           const double *__restrict__ x, double *__restrict__ y) {
     extern __shared__ __align__(16) unsigned char patch_lds[];
     const ptrdiff_t p = xcd_contiguous_block(blockIdx.x, gridDim.x);
     const int off = pv.node_off[p], nloc = pv.node_off[p + 1] - off;
@@ -476,7 +464,7 @@ __global__ void __launch_bounds__(256)
         }
     }
     __syncthreads();
-    patch_scatter_y<double, 1>(nloc, pv.nodes + off, pv.bslot + off, sy, y, part);
+    patch_add_y<double, 1>(nloc, pv.nodes + off, sy, y);
 }
 
 // Node by node, for the small hex8 meshes inside a multigrid hierarchy (below kPatchMinElements), whose
@@ -764,20 +752,19 @@ int hex8_elasticity_diag(ptrdiff_t E, const int32_t *idx, const G *adj, const G 
 }
 template <typename T, typename G>
 int hex8_elasticity_apply_patches(const PatchView &pv, const G *adjp, const G *detp, const float *coeffp, double mu,
-                                  double lambda, const T *x, T *y, T *part, hipStream_t s) {
+                                  double lambda, const T *x, T *y, hipStream_t s) {
     if (pv.npatch == 0) return SFEM_SUCCESS;
     const size_t lds = patch_lds_bytes(pv.maxloc, 3, sizeof(T));
     if (lds > kPatchLdsLimit) {
         set_last_error("hex8 elasticity patches: patch node count exceeds the LDS budget");
         return SFEM_FAILURE;
     }
-    hex8_elasticity_patch_kernel<T, G><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, adjp, detp, coeffp, mu, lambda, x, y,
-                                                                             part);
+    hex8_elasticity_patch_kernel<T, G><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, adjp, detp, coeffp, mu, lambda, x, y);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }
 int laplacian_apply_patches(int nv, const PatchView &pv, const float *fffp, const float *coeffp, const double *x,
-                            double *y, double *part, hipStream_t s) {
+                            double *y, hipStream_t s) {
     if (pv.npatch == 0) return SFEM_SUCCESS;
     const size_t lds = patch_lds_bytes(pv.maxloc, 1, sizeof(double));
     if (lds > kPatchLdsLimit || (nv != 4 && nv != 8)) {
@@ -785,9 +772,9 @@ int laplacian_apply_patches(int nv, const PatchView &pv, const float *fffp, cons
         return SFEM_FAILURE;
     }
     if (nv == 8)
-        laplacian_patch_kernel<8><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, fffp, coeffp, x, y, part);
+        laplacian_patch_kernel<8><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, fffp, coeffp, x, y);
     else
-        laplacian_patch_kernel<4><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, fffp, coeffp, x, y, part);
+        laplacian_patch_kernel<4><<<(unsigned)pv.npatch, 256, lds, s>>>(pv, fffp, coeffp, x, y);
     SFEM_AMD_HIP_CHECK(hipGetLastError());
     return SFEM_SUCCESS;
 }
@@ -800,10 +787,10 @@ int patch_gather_rows(int rows, ptrdiff_t E, const int32_t *perm, const G *in, G
 }
 template int hex8_elasticity_apply_patches<double, float>(const PatchView &, const float *, const float *,
                                                           const float *, double, double, const double *, double *,
-                                                          double *, hipStream_t);
+                                                          hipStream_t);
 template int hex8_elasticity_apply_patches<float, uint16_t>(const PatchView &, const uint16_t *, const uint16_t *,
                                                             const float *, double, double, const float *, float *,
-                                                            float *, hipStream_t);
+                                                            hipStream_t);
 template int patch_gather_rows<float>(int, ptrdiff_t, const int32_t *, const float *, float *, hipStream_t);
 template int patch_gather_rows<uint16_t>(int, ptrdiff_t, const int32_t *, const uint16_t *, uint16_t *, hipStream_t);
 // FP64 operator on float32 geometry words; FP32 operator on bf16 words

@@ -29,19 +29,17 @@ inline size_t patch_lds_bytes(int maxloc, int vs, size_t value_bytes) {
 struct PatchView {
     ptrdiff_t npatch{0}, E{0};
     int maxloc{0};
-    const int32_t *start{nullptr}, *node_off{nullptr}, *nodes{nullptr}, *bslot{nullptr};
+    const int32_t *start{nullptr}, *node_off{nullptr}, *nodes{nullptr};
     const uint16_t *lconn{nullptr};
 };
 // The Laplacian over the patches (nv 4: tet4, 8: hex8; fffp [6][E], coeffp [E] or null in patch-slot
 // order), as hex8_elasticity_apply_patches below.
 int laplacian_apply_patches(int nv, const PatchView &pv, const float *fffp, const float *coeffp, const double *x,
-                            double *y, double *part, hipStream_t s);
-// y += A x over the patches: the patches' own nodes are added to y, the shared ones written to part
-// (node-sorted partial slots, 3 values each) for skeleton_gather.  adjp [9][E], detp and coeffp
-// [E] in patch-slot order (patch_gather_rows).
+                            double *y, hipStream_t s);
+// y += A x over the patches.  adjp [9][E], detp and coeffp [E] in patch-slot order (patch_gather_rows).
 template <typename T, typename G>
 int hex8_elasticity_apply_patches(const PatchView &pv, const G *adjp, const G *detp, const float *coeffp, double mu,
-                                  double lambda, const T *x, T *y, T *part, hipStream_t s);
+                                  double lambda, const T *x, T *y, hipStream_t s);
 // out[k][s] = in[k][perm[s]] for k < rows, s < E
 template <typename G>
 int patch_gather_rows(int rows, ptrdiff_t E, const int32_t *perm, const G *in, G *out, hipStream_t s);

@@ -265,6 +265,52 @@ def test_hex8_elasticity_parity(n, patches):
     assert relerr(host(d), do) < RTOL
 
 
+@pytest.mark.parametrize("kind", ["tet4", "hex8", "elasticity"])
+def test_one_operator_in_two_threads(kind):
+    """First applies of one operator on element patches in two threads, then both adding into one y."""
+    import threading
+
+    n = 19 if kind == "tet4" else 33
+    el, pts = skewed_box(n, tet4=kind == "tet4", perturb=0.02 * 6 / n)
+    E, N = el.shape[1], pts.shape[1] * (3 if kind == "elasticity" else 1)
+    assert E >= 1 << 15
+    m = S.Mesh(S.TET4 if kind == "tet4" else S.HEX8, 1, el, pts.shape[1])
+    rng = np.random.default_rng(5)
+    xs, yo = [rng.uniform(-1, 1, N) for _ in range(2)], [np.zeros(N), np.zeros(N)]
+    if kind == "elasticity":
+        adj, det = O.hex8_adj_det(el, pts)
+        mu, lam = O.lame(1.0, 0.3)
+        op = S.linear_elasticity(m, adj, det, mu, lam)
+        for x, y in zip(xs, yo):
+            O.lib.oracle_hex8_elasticity_apply(E, el, adj, det, mu, lam, None, x, y)
+    else:
+        fff = O.tet4_fff(el, pts) if kind == "tet4" else O.hex8_fff(el, pts)
+        op = S.laplacian(m, fff)
+        for x, y in zip(xs, yo):
+            if kind == "tet4":
+                O.lib.oracle_tet4_laplacian_apply(E, el, fff, x, y)
+            else:
+                O.lib.oracle_hex8_laplacian_apply(E, el, fff, None, x, y)
+    xd, yd, both, failed = [dev(x) for x in xs], [zeros(N), zeros(N)], zeros(N), []
+
+    def run(i):
+        try:
+            for y in (yd[i], both):
+                op.apply(xd[i], y)
+            S.synchronize()
+        except Exception as e:  # seen by the test's thread below
+            failed.append(e)
+
+    ts = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not failed
+    assert relerr(host(yd[0]), yo[0]) < RTOL and relerr(host(yd[1]), yo[1]) < RTOL
+    assert relerr(host(both), yo[0] + yo[1]) < RTOL
+
+
 # One Chebyshev step on rhs = 0 moves x along A x: the overwriting, constrained apply of small hex8 meshes (node by
 # node, or element by element with the option off) against the oracle.  "random": nodes with many more than eight
 # corners, corners that share a node, nodes without any.
