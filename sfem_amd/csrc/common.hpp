@@ -270,7 +270,8 @@ inline unsigned grid_for(ptrdiff_t n, int block = kBlock, unsigned cap = 1u << 2
 }
 
 
-// Dynamic LDS above the default 64 KB needs the function attribute, once per function and device.
+// Dynamic LDS above the default 64 KB needs the function attribute, once per function and device: what the
+// function's static LDS leaves of a CU's 160 KB (asking for more is refused).
 template <auto Fn>
 static int raise_lds_limit(size_t bytes) {
     static std::atomic<uint64_t> done{0};
@@ -279,8 +280,10 @@ static int raise_lds_limit(size_t bytes) {
     SFEM_AMD_HIP_CHECK(hipGetDevice(&dev));
     const uint64_t bit = 1ull << (dev & 63);
     if (done.load(std::memory_order_acquire) & bit) return SFEM_SUCCESS;
-    SFEM_AMD_HIP_CHECK(
-        hipFuncSetAttribute((const void *)Fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    hipFuncAttributes a{};
+    SFEM_AMD_HIP_CHECK(hipFuncGetAttributes(&a, (const void *)Fn));
+    SFEM_AMD_HIP_CHECK(hipFuncSetAttribute((const void *)Fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           160 * 1024 - (int)a.sharedSizeBytes));
     done.fetch_or(bit, std::memory_order_acq_rel);
     return SFEM_SUCCESS;
 }

@@ -104,6 +104,32 @@ def test_cnn_fp32_convolutions_match_oracle(L, E, hidden, layers, channels):
     assert loss2 == loss and np.array_equal(g, g2)
 
 
+@pytest.mark.parametrize("L,channels", [(8, 1), (8, 3), (7, 3)])
+def test_cnn_fp32_batch_matches_its_parts(L, channels):
+    """A batch that takes a block per element, with the largest stages in LDS, against the same elements in
+    batches small enough for several blocks per element (held against the oracle above).  The loss is
+    sum (o - t)^2 / sum t^2, so the parts' losses and gradients add up weighted by their sum t^2."""
+    E, n = 260, (L + 1) ** 3
+    flat = np.concatenate([w.ravel() for w in LS.init_weights(16, 4, 21, channels=channels)]).astype(np.float32)
+    rng = np.random.default_rng(29)
+    z, t = (rng.normal(size=(E, channels, n)).astype(np.float32) for _ in range(2))
+    cnn = S.CNN(16, 4, flat, channels=channels)
+    out = S.DeviceArray(z.size, np.float32)
+    cnn.forward(L, dev(z), out, mode=0)
+    loss, g = cnn.loss_grad(L, dev(z), dev(t))
+    o, lp, gp = np.zeros_like(z), 0.0, np.zeros(g.size)
+    for a in range(0, E, 52):
+        part = S.DeviceArray(z[a:a + 52].size, np.float32)
+        cnn.forward(L, dev(z[a:a + 52]), part, mode=0)
+        o[a:a + 52] = part.numpy().reshape(-1, channels, n)
+        lb, gb = cnn.loss_grad(L, dev(z[a:a + 52]), dev(t[a:a + 52]))
+        w = np.sum(t[a:a + 52].astype(np.float64) ** 2) / np.sum(t.astype(np.float64) ** 2)
+        lp, gp = lp + w * lb, gp + w * gb.astype(np.float64)
+    assert rel(out.numpy().reshape(z.shape), o) < 1e-5
+    assert abs(loss - lp) / lp < 1e-5
+    assert rel(g, gp) < 1e-4
+
+
 def test_cnn_zero_target_is_refused_and_keeps_the_gradient():
     """A target of norm zero is an error, and an Adam step after it still uses the last gradient."""
     L, E = 2, 2
