@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -175,6 +176,8 @@ struct sfem_amd_mesh {
     mutable std::unique_ptr<sfem_amd::ElementPatches> patches, cells;
     // hex8: the elements around each node (lazy, mesh_node_elements)
     mutable std::unique_ptr<sfem_amd::NodeElements> around;
+    mutable std::atomic<const sfem_amd::NodeElements *> around_ready{nullptr};
+    mutable std::mutex lists;  // held while patches, cells or around are made
 };
 
 namespace sfem_amd {
@@ -218,9 +221,26 @@ const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t 
 const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
 const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
 bool may_build_patches(hipStream_t s);
-// Held while lists of a mesh or words of an operator in their order are made: operators on one mesh, or
-// one operator, may run their first applies in several threads.
-std::recursive_mutex &patch_mutex();
+// Something an operator makes at its first use, once, whichever of several threads comes first.  Once made it
+// costs an apply one atomic load: no lock is taken, and what another operator or mesh is making is not waited for.
+// While the stream is being captured nothing is made and no lock is taken either.
+struct LazyPart {
+    // make() is 1 (in use) or -1 (not applicable)
+    template <typename Make>
+    bool ready(hipStream_t s, Make make) {
+        int st = state.load(std::memory_order_acquire);
+        if (st) return st > 0;
+        if (!may_build_patches(s)) return false;
+        std::lock_guard<std::mutex> lock(making);
+        st = state.load(std::memory_order_relaxed);
+        if (!st) state.store(st = make(), std::memory_order_release);
+        return st > 0;
+    }
+
+private:
+    std::atomic<int> state{0};
+    std::mutex making;
+};
 // The corners of a tet4/hex8 mesh by node, built by the first call outside a capture; null where they are not
 // available (the element-wise kernels run then).
 const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s);

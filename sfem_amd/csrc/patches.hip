@@ -312,6 +312,7 @@ __global__ void reseed_kernel(const ptrdiff_t K, const unsigned long long *__res
 // (1.55 for the ordered growth of mesh_patches); sizes spread by a factor of about two around the mean, and
 // cells above 2.5 times the mean are cut.
 const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(m->lists);
     if (m->cells) return m->cells.get();
     const ptrdiff_t E = m->E, N = m->nnodes;
     const int nv = m->nv;
@@ -409,6 +410,7 @@ __global__ void element_major_keys_kernel(const ptrdiff_t n, const ptrdiff_t E, 
 // element, against 1.42 for a perfect 8^3 cube and 8 for no sharing).  A node whose elements have all
 // been assigned is never looked at again, which leaves about one visit per (node, element) pair.
 const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(m->lists);
     if (m->patches) return m->patches.get();
     const int nv = m->nv;
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * nv;
@@ -503,9 +505,10 @@ __global__ void corners_kernel(const ptrdiff_t n, const ptrdiff_t E, const int n
     }
 }
 const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
-    std::lock_guard<std::recursive_mutex> lock(patch_mutex());
-    if (m->around) return m->around.get();
+    if (const NodeElements *ne = m->around_ready.load(std::memory_order_acquire)) return ne;
     if (!may_build_patches(s)) return nullptr;
+    std::lock_guard<std::mutex> lock(m->lists);
+    if (m->around) return m->around.get();
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * m->nv;
     if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)n >= 2147483647.0 || N >= 2147483646) return nullptr;
     auto ne = std::make_unique<NodeElements>();
@@ -525,12 +528,8 @@ const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
     };
     if (work()) return nullptr;
     m->around = std::move(ne);
+    m->around_ready.store(m->around.get(), std::memory_order_release);
     return m->around.get();
-}
-
-std::recursive_mutex &patch_mutex() {
-    static std::recursive_mutex m;
-    return m;
 }
 
 bool may_build_patches(hipStream_t s) {

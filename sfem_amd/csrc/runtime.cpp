@@ -225,7 +225,7 @@ struct LaplacianOp final : OpBase {
     DevArray<double> Kem;  // sshex8 stored sub-element matrices [E][64] (instead of the FFF)
     // tet4/hex8 on element patches: the words in patch-slot order
     DevArray<float> fffp, coeffp;
-    int patch_state{0};  // 0 not yet tried, 1 ready, -1 not applicable
+    LazyPart patch_words;
     int real_type() const override { return std::is_same<T, double>::value ? SFEM_AMD_FLOAT64 : SFEM_AMD_FLOAT32; }
     ptrdiff_t rows() const override { return m->nnodes; }
 
@@ -278,19 +278,16 @@ struct LaplacianOp final : OpBase {
     }
     // tet4/hex8: the element patches of the mesh and this operator's words in their slot order (first use)
     bool patches_ready(hipStream_t s) {
-        std::lock_guard<std::recursive_mutex> lock(patch_mutex());
-        if (patch_state) return patch_state > 0;
-        if (!may_build_patches(s)) return false;
-        patch_state = -1;
+        return patch_words.ready(s, [&] { return make_patch_words(s); });
+    }
+    int make_patch_words(hipStream_t s) {
         const ElementPatches *pt = mesh_cells(m, s);
-        if (!pt || patch_lds_bytes(pt->maxloc, 1, sizeof(double)) > kPatchLdsLimit) return false;
+        if (!pt || patch_lds_bytes(pt->maxloc, 1, sizeof(double)) > kPatchLdsLimit) return -1;
         bool ok = !fffp.alloc((size_t)6 * m->E) &&
                   !patch_gather_rows<float>(6, m->E, pt->perm.p, fff32.p, fffp.p, s);
         if (ok && coeff.p)
             ok = !coeffp.alloc(m->E) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
-        if (!ok || hipStreamSynchronize(s) != hipSuccess) return false;
-        patch_state = 1;
-        return true;
+        return !ok || hipStreamSynchronize(s) != hipSuccess ? -1 : 1;
     }
     int apply_patches(const T *x, T *y, hipStream_t s) {
         const ElementPatches *pt = m->cells.get();
@@ -324,7 +321,7 @@ struct ElasticityOp final : OpBase {
     // hex8 on element patches: geometry and coefficient words in patch-slot order
     DevArray<float> adjp, detp, coeffp;
     DevArray<uint16_t> adjp16, detp16;
-    int patch_state{0};  // 0 not yet tried, 1 ready, -1 not applicable
+    LazyPart patch_words;
     DevArray<double> K;               // sshex8: per-macro 24x24 matrices
     DevArray<float> K32;              // sshex8, FP32 operator: K rounded to float
     DevArray<uint32_t> Apk;           // FP32 matrix cores: K32 split into bf16 A operands
@@ -462,12 +459,11 @@ struct ElasticityOp final : OpBase {
     }
     // hex8: the element patches of the mesh and this operator's words in their slot order (first use)
     bool patches_ready(hipStream_t s) {
-        std::lock_guard<std::recursive_mutex> lock(patch_mutex());
-        if (patch_state) return patch_state > 0;
-        if (!may_build_patches(s)) return false;
-        patch_state = -1;
+        return patch_words.ready(s, [&] { return make_patch_words(s); });
+    }
+    int make_patch_words(hipStream_t s) {
         const ElementPatches *pt = mesh_patches(m, s);
-        if (!pt || patch_lds_bytes(pt->maxloc, 3, sizeof(T)) > kPatchLdsLimit) return false;
+        if (!pt || patch_lds_bytes(pt->maxloc, 3, sizeof(T)) > kPatchLdsLimit) return -1;
         const ptrdiff_t Ep = m->E;
         bool ok;
         if constexpr (std::is_same<T, double>::value)
@@ -480,9 +476,7 @@ struct ElasticityOp final : OpBase {
                  !patch_gather_rows<uint16_t>(1, m->E, pt->perm.p, det16.p, detp16.p, s);
         if (ok && coeff.p)
             ok = !coeffp.alloc(Ep) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
-        if (!ok || hipStreamSynchronize(s) != hipSuccess) return false;
-        patch_state = 1;
-        return true;
+        return !ok || hipStreamSynchronize(s) != hipSuccess ? -1 : 1;
     }
     int apply_patches(const void *xv, void *yv, hipStream_t s) {
         const ElementPatches *pt = m->patches.get();
@@ -540,20 +534,19 @@ struct ConstrainedOp final : OpBase {
     // one is a skeleton (macro-element boundary) dof: its gather then writes y = x there; or as flags on the
     // nodes of an operator that writes every node in one pass (masks_nodes)
     DevArray<uint8_t> cmask, nmask;
-    int cmask_state{0}, nmask_state{0};  // 0: not yet built, 1: in use, -1: not applicable (separate copy)
+    LazyPart cmask_made, nmask_made;
     // the flags for the inner operator's present form (library options may change it), null: separate copy
     const uint8_t *mask(hipStream_t s, bool overwrite) {
         if (inner->masks_nodes(s)) {
             if (!overwrite) return nullptr;
-            if (nmask_state == 0 && may_build_patches(s)) nmask_state = build_nmask() ? -1 : 1;
-            return nmask_state > 0 ? nmask.p : nullptr;
+            return nmask_made.ready(s, [&] { return build_nmask() ? -1 : 1; }) ? nmask.p : nullptr;
         }
-        if (cmask_state == 0) {
-            cmask_state = -1;
-            if (!build_cmask(s)) cmask_state = 1;
+        const bool ok = cmask_made.ready(s, [&] {
+            const int st = build_cmask(s) ? -1 : 1;
             (void)hipGetLastError();
-        }
-        return cmask_state > 0 ? cmask.p : nullptr;
+            return st;
+        });
+        return ok ? cmask.p : nullptr;
     }
     int build_cmask(hipStream_t s) {
         const sfem_amd_mesh *gm = inner->gather_mesh(s);

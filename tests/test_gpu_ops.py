@@ -311,6 +311,48 @@ def test_one_operator_in_two_threads(kind):
     assert relerr(host(both), yo[0] + yo[1]) < RTOL
 
 
+def test_ready_operator_does_not_wait_for_another_mesh():
+    """Applies of an operator whose lists are made, while another thread's first elasticity apply makes
+    another mesh's patches on the host (some 100 ms): each takes a small part of that."""
+    import threading
+    import time
+
+    el, pts = skewed_box(36, perturb=0.003)
+    fff = O.hex8_fff(el, pts)
+    N = pts.shape[1]
+    x = np.random.default_rng(2).uniform(-1, 1, N)
+    op, xd, y = S.laplacian(S.Mesh(S.HEX8, 1, el, N), fff), dev(x), zeros(N)
+    for _ in range(100):
+        op.apply(xd, y)
+    S.synchronize()
+    el2, pts2 = S.box_mesh(97, 97, 97, element_type=S.HEX8)
+    N2 = pts2.shape[1]
+    other = S.linear_elasticity(S.Mesh(S.HEX8, 1, el2, N2), *S.adjugate_det(S.HEX8, 1, el2, pts2), *O.lame(1.0, 0.3))
+    x2, y2, took, failed = dev(np.ones(3 * N2)), zeros(3 * N2), [], []
+
+    def first():
+        try:
+            t = time.perf_counter()
+            other.apply(x2, y2)
+            took.append(time.perf_counter() - t)
+        except Exception as e:  # seen by the test's thread below
+            failed.append(e)
+
+    t = threading.Thread(target=first)
+    t.start()
+    waits = []
+    while t.is_alive():
+        t0 = time.perf_counter()
+        op.apply(xd, y)
+        waits.append(time.perf_counter() - t0)
+        time.sleep(0.0005)
+    t.join()
+    S.synchronize()
+    assert not failed
+    print(f"first apply {1e3 * took[0]:.1f} ms, {len(waits)} applies beside it, the longest {1e3 * max(waits):.2f} ms")
+    assert len(waits) > 1 and max(waits) < 0.5 * took[0]
+
+
 # One Chebyshev step on rhs = 0 moves x along A x: the overwriting, constrained apply of small hex8 meshes (node by
 # node, or element by element with the option off) against the oracle.  "random": nodes with many more than eight
 # corners, corners that share a node, nodes without any.
