@@ -152,6 +152,42 @@ struct ElementPatches {
 struct NodeElements {
     DevArray<int32_t> off, ent;
 };
+
+// Making the lists above allocates and synchronises: not while the stream is being captured.
+bool may_build_patches(hipStream_t s);
+// Something a mesh or an operator makes at its first use, once, whichever of several threads comes first.  Once
+// made it costs an apply one atomic load: no lock is taken, and what another operator or mesh is making is not
+// waited for.  While the stream is being captured nothing is made and no lock is taken either.
+struct LazyPart {
+    // make(): 1 in use; -1 not applicable; 0 failed this time (memory, or another thread's capture), to be tried
+    // again by the next call, and from the second failure on after 16, 32, ... calls
+    template <typename Make>
+    bool ready(hipStream_t s, Make make) {
+        int st = state.load(std::memory_order_acquire);
+        if (st) return st > 0;
+        if (!may_build_patches(s)) return false;
+        std::lock_guard<std::mutex> lock(making);
+        st = state.load(std::memory_order_relaxed);
+        if (st) return st > 0;
+        if (skip > 0) {
+            skip--;
+            return false;
+        }
+        st = make();
+        if (!st) {
+            (void)hipGetLastError();  // the caller goes on without it
+            if (failures < 16) failures++;
+            skip = failures > 1 ? 8 << failures >> 1 : 0;
+        }
+        state.store(st, std::memory_order_release);
+        return st > 0;
+    }
+
+private:
+    std::atomic<int> state{0};
+    std::mutex making;
+    int failures{0}, skip{0};
+};
 }  // namespace sfem_amd
 
 struct sfem_amd_op {
@@ -176,8 +212,8 @@ struct sfem_amd_mesh {
     mutable std::unique_ptr<sfem_amd::ElementPatches> patches, cells;
     // hex8: the elements around each node (lazy, mesh_node_elements)
     mutable std::unique_ptr<sfem_amd::NodeElements> around;
-    mutable std::atomic<const sfem_amd::NodeElements *> around_ready{nullptr};
-    mutable std::mutex lists;  // held while patches, cells or around are made
+    mutable sfem_amd::LazyPart around_made;
+    mutable std::mutex lists;  // held while patches or cells are made
 };
 
 namespace sfem_amd {
@@ -215,32 +251,10 @@ int mesh_skeleton(const sfem_amd_mesh *m, int Lc);
 // The sshex8 mesh's macro elements as (L/Ls)^3 sub-blocks of level Ls (sshex8_subblock_idx), built
 // once per level and shared; null on failure.
 const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t s);
-// Build (once) the element patches of a tet4/hex8 mesh (see patches.hip for the two kinds); null on
-// failure or for other meshes.  Building allocates and synchronises, so not while the stream is being
-// captured (may_build_patches): the element-wise kernels run then, and the next apply tries again.
-const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
-const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
-bool may_build_patches(hipStream_t s);
-// Something an operator makes at its first use, once, whichever of several threads comes first.  Once made it
-// costs an apply one atomic load: no lock is taken, and what another operator or mesh is making is not waited for.
-// While the stream is being captured nothing is made and no lock is taken either.
-struct LazyPart {
-    // make() is 1 (in use) or -1 (not applicable)
-    template <typename Make>
-    bool ready(hipStream_t s, Make make) {
-        int st = state.load(std::memory_order_acquire);
-        if (st) return st > 0;
-        if (!may_build_patches(s)) return false;
-        std::lock_guard<std::mutex> lock(making);
-        st = state.load(std::memory_order_relaxed);
-        if (!st) state.store(st = make(), std::memory_order_release);
-        return st > 0;
-    }
-
-private:
-    std::atomic<int> state{0};
-    std::mutex making;
-};
+// Build (once) the element patches of a tet4/hex8 mesh (see patches.hip for the two kinds), as
+// LazyPart's make() does.
+int mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
+int mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
 // The corners of a tet4/hex8 mesh by node, built by the first call outside a capture; null where they are not
 // available (the element-wise kernels run then).
 const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s);

@@ -133,9 +133,10 @@ __global__ void list_sizes_kernel(const ptrdiff_t n, const int32_t *__restrict__
     GRID_LOOP(i, n) size[i] = off[i + 1] - off[i];
 }
 
-// label: element -> group (device, destroyed); groups become patches of at most cap elements
+// label: element -> group (device, destroyed); groups become patches of at most cap elements.  never: it fails
+// for this mesh whenever it is tried
 int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label, int cap, ElementPatches &pt,
-             hipStream_t s) {
+             bool &never, hipStream_t s) {
     const int nv = m->nv;
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * nv;
     Scratch sc;
@@ -177,6 +178,7 @@ int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label
     int32_t maxloc = 0;
     if (fetch(incl.p, &maxloc, s)) return SFEM_FAILURE;
     if (maxloc > 65535) {
+        never = true;
         set_last_error("element patches: more than 65535 nodes in a patch");
         return SFEM_FAILURE;
     }
@@ -311,16 +313,17 @@ __global__ void reseed_kernel(const ptrdiff_t K, const unsigned long long *__res
 // rounds the cells off.  hex8 box, 440 elements a cell: 1.62, 1.58 patch nodes per element before and after
 // (1.55 for the ordered growth of mesh_patches); sizes spread by a factor of about two around the mean, and
 // cells above 2.5 times the mean are cut.
-const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
+int mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
     std::lock_guard<std::mutex> lock(m->lists);
-    if (m->cells) return m->cells.get();
+    if (m->cells) return 1;
     const ptrdiff_t E = m->E, N = m->nnodes;
     const int nv = m->nv;
-    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)E * nv >= 2147483647.0 || N >= 2147483647) return nullptr;
+    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)E * nv >= 2147483647.0 || N >= 2147483647) return -1;
     // Elements per cell: enough cells for the GPU's 256 CUs several times over, and from there on larger ones,
     // since the shared nodes' part falls with the size; a tetrahedron brings a sixth of a hexahedron's nodes.
     const ptrdiff_t mean = std::min<ptrdiff_t>(std::max<ptrdiff_t>(E / kCellsWanted, kPatchElements),
                                                m->type == SFEM_AMD_TET4 ? kCellTets : kCellHexes);
+    bool never = false;
     auto build = [&]() -> std::unique_ptr<ElementPatches> {
         Scratch sc;
         DevArray<int32_t> label, dist, seed, lo, hi, counter;
@@ -337,6 +340,7 @@ const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
             if (fetch(hi.p + E - 1, &last[0], s) || fetch(lo.p + E - 1, &last[1], s)) return SFEM_FAILURE;
             const ptrdiff_t K = (ptrdiff_t)last[0] + last[1];
             if (K > (ptrdiff_t)kLabelMask) {
+                never = true;
                 set_last_error("element cells: too many cells");
                 return SFEM_FAILURE;
             }
@@ -384,13 +388,14 @@ const ElementPatches *mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
                 LAUNCH(deepest_kernel, E, label.p, depth.p, best.p);
                 LAUNCH(reseed_kernel, K, best.p, seed.p);
             }
-            return assemble(m, label, max_label, (int)std::max<ptrdiff_t>(mean * 5 / 2, kPatchElements), pt, s);
+            return assemble(m, label, max_label, (int)std::max<ptrdiff_t>(mean * 5 / 2, kPatchElements), pt, never,
+                            s);
         };
         auto pt = std::make_unique<ElementPatches>();
         return work(*pt) ? fail() : std::move(pt);
     };
     m->cells = build();
-    return m->cells.get();
+    return m->cells ? 1 : never ? -1 : 0;
 }
 
 // ---------------------------------------------------------------- ordered patches
@@ -409,12 +414,13 @@ __global__ void element_major_keys_kernel(const ptrdiff_t n, const ptrdiff_t E, 
 // On a structured box of hexahedra the patches come out as compact blocks (about 1.55 patch nodes per
 // element, against 1.42 for a perfect 8^3 cube and 8 for no sharing).  A node whose elements have all
 // been assigned is never looked at again, which leaves about one visit per (node, element) pair.
-const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
+int mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
     std::lock_guard<std::mutex> lock(m->lists);
-    if (m->patches) return m->patches.get();
+    if (m->patches) return 1;
     const int nv = m->nv;
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * nv;
-    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)E * nv >= 2147483647.0 || N >= 2147483647) return nullptr;
+    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)E * nv >= 2147483647.0 || N >= 2147483647) return -1;
+    bool never = false;
     constexpr size_t P = kPatchElements;
     auto pt = std::make_unique<ElementPatches>();
     auto work = [&]() -> int {
@@ -486,11 +492,11 @@ const ElementPatches *mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
         }
         DevArray<int32_t> label;
         if (label.upload(patch_of.data(), patch_of.size())) return SFEM_FAILURE;
-        return assemble(m, label, pid, kPatchElements, *pt, s);
+        return assemble(m, label, pid, kPatchElements, *pt, never, s);
     };
-    if (work()) return nullptr;
+    if (work()) return never ? -1 : 0;
     m->patches = std::move(pt);
-    return m->patches.get();
+    return 1;
 }
 
 // ---------------------------------------------------------------- corners by node
@@ -504,13 +510,9 @@ __global__ void corners_kernel(const ptrdiff_t n, const ptrdiff_t E, const int n
         atomicAdd(&count[g], 1);
     }
 }
-const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
-    if (const NodeElements *ne = m->around_ready.load(std::memory_order_acquire)) return ne;
-    if (!may_build_patches(s)) return nullptr;
-    std::lock_guard<std::mutex> lock(m->lists);
-    if (m->around) return m->around.get();
+static int make_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
     const ptrdiff_t E = m->E, N = m->nnodes, n = E * m->nv;
-    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)n >= 2147483647.0 || N >= 2147483646) return nullptr;
+    if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)n >= 2147483647.0 || N >= 2147483646) return -1;
     auto ne = std::make_unique<NodeElements>();
     auto work = [&]() -> int {
         Scratch sc;
@@ -526,10 +528,12 @@ const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
         SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
         return SFEM_SUCCESS;
     };
-    if (work()) return nullptr;
+    if (work()) return 0;
     m->around = std::move(ne);
-    m->around_ready.store(m->around.get(), std::memory_order_release);
-    return m->around.get();
+    return 1;
+}
+const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
+    return m->around_made.ready(s, [&] { return make_node_elements(m, s); }) ? m->around.get() : nullptr;
 }
 
 bool may_build_patches(hipStream_t s) {

@@ -281,13 +281,14 @@ struct LaplacianOp final : OpBase {
         return patch_words.ready(s, [&] { return make_patch_words(s); });
     }
     int make_patch_words(hipStream_t s) {
-        const ElementPatches *pt = mesh_cells(m, s);
-        if (!pt || patch_lds_bytes(pt->maxloc, 1, sizeof(double)) > kPatchLdsLimit) return -1;
+        if (const int st = mesh_cells(m, s); st <= 0) return st;
+        const ElementPatches *pt = m->cells.get();
+        if (patch_lds_bytes(pt->maxloc, 1, sizeof(double)) > kPatchLdsLimit) return -1;
         bool ok = !fffp.alloc((size_t)6 * m->E) &&
                   !patch_gather_rows<float>(6, m->E, pt->perm.p, fff32.p, fffp.p, s);
         if (ok && coeff.p)
             ok = !coeffp.alloc(m->E) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
-        return !ok || hipStreamSynchronize(s) != hipSuccess ? -1 : 1;
+        return ok && hipStreamSynchronize(s) == hipSuccess ? 1 : 0;
     }
     int apply_patches(const T *x, T *y, hipStream_t s) {
         const ElementPatches *pt = m->cells.get();
@@ -462,8 +463,9 @@ struct ElasticityOp final : OpBase {
         return patch_words.ready(s, [&] { return make_patch_words(s); });
     }
     int make_patch_words(hipStream_t s) {
-        const ElementPatches *pt = mesh_patches(m, s);
-        if (!pt || patch_lds_bytes(pt->maxloc, 3, sizeof(T)) > kPatchLdsLimit) return -1;
+        if (const int st = mesh_patches(m, s); st <= 0) return st;
+        const ElementPatches *pt = m->patches.get();
+        if (patch_lds_bytes(pt->maxloc, 3, sizeof(T)) > kPatchLdsLimit) return -1;
         const ptrdiff_t Ep = m->E;
         bool ok;
         if constexpr (std::is_same<T, double>::value)
@@ -476,7 +478,7 @@ struct ElasticityOp final : OpBase {
                  !patch_gather_rows<uint16_t>(1, m->E, pt->perm.p, det16.p, detp16.p, s);
         if (ok && coeff.p)
             ok = !coeffp.alloc(Ep) && !patch_gather_rows<float>(1, m->E, pt->perm.p, coeff.p, coeffp.p, s);
-        return !ok || hipStreamSynchronize(s) != hipSuccess ? -1 : 1;
+        return ok && hipStreamSynchronize(s) == hipSuccess ? 1 : 0;
     }
     int apply_patches(const void *xv, void *yv, hipStream_t s) {
         const ElementPatches *pt = m->patches.get();
@@ -539,7 +541,7 @@ struct ConstrainedOp final : OpBase {
     const uint8_t *mask(hipStream_t s, bool overwrite) {
         if (inner->masks_nodes(s)) {
             if (!overwrite) return nullptr;
-            return nmask_made.ready(s, [&] { return build_nmask() ? -1 : 1; }) ? nmask.p : nullptr;
+            return nmask_made.ready(s, [&] { return build_nmask(); }) ? nmask.p : nullptr;
         }
         const bool ok = cmask_made.ready(s, [&] {
             const int st = build_cmask(s) ? -1 : 1;
@@ -555,15 +557,15 @@ struct ConstrainedOp final : OpBase {
     }
     int build_nmask() {
         const int bs = inner->block_size();
-        if (bs > 8) return SFEM_FAILURE;
+        if (bs > 8) return -1;
         std::vector<int32_t> d(dofs.n);
         if (!d.empty() &&
             hipMemcpy(d.data(), dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) != hipSuccess)
-            return SFEM_FAILURE;
+            return 0;
         std::vector<uint8_t> k((size_t)(inner->rows() / bs), 0);
         for (const int32_t q : d)
             if (q >= 0 && (size_t)(q / bs) < k.size()) k[(size_t)(q / bs)] |= (uint8_t)(1u << (q % bs));
-        return nmask.upload(k.data(), k.size());
+        return nmask.upload(k.data(), k.size()) ? 0 : 1;
     }
     int apply(const void *x, void *y, hipStream_t s) override {
         if (const uint8_t *k = mask(s, false)) return inner->apply_constrained(x, y, k, 0, s);
