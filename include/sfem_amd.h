@@ -406,8 +406,10 @@ int sfem_amd_dense_op_create(int real_type, ptrdiff_t n, const double *matrix, s
  * first apply runs eagerly, the second is captured and launched, later applies with the same
  * (x, y, stream) relaunch the graph and others run eagerly.  For launch-bound sequences without
  * host synchronisation, e.g. a preconditioning V-cycle (max_it 1) with a dense coarse solve; an
- * op whose apply synchronises with the host (a coarse CG) cannot be captured, and its second apply
- * returns the capture error. */
+ * op whose apply synchronises with the host (a coarse CG) cannot be captured and runs eagerly
+ * from then on.  The capture is on a stream of the op's own: other threads may call the library
+ * meanwhile (its synchronous calls wait for the end of the capture), but the HIP runtime refuses
+ * their own hipMemcpy and hipDeviceSynchronize in that time, and drops the capture. */
 int sfem_amd_graph_op_create(sfem_amd_op *op, sfem_amd_op **out);
 /* captured: graphs instantiated (one per initial-guess mode and per accumulating or overwriting
  * apply: the zero-guess overwriting apply a CG makes of its preconditioner records a different

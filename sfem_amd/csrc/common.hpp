@@ -37,12 +37,32 @@ void set_last_error(const std::string &msg);
 // Calls that pass no stream (NULL) run on the legacy default stream: the stream that such a caller's own
 // copies, fills and kernels are on, so nothing has to be ordered across streams.  (On a blocking stream of
 // the library's own, each change between it and the caller's default stream cost about 15 us: a zero fill
-// and an apply of 14 us of kernels took 46 us.)  The default stream cannot be captured, and cannot be used
-// while a blocking stream is: NULL then means library_stream(), a blocking stream per device, which is what
-// graph-replaying operators capture.
+// and an apply of 14 us of kernels took 46 us.)  Two exceptions: in a thread that records a graph-replaying
+// operator NULL is the operator's recording stream (RecordingScope), and while the caller captures a blocking
+// stream, when the default stream may not be used, it is library_stream(), a blocking stream per device.
 hipStream_t library_stream();
 hipStream_t default_stream();
 inline hipStream_t as_stream(void *s) { return s ? reinterpret_cast<hipStream_t>(s) : default_stream(); }
+// Records on rec, a stream of the caller's own, in thread-local mode: begin, the calls, end.  Until end (or the
+// destructor) this thread's calls without a stream run on rec.
+class RecordingScope {
+public:
+    explicit RecordingScope(hipStream_t rec);
+    ~RecordingScope() { (void)end(); }
+    RecordingScope(const RecordingScope &) = delete;
+    RecordingScope &operator=(const RecordingScope &) = delete;
+    bool begun() const { return rec_ != nullptr; }
+    hipGraph_t end();  // null: the capture was dropped
+
+private:
+    hipStream_t rec_;
+};
+// The HIP runtime refuses synchronous copies and device synchronisation in every thread while any stream of the
+// process is being captured, and drops that capture.  The library's own therefore wait for its recordings (some
+// milliseconds at most) and its recordings for them; a recording thread's own do not wait, and are refused.
+hipError_t sync_memcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind);
+hipError_t sync_memset(void *dst, int value, size_t bytes);
+hipError_t sync_device();
 
 // ----------------------------------------------------------------- structured helpers
 // operators/sshex8/sshex8.hpp:18-24: local id = z*(L+1)^2 + y*(L+1) + x

@@ -40,7 +40,7 @@ struct DevArray {
     int upload(const T *h, size_t count) {
         if (alloc(count)) return SFEM_FAILURE;
         // host or device source (unified addressing)
-        if (count) SFEM_AMD_HIP_CHECK(hipMemcpy(p, h, sizeof(T) * count, hipMemcpyDefault));
+        if (count) SFEM_AMD_HIP_CHECK(sync_memcpy(p, h, sizeof(T) * count, hipMemcpyDefault));
         return SFEM_SUCCESS;
     }
 };

@@ -136,8 +136,8 @@ int sfem_amd_cnn_create_channels(int channels, int hidden, int layers, const flo
         }
     }
     if (c->W.upload(h.data(), off) || c->grad.alloc(off) || c->m.alloc(off) || c->v.alloc(off)) return SFEM_FAILURE;
-    SFEM_AMD_HIP_CHECK(hipMemset(c->m.p, 0, sizeof(float) * off));
-    SFEM_AMD_HIP_CHECK(hipMemset(c->v.p, 0, sizeof(float) * off));
+    SFEM_AMD_HIP_CHECK(sync_memset(c->m.p, 0, sizeof(float) * off));
+    SFEM_AMD_HIP_CHECK(sync_memset(c->v.p, 0, sizeof(float) * off));
     for (int l = 0; l < layers; l++) c->acts.push_back(new DevArray<float>());
     if (c->ws.alloc(514)) return SFEM_FAILURE;
     *out = c.release();
@@ -149,13 +149,13 @@ int sfem_amd_cnn_channels(const sfem_amd_cnn *c) { return c ? c->io : -1; }
 
 int sfem_amd_cnn_get_weights(const sfem_amd_cnn *c, float *w) {
     SFEM_AMD_REQUIRE(c && w, "cnn_get_weights: arguments");
-    SFEM_AMD_HIP_CHECK(hipMemcpy(w, c->W.p, sizeof(float) * c->nparams, hipMemcpyDeviceToHost));
+    SFEM_AMD_HIP_CHECK(sync_memcpy(w, c->W.p, sizeof(float) * c->nparams, hipMemcpyDeviceToHost));
     return SFEM_SUCCESS;
 }
 
 int sfem_amd_cnn_set_weights(sfem_amd_cnn *c, const float *w) {
     SFEM_AMD_REQUIRE(c && w, "cnn_set_weights: arguments");
-    SFEM_AMD_HIP_CHECK(hipMemcpy(c->W.p, w, sizeof(float) * c->nparams, hipMemcpyHostToDevice));
+    SFEM_AMD_HIP_CHECK(sync_memcpy(c->W.p, w, sizeof(float) * c->nparams, hipMemcpyHostToDevice));
     c->w16_valid = false;
     bump_state_epoch();
     return SFEM_SUCCESS;
@@ -172,13 +172,13 @@ int sfem_amd_cnn_forward(sfem_amd_cnn *c, int L, ptrdiff_t E, const float *z, fl
                          "cnn_forward: the MFMA path is built for the scalar network of 4 layers of 16");
         if (!c->w16_valid) {
             std::vector<float> h(c->nparams);
-            SFEM_AMD_HIP_CHECK(hipMemcpy(h.data(), c->W.p, sizeof(float) * c->nparams, hipMemcpyDeviceToHost));
+            SFEM_AMD_HIP_CHECK(sync_memcpy(h.data(), c->W.p, sizeof(float) * c->nparams, hipMemcpyDeviceToHost));
             std::vector<uint16_t> hb(kCnnPackedWeights);
             cnn_pack_weights(h.data(), hb.data());
             // allocated once: a graph captured earlier keeps a valid pointer (it re-captures anyway,
             // since weight changes move the state epoch)
             if (c->W16.n != hb.size() && c->W16.alloc(hb.size())) return SFEM_FAILURE;
-            SFEM_AMD_HIP_CHECK(hipMemcpy(c->W16.p, hb.data(), sizeof(uint16_t) * hb.size(), hipMemcpyHostToDevice));
+            SFEM_AMD_HIP_CHECK(sync_memcpy(c->W16.p, hb.data(), sizeof(uint16_t) * hb.size(), hipMemcpyHostToDevice));
             c->w16_valid = true;
         }
         return cnn_infer_mfma(L, E, c->W16.p, z, out, s);

@@ -433,9 +433,9 @@ int mesh_patches(const sfem_amd_mesh *m, hipStream_t s) {
             LAUNCH(element_major_keys_kernel, n, E, nv, m->idx.p, node.p, elem.p);
             if (sc.sort(node.p, snode.p, elem.p, selem.p, n, bits_for(N), s)) return SFEM_FAILURE;
             SFEM_AMD_HIP_CHECK(hipStreamSynchronize(s));
-            SFEM_AMD_HIP_CHECK(hipMemcpy(el.data(), node.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-            SFEM_AMD_HIP_CHECK(hipMemcpy(n2e.data(), selem.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-            SFEM_AMD_HIP_CHECK(hipMemcpy(nodes.data(), snode.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+            SFEM_AMD_HIP_CHECK(sync_memcpy(el.data(), node.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+            SFEM_AMD_HIP_CHECK(sync_memcpy(n2e.data(), selem.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+            SFEM_AMD_HIP_CHECK(sync_memcpy(nodes.data(), snode.p, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
         }
         for (const int32_t g : nodes) n2e_off[(size_t)g + 1]++;
         for (ptrdiff_t g = 0; g < N; g++) n2e_off[g + 1] += n2e_off[g];

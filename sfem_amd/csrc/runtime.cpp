@@ -8,6 +8,8 @@
 #include <cstring>
 #include <memory>
 #include <functional>
+#include <mutex>
+#include <shared_mutex>
 #include <string>
 #include <vector>
 
@@ -39,7 +41,50 @@ hipStream_t library_stream() {
     }
     return streams[dev];
 }
+static thread_local hipStream_t t_recording = nullptr;
+// A recording holds both; a synchronous call passes through the first and holds the second shared, so that calls
+// that overlap each other do not keep a recording waiting.
+static std::mutex g_recording_turn;
+static std::shared_mutex g_recording;
+RecordingScope::RecordingScope(hipStream_t rec) : rec_(nullptr) {
+    g_recording_turn.lock();
+    g_recording.lock();
+    if (hipStreamBeginCapture(rec, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+        t_recording = rec_ = rec;
+    } else {
+        g_recording.unlock();
+        g_recording_turn.unlock();
+    }
+}
+hipGraph_t RecordingScope::end() {
+    if (!rec_) return nullptr;
+    hipGraph_t graph = nullptr;
+    const bool ok = hipStreamEndCapture(rec_, &graph) == hipSuccess;
+    t_recording = rec_ = nullptr;
+    g_recording.unlock();
+    g_recording_turn.unlock();
+    if (!ok && graph) (void)hipGraphDestroy(graph);
+    return ok ? graph : nullptr;
+}
+static std::shared_lock<std::shared_mutex> between_recordings() {
+    if (t_recording) return {};
+    std::lock_guard<std::mutex> turn(g_recording_turn);
+    return std::shared_lock<std::shared_mutex>(g_recording);
+}
+hipError_t sync_memcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
+    const auto lock = between_recordings();
+    return hipMemcpy(dst, src, bytes, kind);
+}
+hipError_t sync_memset(void *dst, int value, size_t bytes) {
+    const auto lock = between_recordings();
+    return hipMemset(dst, value, bytes);
+}
+hipError_t sync_device() {
+    const auto lock = between_recordings();
+    return hipDeviceSynchronize();
+}
 hipStream_t default_stream() {
+    if (t_recording) return t_recording;
     // an error here says that a blocking stream is being captured
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(nullptr, &st) == hipSuccess) return nullptr;
@@ -75,7 +120,7 @@ int mesh_skeleton(const sfem_amd_mesh *m, int Lc) {
     }
     std::vector<int32_t> el((size_t)E * m->nv);
     if (!el.empty())
-        SFEM_AMD_HIP_CHECK(hipMemcpy(el.data(), m->idx.p, sizeof(int32_t) * el.size(), hipMemcpyDeviceToHost));
+        SFEM_AMD_HIP_CHECK(sync_memcpy(el.data(), m->idx.p, sizeof(int32_t) * el.size(), hipMemcpyDeviceToHost));
     // mesh-local index of every skeleton slot of the level-Lc view, in slot order
     std::vector<int> sk_lidx(nsk);
     for (int z = 0; z <= Lc; z++)
@@ -516,8 +561,8 @@ static int skeleton_dof_mask(const SkeletonMap &sk, int bs, const DevArray<int32
     if (bs > 8 || sk.n == 0) return SFEM_FAILURE;
     std::vector<int32_t> node((size_t)sk.n), d(dofs.n);
     if (hipStreamSynchronize(s) != hipSuccess ||
-        hipMemcpy(node.data(), sk.node, sizeof(int32_t) * node.size(), hipMemcpyDeviceToHost) != hipSuccess ||
-        (!d.empty() && hipMemcpy(d.data(), dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) != hipSuccess))
+        sync_memcpy(node.data(), sk.node, sizeof(int32_t) * node.size(), hipMemcpyDeviceToHost) != hipSuccess ||
+        (!d.empty() && sync_memcpy(d.data(), dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) != hipSuccess))
         return SFEM_FAILURE;
     std::vector<uint8_t> mask((size_t)sk.n, 0);
     for (const int32_t q : d) {
@@ -560,7 +605,7 @@ struct ConstrainedOp final : OpBase {
         if (bs > 8) return -1;
         std::vector<int32_t> d(dofs.n);
         if (!d.empty() &&
-            hipMemcpy(d.data(), dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) != hipSuccess)
+            sync_memcpy(d.data(), dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) != hipSuccess)
             return 0;
         std::vector<uint8_t> k((size_t)(inner->rows() / bs), 0);
         for (const int32_t q : d)
@@ -633,7 +678,7 @@ struct TransferOp final : OpBase {
             if (constrained) {
                 auto *c = static_cast<ConstrainedOp *>(constrained.get());
                 std::vector<int32_t> d(c->dofs.n);
-                if (!d.empty() && hipMemcpy(d.data(), c->dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) !=
+                if (!d.empty() && sync_memcpy(d.data(), c->dofs.p, sizeof(int32_t) * d.size(), hipMemcpyDeviceToHost) !=
                                           hipSuccess) {
                     set_last_error("prolongation: reading the constrained dofs failed");
                     return SFEM_FAILURE;
@@ -915,12 +960,14 @@ struct DenseOp final : OpBase {
 
 // Replays the apply of `inner` as a HIP graph.  Per initial-guess mode (set_initial_guess_zero,
 // which changes the recorded sequence) the first call runs eagerly (lazy allocations, one-time
-// kernel attributes), the second captures the launch sequence on its stream and launches the
+// kernel attributes), the second captures the launch sequence and launches the
 // graph; later calls with the same (x, y, stream) and mode relaunch it, other arguments run
-// eagerly.  The inner apply must not synchronise with the host (e.g. a preconditioning V-cycle
-// with a direct coarse solve).  A capture that cannot begin leaves the operator eager; an inner
-// apply that synchronises inside the capture invalidates it, and the HIP runtime then reports
-// that error on the next launch on the stream, so such an apply fails instead of running eagerly.
+// eagerly.  The capture is on a stream of the operator's own, which nothing else runs on, and which is
+// non-blocking, so that the default stream stays usable in other threads meanwhile.  On a stream that
+// the caller is capturing itself the operator runs eagerly, into that capture.
+// The inner apply must not synchronise with the host (e.g. a preconditioning V-cycle
+// with a direct coarse solve).  A capture that cannot begin, or that is dropped (an inner apply that
+// synchronises inside it, another thread's own synchronous HIP calls), leaves the operator eager.
 struct GraphOp final : OpBase {
     std::shared_ptr<OpBase> inner;
     struct Capture {
@@ -934,9 +981,11 @@ struct GraphOp final : OpBase {
     int replays{0};
     bool failed{false};
     bool zero_guess{false};
+    hipStream_t rec{nullptr};
     ~GraphOp() override {
         for (auto &c : cap)
             if (c.exec) (void)hipGraphExecDestroy(c.exec);
+        if (rec) (void)hipStreamDestroy(rec);
     }
     int captured() const {
         int n = 0;
@@ -957,6 +1006,8 @@ struct GraphOp final : OpBase {
     int run(const void *x, void *y, hipStream_t s, bool overwrite) {
         auto on = [&](hipStream_t q) { return overwrite ? inner->apply_overwrite(x, y, q) : inner->apply(x, y, q); };
         auto eager = [&] { return on(s); };
+        hipStreamCaptureStatus outer = hipStreamCaptureStatusNone;
+        if (s && hipStreamIsCapturing(s, &outer) == hipSuccess && outer != hipStreamCaptureStatusNone) return eager();
         Capture &c = cap[(overwrite ? 2 : 0) + (zero_guess ? 1 : 0)];
         const uint64_t now = state_epoch();
         if (c.exec && c.epoch != now) {
@@ -968,18 +1019,14 @@ struct GraphOp final : OpBase {
         }
         if (c.calls++ == 0 || failed) return eager();
         if (!c.exec) {
-            // the default stream cannot be captured: record on the library's, replay on the default one
-            hipStream_t rec = s ? s : library_stream();
-            if (hipStreamBeginCapture(rec, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-                failed = true;
-                (void)hipGetLastError();
-                return eager();
-            }
-            const int err = on(rec);
             hipGraph_t graph = nullptr;
-            const hipError_t e_end = hipStreamEndCapture(rec, &graph);
-            if (err || e_end != hipSuccess || !graph ||
-                hipGraphInstantiate(&c.exec, graph, nullptr, nullptr, 0) != hipSuccess) {
+            int err = SFEM_FAILURE;
+            if (rec || hipStreamCreateWithFlags(&rec, hipStreamNonBlocking) == hipSuccess) {
+                RecordingScope recording(rec);
+                if (recording.begun()) err = on(rec);
+                graph = recording.end();
+            }
+            if (err || !graph || hipGraphInstantiate(&c.exec, graph, nullptr, nullptr, 0) != hipSuccess) {
                 if (graph) (void)hipGraphDestroy(graph);
                 c.exec = nullptr;
                 failed = true;
@@ -1207,7 +1254,7 @@ int sfem_amd_device_count(void) {
 }
 
 int sfem_amd_device_synchronize(void) {
-    SFEM_AMD_HIP_CHECK(hipDeviceSynchronize());
+    SFEM_AMD_HIP_CHECK(sync_device());
     return SFEM_SUCCESS;
 }
 
@@ -1224,11 +1271,11 @@ int sfem_amd_free(void *p) {
     return SFEM_SUCCESS;
 }
 int sfem_amd_memcpy_h2d(void *dst, const void *src, size_t bytes) {
-    SFEM_AMD_HIP_CHECK(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+    SFEM_AMD_HIP_CHECK(sync_memcpy(dst, src, bytes, hipMemcpyHostToDevice));
     return SFEM_SUCCESS;
 }
 int sfem_amd_memcpy_d2h(void *dst, const void *src, size_t bytes) {
-    SFEM_AMD_HIP_CHECK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    SFEM_AMD_HIP_CHECK(sync_memcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return SFEM_SUCCESS;
 }
 int sfem_amd_memset(void *dst, int v, size_t bytes, void *stream) {
@@ -1349,7 +1396,7 @@ int sfem_amd_mesh_derefine(const sfem_amd_mesh *fine, int level, sfem_amd_mesh *
     m->parent = fine;
     // nested levels are prefixes of the fine numbering: node count = max id + 1
     std::vector<int32_t> h(m->idx.n);
-    SFEM_AMD_HIP_CHECK(hipMemcpy(h.data(), m->idx.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost));
+    SFEM_AMD_HIP_CHECK(sync_memcpy(h.data(), m->idx.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost));
     int32_t mx = -1;
     for (int32_t v : h) mx = v > mx ? v : mx;
     m->nnodes = (ptrdiff_t)mx + 1;
@@ -1365,7 +1412,7 @@ int sfem_amd_mesh_element_type(const sfem_amd_mesh *m) { return m ? m->type : -1
 int sfem_amd_mesh_download(const sfem_amd_mesh *m, int32_t *el) {
     CHECK_HANDLE(m);
     std::vector<int32_t> h(m->idx.n);
-    SFEM_AMD_HIP_CHECK(hipMemcpy(h.data(), m->idx.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost));
+    SFEM_AMD_HIP_CHECK(sync_memcpy(h.data(), m->idx.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost));
     if (m->type == SFEM_AMD_SSHEX8) {
         for (ptrdiff_t e = 0; e < m->E; e++)
             for (int v = 0; v < m->nv; v++) el[(size_t)v * m->E + e] = h[(size_t)e * m->nv + v];
@@ -1381,7 +1428,7 @@ void sfem_amd_mesh_destroy(sfem_amd_mesh *m) { delete m; }
 static int soa_upload(DevArray<float> &dst, const float *aos, ptrdiff_t E, int k) {
     if (device_pointer(aos)) {
         if (dst.alloc((size_t)k * E) || aos_to_soa_device(aos, E, k, dst.p, nullptr)) return SFEM_FAILURE;
-        SFEM_AMD_HIP_CHECK(hipDeviceSynchronize());
+        SFEM_AMD_HIP_CHECK(sync_device());
         return SFEM_SUCCESS;
     }
     std::vector<float> h((size_t)k * E);
@@ -1412,7 +1459,7 @@ int sfem_amd_laplacian_create(const sfem_amd_mesh *mesh, const float *fff, const
         SFEM_AMD_REQUIRE(!coeff || device_pointer(coeff), "laplacian_create: fff and coeff in the same memory");
         if (op->fff16.alloc((size_t)6 * E) || aos_to_bf16_soa_device(fff, coeff, E, 6, op->fff16.p, nullptr))
             return SFEM_FAILURE;
-        SFEM_AMD_HIP_CHECK(hipDeviceSynchronize());
+        SFEM_AMD_HIP_CHECK(sync_device());
         *out = wrap(op);
         return SFEM_SUCCESS;
     }
@@ -1477,7 +1524,7 @@ int sfem_amd_linear_elasticity_create(const sfem_amd_mesh *mesh, const float *ad
                     aos_to_bf16_soa_device(adj, nullptr, E, 9, op->adj16.p, nullptr) ||
                     aos_to_bf16_soa_device(det, nullptr, E, 1, op->det16.p, nullptr))
                     return SFEM_FAILURE;
-                SFEM_AMD_HIP_CHECK(hipDeviceSynchronize());
+                SFEM_AMD_HIP_CHECK(sync_device());
                 return SFEM_SUCCESS;
             }
             std::vector<uint16_t> ha((size_t)9 * E), hd(E);
@@ -1518,7 +1565,7 @@ int sfem_amd_linear_elasticity_create(const sfem_amd_mesh *mesh, const float *ad
                                                      nullptr))
                 return SFEM_FAILURE;
         }
-        SFEM_AMD_HIP_CHECK(hipDeviceSynchronize());
+        SFEM_AMD_HIP_CHECK(sync_device());
         return SFEM_SUCCESS;
     };
     if (rt == SFEM_AMD_FLOAT64) {
@@ -1622,7 +1669,7 @@ static int transfer_create(const sfem_amd_mesh *fine, const sfem_amd_mesh *coars
         if (tmp.alloc((size_t)nxe_of(coarse->level) * fine->E)) return SFEM_FAILURE;
         if (sshex8_derefine(fine->E, fine->level, coarse->level, fine->idx.p, tmp.p, nullptr)) return SFEM_FAILURE;
         std::vector<int32_t> h(tmp.n);
-        SFEM_AMD_HIP_CHECK(hipMemcpy(h.data(), tmp.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost));
+        SFEM_AMD_HIP_CHECK(sync_memcpy(h.data(), tmp.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost));
         for (int32_t v : h) SFEM_AMD_REQUIRE(v >= 0 && v < coarse->nnodes, "transfer: meshes are not nested (coarse id out of range)");
     }
     auto make = [&](auto op) {

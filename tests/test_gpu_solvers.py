@@ -589,6 +589,97 @@ def test_graph_replayed_vcycle_matches_eager(real_type):
     assert captured == 2 and replays2 >= replays + its[1] - 2
 
 
+def test_graph_operator_on_a_stream_of_the_caller():
+    """A V-cycle (whose own calls name no stream) replayed on a stream of the caller's: every replay equals
+    the eager cycle."""
+    import ctypes as C
+    hip = C.CDLL(None)  # the HIP runtime that the library has loaded
+    L = 2
+    mel, mpts, el, pts, fff, N, nodes, coeff = _ss_poisson(L, 3, coeff_seed=3)
+    mesh = S.Mesh(S.SSHEX8, L, el, N)
+    h = gmg.SSGMG(mesh, "laplacian", fff, nodes, coeff=coeff, coarse="dense", macro_box=(3, 1.0))
+    P_eager, P_graph = h.preconditioner(graph=False), h.preconditioner(graph=True)
+    stream = C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0  # blocking: in order with the default stream
+    rng = np.random.default_rng(6)
+    r, z = zeros(N), zeros(N)
+    for k in range(4):
+        r.copy_from(rng.uniform(-1, 1, N))
+        want = zeros(N)
+        P_eager.apply(r, want)
+        z.zero()
+        P_graph.apply(r, z, stream.value)
+        assert hip.hipStreamSynchronize(stream) == 0
+        S.synchronize()
+        assert np.linalg.norm(host(z) - host(want)) < 1e-12 * np.linalg.norm(host(want)), k
+    assert S.graph_op_stats(P_graph) == (1, 3)
+    assert hip.hipStreamDestroy(stream) == 0
+
+
+def test_graphs_recorded_in_two_threads_beside_calls_without_a_stream():
+    """While two graph operators record in threads of their own, calls without a stream in this one run
+    at once, outside both graphs, and both recordings succeed.  The recorded sequence is long (2,000
+    Chebyshev steps), so that many such calls fall into it."""
+    import threading
+    import time
+
+    el, pts = O.box_mesh(4, 4, 4)
+    fff = O.hex8_fff(el, pts)
+    N = pts.shape[1]
+    nodes = np.where(pts[0] == 0)[0].astype(np.int32)
+    mesh = S.Mesh(S.HEX8, 1, el, N)
+    b = np.random.default_rng(3).uniform(-1, 1, N)
+    b[nodes] = 0
+
+    def smoother():
+        A = S.constrained(S.laplacian(mesh, fff), nodes)
+        return A, S.cheb3(A, max_it=2000)
+
+    A0, eager = smoother()
+    want = zeros(N)
+    for _ in range(3):
+        eager.apply(dev(b), want)
+    ops = [(A, S.graph_op(P)) for A, P in (smoother() for _ in range(2))]
+    rhs, out = [dev(b) for _ in ops], [zeros(N) for _ in ops]
+    for (_, P), r, y in zip(ops, rhs, out):
+        P.apply(r, y)  # eager
+    S.synchronize()
+    recording, failed = [None, None], []
+
+    def record(i):
+        try:
+            t = time.perf_counter()
+            ops[i][1].apply(rhs[i], out[i])  # recorded, then launched
+            recording[i] = (t, time.perf_counter())
+        except Exception as e:  # seen by the test's thread below
+            failed.append(e)
+
+    ts = [threading.Thread(target=record, args=(i,)) for i in range(2)]
+    a, n, calls = S.DeviceArray(1000), 0, []
+    for t in ts:
+        t.start()
+    while any(t.is_alive() for t in ts):
+        n += 1
+        t0 = time.perf_counter()
+        assert S.lib.sfem_amd_blas_values(S.FLOAT64, 1000, float(n), S._dptr(a), None) == 0
+        got = a.numpy()
+        calls.append((t0, time.perf_counter()))
+        assert np.all(got == n), (n, got[:4])
+    for t in ts:
+        t.join()
+    assert not failed
+    inside = [sum(lo < p and q < hi for p, q in calls) for lo, hi in recording]
+    print(f"calls inside each recording: {inside}", flush=True)
+    assert min(inside) > 0
+    for k, ((_, P), r, y) in enumerate(zip(ops, rhs, out)):
+        assert S.graph_op_stats(P) == (1, 1), k
+        a.fill(-1.0)
+        P.apply(r, y)
+        S.synchronize()
+        assert np.linalg.norm(host(y) - host(want)) <= 1e-12 * np.linalg.norm(host(want))
+        assert np.all(a.numpy() == -1)  # not in the graph
+
+
 def test_block_jacobi_smoother_parity_and_default_gmg():
     """Block-Jacobi stationary smoother (3x3 nodal blocks, omega 1/3, constrained rows as unit
     rows) against the oracle's, and MG-PCG with the reference's default smoothers on elasticity."""
