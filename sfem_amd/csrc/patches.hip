@@ -538,7 +538,9 @@ const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s) {
 
 bool may_build_patches(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(s, &st);
+    if (e == hipErrorStreamCaptureImplicit) (void)hipGetLastError();  // a blocking stream is being captured
+    return e == hipSuccess && st == hipStreamCaptureStatusNone;
 }
 
 }  // namespace sfem_amd

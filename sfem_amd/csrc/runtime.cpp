@@ -32,8 +32,10 @@ void set_last_error(const std::string &msg) { g_last_error = msg; }
 hipStream_t library_stream() {
     constexpr int kMaxDevices = 64;
     static hipStream_t streams[kMaxDevices] = {};
+    static std::mutex making;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+    std::lock_guard<std::mutex> lock(making);
     if (!streams[dev]) {
         hipStream_t st = nullptr;
         if (hipStreamCreate(&st) != hipSuccess) return nullptr;
@@ -85,9 +87,10 @@ hipError_t sync_device() {
 }
 hipStream_t default_stream() {
     if (t_recording) return t_recording;
-    // an error here says that a blocking stream is being captured
+    // this error says that a blocking stream is being captured; any other is left for the caller's own calls to
+    // report
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(nullptr, &st) == hipSuccess) return nullptr;
+    if (hipStreamIsCapturing(nullptr, &st) != hipErrorStreamCaptureImplicit) return nullptr;
     (void)hipGetLastError();
     return library_stream();
 }
