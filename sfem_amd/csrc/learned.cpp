@@ -33,8 +33,11 @@ struct sfem_amd_cnn {
 
 namespace {
 
+// A workspace of a captured graph (a smoother over this network on the FP32 path) may be among those that grow: the
+// epoch moves before the old one is freed, so that no such graph is launched again.
 int ensure(DevArray<float> &a, size_t n) {
     if (a.n >= n) return SFEM_SUCCESS;
+    if (a.p) bump_state_epoch();
     return a.alloc(n);
 }
 

@@ -329,6 +329,47 @@ def test_graph_replayed_learned_hierarchy_follows_switches_and_fallback():
     assert results[0][1] == 0 and results[0][2] == 1
 
 
+def test_graph_over_a_learned_smoother_follows_the_network_workspaces():
+    """The FP32 path's activations are workspaces of the network, which a larger batch replaces: a graph
+    over a smoother that was captured before is captured again, and its output equals the eager one's."""
+    L = 2
+    mel, mpts = S.box_mesh(3, 3, 3, element_type=S.HEX8)
+    el, pts = S.sshex8_refine(L, mel, mpts)
+    N, n = pts.shape[1], (L + 1) ** 3
+    mesh = S.Mesh(S.SSHEX8, L, el, N)
+    bc = np.where(pts[2] < 1e-6)[0].astype(np.int32)
+    A = S.constrained(S.laplacian(mesh, S.fff(S.HEX8, 1, mel, mpts), real_type=S.FLOAT32), bc)
+    d = S.DeviceArray(N, np.float32)
+    A.diag(d)
+    nets = [S.CNN(16, 4, seed=2) for _ in range(2)]  # alike: one for the graph, one for the eager smoother
+    graph, eager = (S.learned_smoother(A, mesh, c, d, mode=0) for c in nets)
+    graph = S.graph_op(graph)
+    rng = np.random.default_rng(8)
+    b, y = dev(rng.uniform(-1, 1, N)), S.DeviceArray(N, np.float32)
+
+    def check():
+        x = rng.uniform(-1, 1, N)
+        want = dev(x)
+        y.copy_from(x.astype(np.float32))
+        eager.apply(b, want)
+        graph.apply(b, y)
+        S.synchronize()
+        assert rel(y.numpy(), want.numpy()) < 1e-6
+
+    for _ in range(3):
+        check()
+    assert S.graph_op_stats(graph) == (1, 2)
+    for batch in (3 * mel.shape[1], 40 * mel.shape[1]):
+        z, t = (dev(rng.normal(size=batch * n)) for _ in range(2))
+        nets[0].loss_grad(L, z, t)  # no step: the weights stay
+        replays = S.graph_op_stats(graph)[1]
+        check()  # eager
+        assert S.graph_op_stats(graph) == (0, replays)
+        for k in range(2):
+            check()
+            assert S.graph_op_stats(graph) == (1, replays + k + 1)
+
+
 def test_vector_cnn_forward_and_gradient_match_oracle():
     """The 3-channel network (one channel per displacement component) against the float64 oracle:
     forward and the loss gradient of every layer."""
