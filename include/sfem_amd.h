@@ -18,7 +18,9 @@
  * Operator apply ACCUMULATES, y += A x (frontend/sfem_Function.cpp:481-496); solvers
  * use x as initial guess and output (algebra/sfem_cg.hpp:207-213).
  * `stream` is a hipStream_t passed as void*; NULL is the default stream.  Calls do
- * not synchronise except where they return a host scalar (dot, norm, solve).
+ * not synchronise except where they return a host scalar (dot, norm, solve), and applies
+ * where they make, once, what the operator or its mesh keeps (index lists, the partitions
+ * of the option "hex8_patches" below, workspaces).
  * Objects are not re-entrant: calls that overlap on one handle race.  A mesh must outlive
  * the operators and transfers created on it; operators built from other operators (solvers,
  * constrained operators, multigrid) keep shared references to them.
@@ -64,8 +66,10 @@ const char *sfem_amd_last_error(void);
  * 2 the stencil form (levels 2-6, 8, 10, 12, 16).  Both give the reference's operator; the
  * summation order differs.  "hex8_patches" (default 1): tet4 and hex8 applies on meshes of at least
  * 2^15 elements run on element patches (512 or 2,048 elements grown over shared nodes, accumulated in
- * LDS and added to y with atomics; the partition is made by a mesh's first apply, the elasticity's on
- * the host), and the overwriting applies inside solvers on smaller hex8 meshes node by node; 0 runs one
+ * LDS and added to y with atomics; the partition is made inside an apply: the elasticity's by the first
+ * one, on the host, the Laplacian's once a mesh's element-wise applies have cost about as much, after 25
+ * to 105 of them, or before a graph op records one; 2 makes the Laplacian's by the first apply too, for
+ * programs that capture applies themselves), and the overwriting applies inside solvers on smaller hex8 meshes node by node; 0 runs one
  * element per lane with atomics.
  * "mixed_cg" (default 1): flexible CGs created afterwards around a bridged FP32 preconditioner keep
  * z in FP32 (see sfem_amd_cg_create; the same iterates); 0 runs them through the bridge's casts. */

@@ -163,9 +163,14 @@ struct LazyPart {
     // again by the next call, and from the second failure on after 16, 32, ... calls
     template <typename Make>
     bool ready(hipStream_t s, Make make) {
+        return ready(s, make, [] { return true; });
+    }
+    // due(): false to leave the making to a later call
+    template <typename Make, typename Due>
+    bool ready(hipStream_t s, Make make, Due due) {
         int st = state.load(std::memory_order_acquire);
         if (st) return st > 0;
-        if (!may_build_patches(s)) return false;
+        if (!due() || !may_build_patches(s)) return false;
         std::lock_guard<std::mutex> lock(making);
         st = state.load(std::memory_order_relaxed);
         if (st) return st > 0;
@@ -210,6 +215,7 @@ struct sfem_amd_mesh {
     mutable std::map<int, std::unique_ptr<sfem_amd_mesh>> sub;
     // tet4/hex8: element patches (lazy, mesh_patches and mesh_cells)
     mutable std::unique_ptr<sfem_amd::ElementPatches> patches, cells;
+    mutable std::atomic<int> laplacian_applies{0};  // element by element, see cells_due
     // hex8: the elements around each node (lazy, mesh_node_elements)
     mutable std::unique_ptr<sfem_amd::NodeElements> around;
     mutable sfem_amd::LazyPart around_made;
@@ -231,8 +237,9 @@ extern int g_elasticity_form;
 // patches: hex8 Laplacian 8,000 elements 6.8 / 8.2 us, 13,824 8.1 / 7.8, 32,768 15.1 / 7.9, 262,144 94 / 11;
 // tet4 6,000 5.5 / 5.2 us, 16,464 5.7 / 4.4, 34,992 9.0 / 4.8, 279,936 48 / 6.5; FP64 hex8 elasticity 8,000
 // 10 / 13 us, 13,824 17 / 14, 32,768 33 / 15.  The line lies above the crossing (about 12,000 elements)
-// because making the patches costs the first apply about 3 ms, at 2^14 elements over 500 applies' gain.
-extern bool g_hex8_patches;
+// because little is gained near it: at 2^15 the patches' 1.0 (tet4) and 1.5 ms (hex8) are earned back after about 230
+// and 210 applies on them, at 2^14 tetrahedra after 800.
+extern int g_hex8_patches;
 constexpr ptrdiff_t kPatchMinElements = (ptrdiff_t)1 << 15;
 // elements per cell of mesh_cells: at least kPatchElements, then as many as leave kCellsWanted cells, at
 // most kCellHexes or kCellTets (flat around these: 1.93M hexahedra at 384, 512, 768, 1,024 elements a cell
@@ -255,6 +262,21 @@ const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t 
 // LazyPart's make() does.
 int mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
 int mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
+// A Laplacian's applies run element by element until they have cost about what making the cells costs, so that a mesh
+// with few applies pays for no cells and one with many at most twice what they cost.  Cells take 1.0, 2.3, 11.9 ms for
+// 3.5e4, 2.0e5, 2.4e6 tetrahedra and 1.5, 2.7, 12.4 ms for 3.6e4, 2.0e5, 2.0e6 hexahedra: as long as 103, 65, 26 and
+// 92, 33, 19 element-wise applies, near 25 + 2.6e6 / E for both.  The words in their order, which a further operator on
+// the mesh makes at its first apply, take 0.02 to 0.2 ms (that apply is then 33 us in place of 23 for 3.5e4
+// tetrahedra, 71 in place of 122 for 5.8e5).
+constexpr double kCellsAfter = 25, kCellsAfterBy = 2.6e6;
+// In an apply that will be replayed (GraphOp's eager one, before its recording) they are made at once.
+struct ReplayedScope {
+    bool before;
+    ReplayedScope();
+    ~ReplayedScope();
+    ReplayedScope(const ReplayedScope &) = delete;
+    ReplayedScope &operator=(const ReplayedScope &) = delete;
+};
 // The corners of a tet4/hex8 mesh by node, built by the first call outside a capture; null where they are not
 // available (the element-wise kernels run then).
 const NodeElements *mesh_node_elements(const sfem_amd_mesh *m, hipStream_t s);

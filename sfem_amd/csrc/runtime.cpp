@@ -215,7 +215,11 @@ bool g_fused_chebyshev = false;
 bool g_mixed_cg = true;
 bool g_atomic_skeleton = false;
 int g_elasticity_form = 0;
-bool g_hex8_patches = true;
+int g_hex8_patches = 1;  // 2: a Laplacian's patches at its first apply
+
+static thread_local bool t_replayed = false;
+ReplayedScope::ReplayedScope() : before(t_replayed) { t_replayed = true; }
+ReplayedScope::~ReplayedScope() { t_replayed = before; }
 
 const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t s) {
     auto &slot = m->sub[Ls];
@@ -324,9 +328,19 @@ struct LaplacianOp final : OpBase {
                                                            x, y, part.p, sk, s, ow, g_atomic_skeleton);
         }
     }
-    // tet4/hex8: the element patches of the mesh and this operator's words in their slot order (first use)
+    // tet4/hex8: the element patches of the mesh and this operator's words in their slot order
     bool patches_ready(hipStream_t s) {
-        return patch_words.ready(s, [&] { return make_patch_words(s); });
+        return patch_words.ready(s, [&] { return make_patch_words(s); }, [&] { return cells_due(s); });
+    }
+    // whether this apply should make them (see kCellsAfter).  The next one should where this one is being captured:
+    // it will be replayed, element by element, and so will what is captured next.
+    bool cells_due(hipStream_t s) {
+        constexpr int kNow = 1 << 20;
+        if (g_hex8_patches == 2 || t_replayed) return true;
+        const int n = m->laplacian_applies.load(std::memory_order_relaxed);
+        const bool capture = !may_build_patches(s);
+        if (n < kNow) m->laplacian_applies.store(capture ? kNow : n + 1, std::memory_order_relaxed);
+        return !capture && n >= kCellsAfter + kCellsAfterBy / (double)m->E;
     }
     int make_patch_words(hipStream_t s) {
         if (const int st = mesh_cells(m, s); st <= 0) return st;
@@ -1020,7 +1034,11 @@ struct GraphOp final : OpBase {
             c.exec = nullptr;
             c.calls = 0;
         }
-        if (c.calls++ == 0 || failed) return eager();
+        if (failed) return eager();
+        if (c.calls++ == 0) {
+            ReplayedScope replayed;
+            return eager();
+        }
         if (!c.exec) {
             hipGraph_t graph = nullptr;
             int err = SFEM_FAILURE;
@@ -1236,7 +1254,7 @@ int sfem_amd_set_option(const char *name, int value) {
         return SFEM_SUCCESS;
     }
     if (std::strcmp(name, "hex8_patches") == 0) {
-        g_hex8_patches = value != 0;
+        g_hex8_patches = value == 2 ? 2 : value != 0;
         bump_state_epoch();
         return SFEM_SUCCESS;
     }
