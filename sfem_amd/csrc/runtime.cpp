@@ -2206,8 +2206,10 @@ int sfem_amd_op_benchmark(sfem_amd_op *op, const void *x, void *y, int warmup, i
     CHECK_HANDLE(op);
     SFEM_AMD_REQUIRE(reps > 0 && total_ms, "benchmark: reps > 0 and an output pointer required");
     hipStream_t s = as_stream(stream);
-    for (int i = 0; i < warmup; i++)
+    for (int i = 0; i < warmup; i++) {
+        ReplayedScope repeated;  // what many applies would make is made by the untimed ones
         if (op->impl->apply(x, y, s)) return SFEM_FAILURE;
+    }
     DevArray<double> scratch;
     if (flush_bytes && scratch.alloc((flush_bytes + 7) / 8)) return SFEM_FAILURE;
     // the events are destroyed on every exit path
