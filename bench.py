@@ -370,7 +370,7 @@ def hex8_elasticity_config3(S, args, n=128, rtol=1e-10):
                                 "first_apply_seconds": first}
     out["apply_fp64"]["traffic"] = profiled_traffic(PROFILE_HEX8)
     out["apply_fp64"]["traffic_source"] = ("profiles/hex8_elasticity_apply_128cube.md (rocprofv3 --pmc FETCH_SIZE, "
-                                           "WRITE_SIZE per dispatch, patch kernel + gather, copy-calibrated)")
+                                           "WRITE_SIZE per dispatch, patch kernel, copy-calibrated)")
     out["apply_fp32"]["rel_error_vs_fp64"] = float(np.linalg.norm(ys["fp32"] - ys["fp64"]) /
                                                    np.linalg.norm(ys["fp64"]))
     out["apply_fp32"]["note"] = ("FP32 sum-factorised arithmetic on bf16 geometry words; error against the FP64 apply, "

@@ -45,7 +45,7 @@ inline std::vector<int> derefinement_levels(int L) {
 
 namespace detail {
 // zero-filled device memory (the diagonal assemblies accumulate into their output); the fill runs on
-// the library stream, which the assemblies below also use
+// the default stream, which the assemblies below also use
 struct DeviceBuffer {
     void *p{nullptr};
     explicit DeviceBuffer(size_t bytes) : p(sfem_amd_malloc(bytes ? bytes : 1)) {

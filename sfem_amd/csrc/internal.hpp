@@ -241,10 +241,10 @@ extern int g_elasticity_form;
 // and 210 applies on them, at 2^14 tetrahedra after 800.
 extern int g_hex8_patches;
 constexpr ptrdiff_t kPatchMinElements = (ptrdiff_t)1 << 15;
-// elements per cell of mesh_cells: at least kPatchElements, then as many as leave kCellsWanted cells, at
-// most kCellHexes or kCellTets (flat around these: 1.93M hexahedra at 384, 512, 768, 1,024 elements a cell
+// elements per cell of mesh_cells: kHexCell hexahedra; tetrahedra as many as leave kTetCellsWanted cells, within
+// kTetCellLeast and kTetCellMost (flat around these: 1.93M hexahedra at 384, 512, 768, 1,024 elements a cell
 // within 4% of each other; 2.41M tetrahedra at 1,024 to 3,072 within 3%)
-constexpr ptrdiff_t kCellsWanted = 1024, kCellHexes = 512, kCellTets = 2048;
+constexpr ptrdiff_t kHexCell = 512, kTetCellsWanted = 1024, kTetCellLeast = 512, kTetCellMost = 2048;
 // Host-side state that a captured HIP graph depends on (library options, switch selections, CNN
 // weights) changes the state epoch; graph-replaying operators re-capture when it moved.
 uint64_t state_epoch();
@@ -269,7 +269,8 @@ int mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
 // the mesh makes at its first apply, take 0.02 to 0.2 ms (that apply is then 33 us in place of 23 for 3.5e4
 // tetrahedra, 71 in place of 122 for 5.8e5).
 constexpr double kCellsAfter = 25, kCellsAfterBy = 2.6e6;
-// In an apply that will be replayed (GraphOp's eager one, before its recording) they are made at once.
+// In an apply that will be repeated (GraphOp's eager one, before its recording; a benchmark's untimed ones) they are
+// made at once.
 struct ReplayedScope {
     bool before;
     ReplayedScope();

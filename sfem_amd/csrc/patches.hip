@@ -5,8 +5,8 @@
 //   patches (hex8 elasticity, bound by its arithmetic) full patches of 512 elements, two rounds of a
 //           256-thread block, with the fewest shared nodes; grown in order on the host, tenths of a
 //           second for millions of elements.
-// Both end in assemble(): elements sorted by patch, patch node lists, local numbering and the shared
-// nodes' partial slots, on the device.  Setup only, once per mesh, deterministic.
+// Both end in assemble(): elements sorted by patch, patch node lists and local numbering, on the device.
+// Setup only, once per mesh, deterministic.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -188,6 +188,7 @@ int assemble(const sfem_amd_mesh *m, DevArray<int32_t> &label, int64_t max_label
 }
 
 // ---------------------------------------------------------------- cells
+// C. Wellons' "lowbias32" integer hash (published with his search for hash functions of this form, 2018)
 __host__ __device__ __forceinline__ uint32_t mix32(uint32_t h) {
     h ^= h >> 16;
     h *= 0x7feb352du;
@@ -320,10 +321,11 @@ int mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
     const ptrdiff_t E = m->E, N = m->nnodes;
     const int nv = m->nv;
     if (m->type == SFEM_AMD_SSHEX8 || E <= 0 || (double)E * nv >= 2147483647.0 || N >= 2147483647) return -1;
-    // Elements per cell: enough cells for the GPU's 256 CUs several times over, and from there on larger ones,
-    // since the shared nodes' part falls with the size; a tetrahedron brings a sixth of a hexahedron's nodes.
-    const ptrdiff_t mean = std::min<ptrdiff_t>(std::max<ptrdiff_t>(E / kCellsWanted, kPatchElements),
-                                               m->type == SFEM_AMD_TET4 ? kCellTets : kCellHexes);
+    // Elements per cell.  Tetrahedra, of which a hexahedron's nodes hold six: enough cells for the GPU's 256 CUs several
+    // times over, and from there on larger ones, since the shared nodes' part falls with the size.
+    const ptrdiff_t mean = m->type == SFEM_AMD_TET4
+                                   ? std::min(std::max(E / kTetCellsWanted, kTetCellLeast), kTetCellMost)
+                                   : kHexCell;
     bool never = false;
     auto build = [&]() -> std::unique_ptr<ElementPatches> {
         Scratch sc;

@@ -95,7 +95,7 @@ def _isolated(nv, E):
 
 
 # element patches from 2^15 elements on: just below and above, ragged last patches, shuffled elements and
-# nodes, the large tet4 patches (2^20), elements without neighbours (a patch each)
+# nodes, the large tet4 patches (2^20), elements without neighbours (grouped by their numbers)
 @pytest.mark.parametrize("kind,n,mesh", [("tet4", 17, "box"), ("tet4", 18, "box"), ("tet4", 23, "shuffled"),
                                          ("tet4", 56, "box"), ("tet4", 0, "isolated"), ("hex8", 31, "box"),
                                          ("hex8", 32, "box"), ("hex8", 37, "shuffled"), ("hex8", 0, "isolated")])
@@ -174,7 +174,7 @@ def test_sshex8_laplacian_fp32_bf16_error_stated():
 
 @pytest.mark.parametrize("L,n", [(1, 3), (2, 3), (3, 2), (4, 3), (5, 2), (6, 2), (8, 3), (10, 1), (12, 1), (16, 2)])
 def test_sshex8_laplacian_fp32_every_level(L, n):
-    """The FP32 apply (LDS-staged kernel up to L=12, line-thread kernel at L=16) against the FP64
+    """The FP32 apply against the FP64
     oracle on the same geometry words (the FP32 operator folds the per-element coefficient into
     the FFF and rounds the products to bf16), accumulate semantics: only the FP32 arithmetic
     differs (< 1e-5); two applies give the same words."""
