@@ -313,6 +313,51 @@ def test_one_operator_in_two_threads(kind):
     assert relerr(host(both), yo[0] + yo[1]) < RTOL
 
 
+def _mix32(h):
+    """The seed hash of the element cells."""
+    h = h.astype(np.uint32)
+    h ^= h >> np.uint32(16)
+    h *= np.uint32(0x7feb352d)
+    h ^= h >> np.uint32(15)
+    h *= np.uint32(0x846ca68b)
+    return h ^ (h >> np.uint32(16))
+
+
+# Cells of unusual meshes: "star" hexahedra around one node, which one cell takes whole (its pieces hold more
+# nodes than fit in LDS: element by element then); "chain" hexahedra in a row, numbered so that all the seeds lie
+# at one end and the growth ends before it reaches the other (the rest is grouped by its numbers)
+@pytest.mark.parametrize("mesh", ["star", "chain"])
+def test_laplacian_cells_of_unusual_meshes(mesh):
+    E = 1 << 15
+    if mesh == "star":
+        el = (1 + np.arange(7 * E).reshape(7, E)).astype(np.int32)
+        el = np.vstack([np.zeros((1, E), np.int32), el])
+        N = 7 * E + 1
+    else:
+        ids = np.arange(E)
+        seed = (ids == 0) | (_mix32(ids) < np.uint32(4294967295.0 / 512))
+        position = np.empty(E, np.int64)  # of each element in the row
+        position[np.concatenate([ids[seed], ids[~seed]])] = ids
+        assert 32 < seed.sum() < 128 and E - seed.sum() > 4096  # more than the growth's rounds
+        quad = 4 * position[None, :] + np.arange(4)[:, None]
+        el = np.vstack([quad, quad + 4]).astype(np.int32)
+        N = 4 * (E + 1)
+    rng = np.random.default_rng(17)
+    fff = rng.uniform(0.1, 1, (E, 6)).astype(np.float32)
+    x, yo = rng.uniform(-1, 1, N), rng.uniform(-1, 1, N)
+    y, xd = dev(yo), dev(x)
+    S.set_option("hex8_patches", 2)
+    try:
+        op = S.laplacian(S.Mesh(S.HEX8, 1, el, N), fff)
+        for _ in range(2):
+            op.apply(xd, y)
+            O.lib.oracle_hex8_laplacian_apply(E, el, fff, None, x, yo)
+        S.synchronize()
+    finally:
+        S.set_option("hex8_patches", 1)
+    assert relerr(host(y), yo) < RTOL
+
+
 def memory_taken(f):
     """Device memory that a call takes and keeps."""
     hip = C.CDLL(None)  # the HIP runtime that the library has loaded
