@@ -310,11 +310,10 @@ __global__ void reseed_kernel(const ptrdiff_t K, const unsigned long long *__res
 }  // namespace
 
 // Neighbourhoods of seeds: every element joins the nearest seed (breadth-first over shared nodes, all
-// cells at once).  Random seeds first; then, once, each cell's deepest element becomes its seed, which
-// rounds the cells off.  Not at all, once, twice: 8.1, 12.4, 17.2 ms for 1.95M hexahedra, whose applies take 48.8,
-// 48.0, 47.6 us; 8.1, 11.9, 15.7 ms for 2.43M tetrahedra of a box (32.9, 29.2, 28.8 us).  (1.62 patch nodes per
-// element from the random seeds on a hex8 box, 440 elements a cell; 1.55 for the ordered growth of mesh_patches.)
-// Sizes spread by a factor of about two around the mean, and cells above 2.5 times the mean are cut.
+// cells at once).  Random seeds first; then, twice, each cell's deepest element becomes its seed, which
+// rounds the cells off.  hex8 box, 440 elements a cell: 1.62, 1.58 patch nodes per element before and after
+// (1.55 for the ordered growth of mesh_patches); sizes spread by a factor of about two around the mean, and
+// cells above 2.5 times the mean are cut.
 int mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
     std::lock_guard<std::mutex> lock(m->lists);
     if (m->cells) return 1;
@@ -350,7 +349,7 @@ int mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
             if (seed.alloc(K) || best.alloc(K)) return SFEM_FAILURE;
             LAUNCH(seed_list_kernel, E, lo.p, hi.p, seed.p);
             int64_t max_label = K - 1;
-            constexpr int kSmooth = 1;
+            constexpr int kSmooth = 2;
             for (int pass = 0;; pass++) {
                 LAUNCH(fill_kernel<int32_t>, E, -1, dist.p);
                 LAUNCH(fill_kernel<uint32_t>, N, kNoKey, nkey.p);
