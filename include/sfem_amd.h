@@ -67,8 +67,8 @@ const char *sfem_amd_last_error(void);
  * summation order differs.  "hex8_patches" (default 1): tet4 and hex8 applies on meshes of at least
  * 2^15 elements run on element patches (512 or 2,048 elements grown over shared nodes, accumulated in
  * LDS and added to y with atomics; the partition is made inside an apply: the elasticity's by the first
- * one, on the host, the Laplacian's once a mesh's element-wise applies have cost about as much, after 25
- * to 105 of them, or before a graph op records one; 2 makes the Laplacian's by the first apply too, for
+ * one, on the host, the Laplacian's once a mesh's element-wise applies have cost about as much, after 30
+ * to 134 of them, or before a graph op records one; 2 makes the Laplacian's by the first apply too, for
  * programs that capture applies themselves), and the overwriting applies inside solvers on smaller hex8 meshes node by node; 0 runs one
  * element per lane with atomics.
  * "mixed_cg" (default 1): flexible CGs created afterwards around a bridged FP32 preconditioner keep

@@ -237,8 +237,8 @@ extern int g_elasticity_form;
 // patches: hex8 Laplacian 8,000 elements 6.8 / 8.2 us, 13,824 8.1 / 7.8, 32,768 15.1 / 7.9, 262,144 94 / 11;
 // tet4 6,000 5.5 / 5.2 us, 16,464 5.7 / 4.4, 34,992 9.0 / 4.8, 279,936 48 / 6.5; FP64 hex8 elasticity 8,000
 // 10 / 13 us, 13,824 17 / 14, 32,768 33 / 15.  The line lies above the crossing (about 12,000 elements)
-// because little is gained near it: at 2^15 the patches' 1.0 (tet4) and 1.5 ms (hex8) are earned back after about 230
-// and 210 applies on them, at 2^14 tetrahedra after 800.
+// because little is gained near it: at 2^15 the patches' 1.3 (tet4) and 2.0 ms (hex8) are earned back after about 300
+// and 280 applies on them, at 2^14 tetrahedra after 1,000.
 extern int g_hex8_patches;
 constexpr ptrdiff_t kPatchMinElements = (ptrdiff_t)1 << 15;
 // elements per cell of mesh_cells: kHexCell hexahedra; tetrahedra as many as leave kTetCellsWanted cells, within
@@ -263,12 +263,12 @@ const sfem_amd_mesh *mesh_subblocks(const sfem_amd_mesh *m, int Ls, hipStream_t 
 int mesh_patches(const sfem_amd_mesh *m, hipStream_t s);
 int mesh_cells(const sfem_amd_mesh *m, hipStream_t s);
 // A Laplacian's applies run element by element until they have cost about what making the cells costs, so that a mesh
-// with few applies pays for no cells and one with many at most twice what they cost.  Cells take 1.0, 2.3, 11.9 ms for
-// 3.5e4, 2.0e5, 2.4e6 tetrahedra and 1.5, 2.7, 12.4 ms for 3.6e4, 2.0e5, 2.0e6 hexahedra: as long as 103, 65, 26 and
-// 92, 33, 19 element-wise applies, near 25 + 2.6e6 / E for both.  The words in their order, which a further operator on
+// with few applies pays for no cells and one with many at most twice what they cost.  Cells take 1.2, 2.9, 15.7 ms for
+// 3.5e4, 2.0e5, 2.4e6 tetrahedra and 2.0, 3.5, 17.2 ms for 3.6e4, 2.0e5, 2.0e6 hexahedra: as long as 134, 82, 34 and
+// 119, 43, 26 element-wise applies, near 30 + 3.4e6 / E for both.  The words in their order, which a further operator on
 // the mesh makes at its first apply, take 0.02 to 0.2 ms (that apply is then 33 us in place of 23 for 3.5e4
 // tetrahedra, 71 in place of 122 for 5.8e5).
-constexpr double kCellsAfter = 25, kCellsAfterBy = 2.6e6;
+constexpr double kCellsAfter = 30, kCellsAfterBy = 3.4e6;
 // In an apply that will be repeated (GraphOp's eager one, before its recording; a benchmark's untimed ones) they are
 // made at once.
 struct ReplayedScope {

@@ -311,9 +311,12 @@ __global__ void reseed_kernel(const ptrdiff_t K, const unsigned long long *__res
 
 // Neighbourhoods of seeds: every element joins the nearest seed (breadth-first over shared nodes, all
 // cells at once).  Random seeds first; then, twice, each cell's deepest element becomes its seed, which
-// rounds the cells off.  hex8 box, 440 elements a cell: 1.62, 1.58 patch nodes per element before and after
-// (1.55 for the ordered growth of mesh_patches); sizes spread by a factor of about two around the mean, and
-// cells above 2.5 times the mean are cut.
+// rounds the cells off.  Not at all, once, twice, making them and an apply: 8.1, 12.4, 17.2 ms and 48.8, 48.0,
+// 47.6 us for 1.95M hexahedra; 8.1, 11.9, 15.7 ms and 32.9, 29.2, 28.8 us for 2.43M tetrahedra of a box; once and
+// twice 48.0 and 46.5 us a pass for 2.41M shuffled ones.  The first time is earned back after 1,000 to 5,400 applies, the
+// second after 3,000 to 12,000, and only meshes that have had many get cells at all (kCellsAfter).  hex8 box, 440
+// elements a cell: 1.62, 1.58 patch nodes per element before and after (1.55 for the ordered growth of
+// mesh_patches); sizes spread by a factor of about two around the mean, and cells above 2.5 times the mean are cut.
 int mesh_cells(const sfem_amd_mesh *m, hipStream_t s) {
     std::lock_guard<std::mutex> lock(m->lists);
     if (m->cells) return 1;
