@@ -794,7 +794,7 @@ template int scatter_elements<float>(ptrdiff_t, int, const int32_t *, int, int, 
 // What bounds it: the hidden layers' products (15 per 16 cells, plane and sign at 16 cycles) and their operand
 // reads (5 of 1 KB) take about the same time, 13,000 cycles per element at L = 8.  Whole-element layers (14
 // products for 14 reads, 141 KB of LDS, one block per CU and nothing to overlap a layer's barriers) took
-// 3.14 ms for 32,768 elements of L = 8; this form 1.53 ms (890 TFLOP/s; a large bf16 matrix product
+// 3.14 ms for 32,768 elements of L = 8; this form 1.56-1.64 ms (830-870 TFLOP/s; a large bf16 product
 // reaches 1,190 on the same card), of which layers 1 and 4 take 0.2.
 //
 // A plane is its lines with one halo cell each, LS = L + 2 cells apart, so that the cell after a line's last

@@ -273,9 +273,9 @@ __global__ void __launch_bounds__(256)
 // are gathered into LDS once (x), the elements accumulate into LDS (y, LDS atomics), then every patch
 // node is added to y with a global atomic, consecutive lanes on consecutive entries of y: nodes that
 // several patches share need no further pass.  (Shared nodes written to partials instead, summed by a
-// gather kernel, the others added without atomics: 73 against 52 us at 1.93M hexahedra, Laplacian; 176
-// against 133 us at 2.10M, FP64 elasticity (FP32 103 against 85), where a lane per node with its three components apart
-// takes 244 us.)  It also lets several streams apply one operator, or add into one y.  The
+// gather kernel, the others added without atomics, a pass with its zero fill on one mesh: 72 against 52 us at 1.93M
+// hexahedra, Laplacian; 175 against 131 us at 2.10M, FP64 elasticity (FP32 101 against 87), where a lane per node with
+// its three components apart takes 244 us.  Three meshes in turn, which leave nothing in the caches: 56 and 154 us.)  It also lets several streams apply one operator, or add into one y.  The
 // geometry and coefficient words are stored in patch-slot order, so every read of them coalesces.
 // The LDS accumulator is FP64 for both value types: ds_add_f64 keeps pace with the arithmetic, while
 // ds_add_f32 measured 7x the LDS busy cycles and 100x the LDS wait of the whole FP64 kernel here.
