@@ -358,6 +358,24 @@ def test_laplacian_cells_of_unusual_meshes(mesh):
     assert relerr(host(y), yo) < RTOL
 
 
+@pytest.fixture(scope="module")
+def kernels_loaded():
+    """Applies of every kind on patches and without them: loading their kernels takes device memory as well."""
+    x, y = dev(np.ones(3 * 40 ** 3)), zeros(3 * 40 ** 3)
+    for tet4, n in ((True, 18), (False, 33)):
+        el, pts = O.box_mesh(n + 1, n + 1, n + 1, tet4=tet4)
+        m = S.Mesh(S.TET4 if tet4 else S.HEX8, 1, el, pts.shape[1])
+        ops = [S.laplacian(m, O.tet4_fff(el, pts) if tet4 else O.hex8_fff(el, pts))]
+        if not tet4:
+            ops.append(S.linear_elasticity(m, *O.hex8_adj_det(el, pts), *O.lame(1.0, 0.3)))
+        for patches in (0, 2):
+            S.set_option("hex8_patches", patches)
+            for op in ops:
+                S._check(S.lib.sfem_amd_op_apply(op.h, S._dptr(x), S._dptr(y), None), "op_apply")
+    S.set_option("hex8_patches", 1)
+    S.synchronize()
+
+
 def memory_taken(f):
     """Device memory that a call takes and keeps."""
     hip = C.CDLL(None)  # the HIP runtime that the library has loaded
@@ -369,7 +387,7 @@ def memory_taken(f):
 
 
 @pytest.mark.parametrize("kind,n", [("tet4", 18), ("tet4", 40), ("hex8", 33), ("hex8", 64)])
-def test_laplacian_patches_are_made_after_some_applies(kind, n):
+def test_laplacian_patches_are_made_after_some_applies(kind, n, kernels_loaded):
     """The first applies of a mesh run element by element and keep no memory; one of the next hundred or so
     makes the patches, which the later ones run on.  A second operator on the mesh makes its words at its
     first apply; inside a graph operator the patches are made before the recording."""
@@ -430,7 +448,7 @@ def test_laplacian_patches_are_made_after_some_applies(kind, n):
 
 
 @pytest.mark.parametrize("kind", ["laplacian", "elasticity"])
-def test_patches_that_could_not_be_made_are_tried_again(kind):
+def test_patches_that_could_not_be_made_are_tried_again(kind, kernels_loaded):
     """While a stream is captured in global mode no memory can be had: an apply then runs element by element,
     and the next one makes the patches (seen by the memory they take)."""
     hip = C.CDLL(None)
