@@ -616,6 +616,22 @@ def test_graph_operator_on_a_stream_of_the_caller():
     assert hip.hipStreamDestroy(stream) == 0
 
 
+def test_graph_operator_over_one_that_synchronises_runs_eagerly():
+    el, pts = O.box_mesh(5, 5, 5)
+    fff = O.hex8_fff(el, pts)
+    N = pts.shape[1]
+    nodes = np.where(pts[0] == 0)[0].astype(np.int32)
+    A = S.constrained(S.laplacian(S.Mesh(S.HEX8, 1, el, N), fff), nodes)
+    b = np.random.default_rng(1).uniform(-1, 1, N)
+    b[nodes] = 0
+    P = S.graph_op(S.cg(A, rtol=1e-10))
+    for k in range(3):
+        x = zeros(N)
+        P.apply(dev(b), x)
+        assert true_residual(A, dev(b), x) < 2e-10, k
+    assert S.graph_op_stats(P) == (-1, 0)
+
+
 def test_graphs_recorded_in_two_threads_beside_calls_without_a_stream():
     """While two graph operators record in threads of their own, calls without a stream in this one run
     at once, outside both graphs, and both recordings succeed.  The recorded sequence is long (2,000
